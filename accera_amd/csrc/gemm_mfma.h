@@ -132,13 +132,105 @@ struct OperandTile {
     }
 
     // ---- register-staged fill ----
-    // EDGE 0: full tiles.  1: tiles that end past M / N / K, every row of the operand 16 bytes aligned and K (and the
-    // contiguous extent) a multiple of the 16-byte vector: chunks are in or out as a whole.  2: any sizes, leading
-    // dimensions and pointers: chunks lie anywhere (the loads are declared unaligned; the hardware takes them), and the
-    // chunk that straddles the end of a row is put together from single elements.
-    template <int EDGE>
-    __device__ static __forceinline__ void load_global(i32x4 (&regs)[PER_THREAD], const char* base, int r0, int k0,
-                                                       int64_t ld, int rmax, int K, int tid)
+    // Full tiles: chunk after chunk from where the tile lies.
+    __device__ static __forceinline__ void load_global(i32x4 (&regs)[PER_THREAD], const char* base, int r0, int k0, int64_t ld, int tid)
+    {
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+            int id = tid + i * NT;
+            int row = id / CPR, c = id % CPR;
+            regs[i] = *(const i32x4*)(base + global_off(row, c, r0, k0, ld));
+        }
+    }
+
+    // Tiles that end past M / N / K, of operands whose rows hold at least one 16-byte chunk.  Every chunk is one load without a
+    // branch: one that would cross the end of its row is fetched so that it ends there, and put right when it goes to LDS
+    // (realign); for a row past the end the last one is fetched, and what comes of it does not matter past M / N, where it is
+    // multiplied into rows of C that are not stored, and is overwritten past K (zero_past_k).
+    // (Put together from single elements behind branches, a straddling chunk was 8 or 16 loads that the whole wave waited
+    // for, and every join of the branches a wait for memory: 1234x5678x4321 fp16 204 us, int8 3139x1152x6185 with both operands
+    // column-major 202 us; 116 and 66 us this way and with the ring below.  A test around each load alone is as slow: 3520x1088x5610 bf16 97 us without,
+    // 276 with.)
+    // ANY: any alignment (the loads are declared unaligned; the hardware takes them).
+    template <bool ANY>
+    __device__ static __forceinline__ void load_edge(i32x4 (&regs)[PER_THREAD], const char* base, int r0, int k0, int64_t ld,
+                                                     int rmax, int K, int tid)
+    {
+        typedef i32x4 __attribute__((aligned(1))) i32x4_any;
+        constexpr int VEC = 16 / ES;
+        const int c = tid % CPR; // (a pass of the workgroup covers whole rows: the same chunk column in every pass)
+        // position along the contiguous index and its last chunk; what is uniform goes into the scalar base, so that the lanes'
+        // offsets are 32-bit and not negative
+        const int along = (KC ? k0 : r0) + c * VEC, last = (KC ? K : rmax) - VEC;
+        const int along0 = (KC ? k0 : r0) < last ? (KC ? k0 : r0) : last;
+        const unsigned along_off = (unsigned)(((along < last ? along : last) - along0) * ES);
+        const int across0 = KC ? r0 : k0, across_left = (KC ? rmax : K) - 1 - across0; // (>= 0)
+        const char* b = base + ((int64_t)across0 * ld + along0) * ES;
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+            const int row = tid / CPR + i * ROWS_PER_PASS;
+            const unsigned off = (unsigned)(row < across_left ? row : across_left) * ((unsigned)ld * ES) + along_off;
+            if constexpr (ANY) regs[i] = *(const i32x4_any*)(b + off);
+            else regs[i] = *(const i32x4*)(b + off);
+        }
+    }
+
+    // Is some chunk of the tile fetched early, so that its end is the end of its row?  (the same for the whole workgroup; a
+    // row of whole chunks never has one)
+    __device__ static __forceinline__ bool straddles(int r0, int k0, int rmax, int K)
+    {
+        constexpr int VEC = 16 / ES;
+        return KC ? k0 + BK > K && K % VEC != 0 : r0 + R > rmax && rmax % VEC != 0;
+    }
+    // Move such chunks to their places: down by as many bytes as they were fetched early, zeros from above.
+    __device__ static __forceinline__ void realign(i32x4 (&regs)[PER_THREAD], int r0, int k0, int rmax, int K, int tid)
+    {
+        constexpr int VEC = 16 / ES;
+        const int along = (KC ? k0 : r0) + tid % CPR * VEC, last = (KC ? K : rmax) - VEC;
+        const int early = along > last ? (along - last) * ES : 0; // (16 and more: outside as a whole)
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+            int w[5] = {regs[i][0], regs[i][1], regs[i][2], regs[i][3], 0};
+            if (early & 8) { w[0] = w[2]; w[1] = w[3]; w[2] = w[3] = 0; }
+            if (early & 4) { w[0] = w[1]; w[1] = w[2]; w[2] = w[3]; w[3] = 0; }
+            if constexpr (ES < 4) {
+#pragma unroll
+                for (int d = 0; d < 4; ++d) w[d] = (int)__builtin_amdgcn_alignbyte((unsigned)w[d + 1], (unsigned)w[d], (unsigned)early & 3);
+            }
+            regs[i] = i32x4{w[0], w[1], w[2], w[3]};
+        }
+    }
+    // Zeros for what lies past the end of K, over what store_lds has just written there (a wave's LDS accesses complete in
+    // order): K's padding has to be zeros, rows past M / N are multiplied into rows of C that are not stored and may hold
+    // anything.  (Two instructions per chunk; selected chunk by chunk in registers it was nine, and the small problems, which are
+    // bound by the fetch of instructions that run once, lost 0.5 us of 3.5: 80x128x48 fp16.)
+    __device__ static __forceinline__ void zero_past_k(char* lds, int k0, int K, int tid)
+    {
+        constexpr int VEC = 16 / ES;
+        const int c = tid % CPR;
+        const i32x4 zero = {0, 0, 0, 0};
+        if constexpr (KC) {
+            if (k0 + c * VEC >= K) {
+#pragma unroll
+                for (int i = 0; i < PER_THREAD; ++i) {
+                    const int row = tid / CPR + i * ROWS_PER_PASS;
+                    *(i32x4*)(lds + row * ROW_BYTES + swizzle(row, c) * 16) = zero;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PER_THREAD; ++i) {
+                const int row = tid / CPR + i * ROWS_PER_PASS;
+                if (k0 + row >= K) *(i32x4*)(lds + row * ROW_BYTES + swizzle(row, c) * 16) = zero;
+            }
+        }
+    }
+
+    // The same with every chunk tested: nothing outside is fetched, zeros take its place, and (ANY) a chunk that straddles the
+    // end of its row is put together from single elements, whatever the length of the row.
+    template <bool ANY>
+    __device__ static __forceinline__ void load_checked(i32x4 (&regs)[PER_THREAD], const char* base, int r0, int k0,
+                                                        int64_t ld, int rmax, int K, int tid)
     {
         typedef i32x4 __attribute__((aligned(1))) i32x4_any;
         constexpr int VEC = 16 / ES;
@@ -146,7 +238,7 @@ struct OperandTile {
         for (int i = 0; i < PER_THREAD; ++i) {
             int id = tid + i * NT;
             int row = id / CPR, c = id % CPR;
-            if constexpr (EDGE == 2) {
+            if constexpr (ANY) {
                 // elements of this chunk inside the matrix: all of them, the first few, or none
                 const bool row_in = KC ? (r0 + row) < rmax : (k0 + row) < K;
                 const int left = KC ? K - (k0 + c * VEC) : rmax - (r0 + c * VEC);
@@ -170,13 +262,11 @@ struct OperandTile {
                     }
                     regs[i] = v;
                 }
-            } else if constexpr (EDGE == 1) {
+            } else {
                 if (in_bounds(row, c, r0, k0, rmax, K))
                     regs[i] = *(const i32x4*)(base + global_off(row, c, r0, k0, ld));
                 else
                     regs[i] = i32x4{0, 0, 0, 0};
-            } else {
-                regs[i] = *(const i32x4*)(base + global_off(row, c, r0, k0, ld));
             }
         }
     }
@@ -350,7 +440,7 @@ __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, i
 template <int IN_, int BM_, int BN_, int WAVES_M_, int WAVES_N_, bool A_KC_, bool B_KC_, bool DIRECT_, bool EDGE_, int KB_, int STAGES_,
           bool PINGPONG_ = false, bool TIMED_ = false, bool ANY_ = false>
 struct MfmaConfig {
-    // ANY (an EDGE build): operands of any size, leading dimension and alignment (see OperandTile::load_global)
+    // ANY (an EDGE build): operands of any size, leading dimension and alignment (see OperandTile::load_edge)
     static constexpr bool ANY = ANY_;
     static_assert(!ANY_ || EDGE_, "the any-shape fill is a form of the edge fill");
     static constexpr bool PINGPONG = PINGPONG_;
@@ -423,7 +513,6 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
     constexpr int IN = Cfg::IN, BM = Cfg::BM, BN = Cfg::BN, WAVES_M = Cfg::WAVES_M, WAVES_N = Cfg::WAVES_N;
     constexpr int KB = Cfg::KB, STAGES = Cfg::STAGES, NT = Cfg::NT;
     constexpr bool A_KC = Cfg::A_KC, B_KC = Cfg::B_KC, DIRECT = Cfg::DIRECT, EDGE = Cfg::EDGE;
-    constexpr int FILL_MODE = Cfg::ANY ? 2 : (EDGE ? 1 : 0);
     constexpr int ES = InTraits<IN>::ES;
     constexpr int BK = KB / ES;
     constexpr int KSTEPS = KB / 32;
@@ -698,41 +787,88 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
         }
     } else {
         // Register-staged fill: a K tile travels global memory -> registers -> LDS.  The LDS side is double-buffered; the
-        // register side is a ring of R tiles, so that R loads are in flight while one tile is multiplied (a 64 x 64 tile is
+        // register side is a ring of RING tiles, so that RING loads are in flight while one tile is multiplied (a 64 x 64 tile is
         // multiplied in a fraction of the time its load takes: with one tile in flight a k-step costs the memory latency).
-        // Tile t sits in slot t % R; the slot of the tile that has just gone to LDS is refilled with tile t + R.
-        // (measured on the odd shapes of the reference's lists, ring of three against one: fp16 7 - 10 % faster -- 1000^3 12.5 ->
-        // 11.7 us, 5041x192x720 10.2 -> 9.1, 600x64x196 6.7 -> 5.8 -- int8 3 - 4 % slower, so 16-bit inputs only)
-        constexpr int R = Cfg::ANY && BM * BN <= 64 * 64 && ES == 2 ? 3 : 1;
-        i32x4 ra[R][TA::PER_THREAD], rb[R][TB::PER_THREAD];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (r < KT) {
-                TA::template load_global<FILL_MODE>(ra[r], Ab, m0, r * BK, lda, p.M, p.K, tid);
-                TB::template load_global<FILL_MODE>(rb[r], Bb, n0, r * BK, ldb, p.N, p.K, tid);
-            }
-        TA::store_lds(ra[0], smem, tid);
-        TB::store_lds(rb[0], smem + TA::TILE_BYTES, tid);
-        __syncthreads();
-        for (int kt0 = 0; kt0 < KT; kt0 += R) {
-#pragma unroll
-            for (int u = 0; u < R; ++u) {
-                const int kt = kt0 + u;
-                if (kt >= KT) break;
-                char* cur = smem + (kt & 1) * STAGE_BYTES;
-                char* nxt = smem + ((kt + 1) & 1) * STAGE_BYTES;
-                if (kt + R < KT) {
-                    TA::template load_global<FILL_MODE>(ra[u], Ab, m0, (kt + R) * BK, lda, p.M, p.K, tid);
-                    TB::template load_global<FILL_MODE>(rb[u], Bb, n0, (kt + R) * BK, ldb, p.N, p.K, tid);
+        // Tile t sits in slot t % RING; the slot of the tile that has just gone to LDS is refilled with tile t + RING.
+        // The waits for memory count the loads that are younger than the ones waited for, and the compiler counts none that
+        // stand behind a branch: the loop that fetches without one keeps the ring full, the last tiles are a copy of it with tests.
+        constexpr int RING = EDGE ? (BM * BN <= 64 * 64 ? 3 : BM * BN <= 128 * 128 ? 2 : 1) : 1;
+        i32x4 ra[RING][TA::PER_THREAD], rb[RING][TB::PER_THREAD];
+        // (CHECKED: chunk by chunk, see OperandTile::load_checked)
+        auto staged_loop = [&](auto checked_tag) __attribute__((always_inline)) {
+            constexpr bool CHECKED = decltype(checked_tag)::value;
+            auto load = [&](int r, int kt) __attribute__((always_inline)) {
+                if constexpr (!EDGE) {
+                    TA::load_global(ra[r], Ab, m0, kt * BK, lda, tid);
+                    TB::load_global(rb[r], Bb, n0, kt * BK, ldb, tid);
+                } else if constexpr (CHECKED) {
+                    TA::template load_checked<Cfg::ANY>(ra[r], Ab, m0, kt * BK, lda, p.M, p.K, tid);
+                    TB::template load_checked<Cfg::ANY>(rb[r], Bb, n0, kt * BK, ldb, p.N, p.K, tid);
+                } else {
+                    TA::template load_edge<Cfg::ANY>(ra[r], Ab, m0, kt * BK, lda, p.M, p.K, tid);
+                    TB::template load_edge<Cfg::ANY>(rb[r], Bb, n0, kt * BK, ldb, p.N, p.K, tid);
                 }
+            };
+            auto store = [&](int r, int kt) __attribute__((always_inline)) {
+                char* to = smem + (kt & 1) * STAGE_BYTES;
+                if constexpr (Cfg::ANY && !CHECKED) {
+                    if (TA::straddles(m0, kt * BK, p.M, p.K)) TA::realign(ra[r], m0, kt * BK, p.M, p.K, tid);
+                    if (TB::straddles(n0, kt * BK, p.N, p.K)) TB::realign(rb[r], n0, kt * BK, p.N, p.K, tid);
+                }
+                TA::store_lds(ra[r], to, tid);
+                TB::store_lds(rb[r], to + TA::TILE_BYTES, tid);
+                if constexpr (EDGE && !CHECKED) {
+                    if ((kt + 1) * BK > p.K) {
+                        TA::zero_past_k(to, kt * BK, p.K, tid);
+                        TB::zero_past_k(to + TA::TILE_BYTES, kt * BK, p.K, tid);
+                    }
+                }
+            };
+            auto multiply = [&](int kt) __attribute__((always_inline)) {
+                const char* cur = smem + (kt & 1) * STAGE_BYTES;
                 load_first_frags(cur, cur + TA::TILE_BYTES);
                 mma_tile(cur, cur + TA::TILE_BYTES, cur, cur + TA::TILE_BYTES, std::false_type{}, std::false_type{}, 0, 0);
-                if (kt + 1 < KT) {
-                    TA::store_lds(ra[(u + 1) % R], nxt, tid);
-                    TB::store_lds(rb[(u + 1) % R], nxt + TA::TILE_BYTES, tid);
+            };
+#pragma unroll
+            for (int r = 0; r < RING; ++r)
+                if (r < KT) load(r, r);
+            store(0, 0);
+            __syncthreads();
+            int kt0 = 0;
+            if constexpr (!CHECKED) {
+                for (; kt0 + 2 * RING <= KT; kt0 += RING) {
+#pragma unroll
+                    for (int u = 0; u < RING; ++u) {
+                        load(u, kt0 + u + RING);
+                        multiply(kt0 + u);
+                        store((u + 1) % RING, kt0 + u + 1);
+                        __syncthreads();
+                    }
                 }
-                __syncthreads();
             }
+            for (; kt0 < KT; kt0 += RING) {
+#pragma unroll
+                for (int u = 0; u < RING; ++u) {
+                    const int kt = kt0 + u;
+                    if (kt >= KT) break;
+                    if (kt + RING < KT) load(u, kt + RING);
+                    multiply(kt);
+                    if (kt + 1 < KT) store((u + 1) % RING, kt + 1);
+                    __syncthreads();
+                }
+            }
+        };
+        if constexpr (EDGE) {
+            // Chunk by chunk: rows shorter than a chunk; and the smallest problems, K of no more tiles than are fetched before
+            // the first is waited for, where no chunk straddles the end of a row and what is outside need not be fetched
+            // (6016x16x128 bf16 3.3 us, 4.2 with the other loop; 80x128x48 3.4 / 4.3; where chunks do straddle the other is ahead
+            // however short K is: 1280x6214x96 fp16 14.2 / 10.3).
+            constexpr int VEC = 16 / ES;
+            const int ext_a = A_KC ? p.K : p.M, ext_b = B_KC ? p.K : p.N;
+            if (ext_a < VEC || ext_b < VEC || (KT <= RING && ext_a % VEC == 0 && ext_b % VEC == 0)) staged_loop(std::true_type{});
+            else staged_loop(std::false_type{});
+        } else {
+            staged_loop(std::false_type{});
         }
     }
 

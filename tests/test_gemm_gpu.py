@@ -1419,3 +1419,49 @@ def test_small_tiles_are_chosen_for_problems_that_would_not_fill_the_chip():
     run_case("bf16", "f32", 1536, 1152, 2048, seed=2301, b_layout="col", prologue=ora.PRO_NONE)
     run_case("i8", "i32", 1024, 960, 1024, seed=2302, a_layout="col")
     run_case("i8", "i8", 1000, 1024, 512, seed=2303)
+
+
+@pytest.mark.parametrize("in_type,out_type", [("f16", "f32"), ("bf16", "bf16"), ("i8", "i32"), ("f32", "f32")])
+@pytest.mark.parametrize("a_layout", ["row", "col"])
+@pytest.mark.parametrize("b_layout", ["row", "col"])
+def test_register_staged_fills_at_the_ends_of_rows_and_tiles(in_type, out_type, a_layout, b_layout):
+    """The fills that fetch rows and chunks from inside the matrix for those past its end: operands that lie in larger
+    matrices of NaN (int8: of 101), K from less than one 16-byte load to more tiles than the register ring has slots."""
+    import accera_amd as acc
+    import torch
+    from accera_amd import _lib
+    es = {"f16": 2, "bf16": 2, "i8": 1, "f32": 4}[in_type]
+    vec = 16 // es
+    rng = np.random.default_rng(77)
+
+    def inside(X, layout, whole):
+        """X on the device, in the middle of a matrix of poison (whole: rows and row starts in whole 16-byte pieces)"""
+        S = X.T if layout == "col" else X
+        off, more = (vec, 3 * vec) if whole else (1, 3)
+        big = np.full((S.shape[0] + 2, (S.shape[1] + more + vec - 1) // vec * vec if whole else S.shape[1] + more), 101 if in_type == "i8" else
+                      0x7fc0 if in_type == "bf16" else np.nan, S.dtype)
+        big[1:1 + S.shape[0], off:off + S.shape[1]] = S
+        d = to_device(big, in_type)[1:1 + S.shape[0], off:off + S.shape[1]]
+        return d.t() if layout == "col" else d
+
+    for v in range(_lib.num_variants()):
+        name = _lib.variant_name(v)
+        if "edge" not in name or ("A=col-major" in name) != (a_layout == "col") or (" B=col-major" in name) != (b_layout == "col"):
+            continue
+        whole = "any-alignment" not in name
+        bm, bn = map(int, re.search(r"mfma (\d+)x(\d+)", name).groups())
+        bk = int(re.search(r"kb(\d+)", name).group(1)) // es
+        ring = 3 if bm * bn <= 64 * 64 else 2
+        if whole:
+            sizes = [(bm + vec, 3 * vec, k) for k in (vec, bk - vec, bk, ring * bk + vec, (2 * ring + 1) * bk - vec)]
+        else:
+            sizes = [(bm + 1, vec + 1, k) for k in (vec - 1, vec, bk - 1, bk + vec + 1, ring * bk, (2 * ring + 1) * bk + 3)]
+            sizes += [(vec - 1, bn + vec - 1, bk + 1), (bm, bn, 2 * ring * bk), (3, 2, 3)]
+        for M, N, K in sizes:
+            print(name, in_type, a_layout, b_layout, M, N, K, flush=True)
+            A, B = make_input(rng, (M, K), in_type), make_input(rng, (K, N), in_type)
+            C0 = make_c0(rng, (M, N), out_type)
+            dA, dB, dC = inside(A, a_layout, whole), inside(B, b_layout, whole), to_device(C0, out_type)
+            acc.gemm_relu(dA, dB, dC, prologue=acc.PROLOGUE_NONE, variant=v)
+            torch.cuda.synchronize()
+            assert_matches(to_host(dC, out_type), ora.gemm_relu_exact(A, B, C0, in_type, out_type, ora.PRO_NONE, ora.EPI_RELU), out_type, K)
