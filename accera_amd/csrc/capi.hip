@@ -789,7 +789,7 @@ int run(const Problem& pb, const Choice& c, hipStream_t stream, LaunchGeom* geom
         if (split) {
             float* ws = nullptr;
             if (!dry_run) {
-                const size_t floats = (size_t)sp.splits * (size_t)g.M * (size_t)g.N;
+                const size_t floats = (size_t)sp.splits * (size_t)g.M * (size_t)g.N + 3; // (the reduction reads whole pieces of four; the built-in array has its counters behind)
                 unsigned* unused = nullptr;
                 if (static_ws) {
                     e = static_workspace(&ws);

@@ -1465,3 +1465,31 @@ def test_register_staged_fills_at_the_ends_of_rows_and_tiles(in_type, out_type, 
             acc.gemm_relu(dA, dB, dC, prologue=acc.PROLOGUE_NONE, variant=v)
             torch.cuda.synchronize()
             assert_matches(to_host(dC, out_type), ora.gemm_relu_exact(A, B, C0, in_type, out_type, ora.PRO_NONE, ora.EPI_RELU), out_type, K)
+
+
+@pytest.mark.parametrize("in_type,out_type", [("f16", "f16"), ("i8", "i16")])
+@pytest.mark.parametrize("N", [1, 2, 3, 5, 62, 63])
+def test_k_split_of_outputs_whose_rows_are_not_whole_vectors(in_type, out_type, N):
+    """The reduction's pieces start at any dword and end past the row: 33 rows, 2 to 9 slices, C read and scaled."""
+    import accera_amd as acc
+    import torch
+    rng = np.random.default_rng(N)
+    M, K = 33, 1160
+    A, B, C0 = make_input(rng, (M, K), in_type), make_input(rng, (K, N), in_type), make_c0(rng, (M, N), out_type)
+    v = _named("64x64", "any-alignment")
+    dA, dB = to_device(A, in_type), to_device(B, in_type)
+    for splits in (2, 8, 9):
+        for col in (False, True):
+            dC = to_device(np.asfortranarray(C0) if col else C0, out_type)
+            if col and N > 1:  # (a column-major C: the transposed product, M columns)
+                acc.gemm_relu(dA, dB, dC, prologue=acc.PROLOGUE_SCALE, prologue_arg=2.0, epilogue=acc.EPILOGUE_NONE, k_splits=splits)
+            else:
+                acc.gemm_relu(dA, dB, dC, prologue=acc.PROLOGUE_SCALE, prologue_arg=2.0, epilogue=acc.EPILOGUE_NONE, variant=v, k_splits=splits)
+            torch.cuda.synchronize()
+            if in_type == "i8":
+                want = (A.astype(np.int64) @ B.astype(np.int64) + 2 * C0.astype(np.int64)).astype(np.int16)
+                assert np.array_equal(to_host(dC, out_type), want)
+            else:
+                want = A.astype(np.float64) @ B.astype(np.float64) + 2.0 * C0.astype(np.float64)
+                # (fp16's last rounding, 2^-11 of the value, and 32-bit sums of 1160 products of at most 1)
+                np.testing.assert_allclose(to_host(dC, out_type).astype(np.float64), want, rtol=2.0 ** -10, atol=1e-3)
