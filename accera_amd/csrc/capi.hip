@@ -296,17 +296,31 @@ hipError_t static_workspace(float** ptr)
 int auto_skinny_splits(int variant, const GemmArgs& g)
 {
     // One workgroup per column block streams all of K unless that leaves most CUs idle;
-    // splitting K costs a trip through the scratch buffer, so it is only used to reach
-    // about one workgroup per CU, with at least 256 k rows per slice.
+    // splitting K costs a trip through the scratch buffer, so it has to be worth that, with
+    // at least 256 k rows per slice.
     // (a batch is one launch: the column blocks of all its problems fill the chip together -- 128 problems of 8 x 128 x 4096
     // took 96.7 us in 16 slices each, which a single problem of that shape would want, and take a quarter of that unsplit)
     const int64_t all_blocks = (int64_t)skinny_column_blocks(variant, g.N) * (g.batch > 1 ? g.batch : 1);
     const int blocks = all_blocks > 4096 ? 4096 : (int)all_blocks;
-    int splits = blocks >= 128 ? 1 : (256 + blocks - 1) / blocks;
-    const int max_splits = g.K / 256 > 0 ? g.K / 256 : 1;
-    if (splits > max_splits) splits = max_splits;
-    if (splits < 1) splits = 1;
-    return splits;
+    if (blocks >= 128) return 1;
+    // The fewest microseconds of: a slice of a block at the rate one CU streams such pieces (out of HBM 36 KB / us, int8 half
+    // lines 20; a B of less than 32 MB, mostly out of the Infinity Cache, 62 less half a KB per row, and 34), never less than all of B at the chip's rate (5.5, 4.2 MB / us), and for a split the second trip through
+    // memory, 3 us, 0.1 per row and 0.15 per slice.  Never more workgroups than CUs: a second round of a few costs as much as the first.
+    // (us, as many slices as gave at least 256 workgroups / this: fp16 22x5056x1408 11.1 in four / 6.4 unsplit, 18x3904x2752
+    // 11.8 in five / 8.8 unsplit, 16x1088x5440 11.1 in 16 / 9.4 in eight, bf16 8x3456x21952 42.2 in five / 28.9 in four, int8
+    // 15x5696x1536 8.8 in three / 5.1 unsplit)
+    const bool i8 = g.in_type == T_I8;
+    const bool cached = (int64_t)g.K * g.N * elem_size(g.in_type) * (g.batch > 1 ? g.batch : 1) < ((int64_t)32 << 20);
+    const double cu_rate = i8 ? (cached ? 34e3 : 20e3) : (cached ? 62e3 - 0.5e3 * g.M : 36e3);
+    const double k_us = (double)g.K * skinny_variant(variant).cols * elem_size(g.in_type) / cu_rate;
+    const double chip_us = (double)g.K * g.N * elem_size(g.in_type) * (g.batch > 1 ? g.batch : 1) / (i8 ? 4.2e6 : 5.5e6);
+    int best = 1;
+    double best_us = 0;
+    for (int s = 1; s == 1 || (s * blocks <= kComputeUnits && g.K / s >= 256); ++s) {
+        const double us = std::max(k_us / s, chip_us) + (s > 1 ? 3.0 + 0.1 * g.M + 0.15 * s : 0.0);
+        if (s == 1 || us < best_us) { best = s; best_us = us; }
+    }
+    return best;
 }
 
 // Automatic MFMA tile choice.  Cost of a candidate = rounds of workgroups over the 256 CUs
@@ -326,6 +340,16 @@ int auto_mfma_variant(const Problem& pb, int only_tile = 0, bool short_rows = fa
     int best = -1;
     double best_cost = 0;
     int best_rank = 0;
+    // Problems that only the register-staged kernels take, K of 64 (int8 128) to 2048 bytes: the 64 x 64 tiles, of which a CU holds four,
+    // hide each other's fetches and are ahead of the 128 x 128 ones whatever their number (us, 128 x 128 / 64 x 64: fp16
+    // 704x3136x48 8.5 / 5.4, 596x3840x696 18.6 / 15.0, 4936x640x112 7.6 / 6.1, 5808x384x496 11.5 / 10.7, bf16 2112x973x448 with
+    // a column-major A 14.5 / 11.6, 6688x768x933 36.1 / 31.8; int8 320x960x32, 190 of them, all write-back, 71.9 / 91.2)
+    // (not with many long tiles, where what the larger ones save in fetches counts: fp16 3712x5694x912 87 / 110)
+    const int64_t k_bytes = (int64_t)pb.g.K * elem_size(pb.g.in_type);
+    const int64_t small_tiles = (int64_t)((pb.g.M + 63) / 64) * ((pb.g.N + 63) / 64) * (pb.g.batch > 1 ? pb.g.batch : 1);
+    bool staged_short_k = k_bytes >= (pb.g.in_type == T_I8 ? 128 : 64) && k_bytes <= 2048 && small_tiles * k_bytes <= 3000000 && pb.g.in_type != T_F32;
+    for (int i = 0; i < n && staged_short_k; ++i)
+        if (tab[i].direct && (tab[i].w4 || pb.g.M >= tab[i].bm || streamed_b(pb, (int64_t)16 << 20)) && mfma_can_take(tab[i], pb)) staged_short_k = false;
     for (int i = 0; i < n; ++i) {
         const MfmaVariant& v = tab[i];
         if (only_tile && (v.bm != only_tile || v.bn != only_tile)) continue;
@@ -369,7 +393,8 @@ int auto_mfma_variant(const Problem& pb, int only_tile = 0, bool short_rows = fa
         // (measured, 64x64 against 128x128 tiles: fp32, bound by its slow MFMAs, 1024^3 20.7 against 63.7 us and 3072x1024x1024
         // 53 against 66; 8- and 16-bit inputs win while a CU has at most two of them -- fp16 1024^3 6.6 against 9.5 us,
         // 1536x1152x2048 14.4 against 17.0 -- and lose beyond: 3072x1024x1024 13.1 against 9.8, 2048^3 30.3 against 21.2)
-        if (v.bm * v.bn <= 64 * 64) cost /= pb.g.in_type == T_F32 ? 1.0 : per_cu <= 2 ? 0.75 : 0.5;
+        if (staged_short_k && v.bm * v.bn <= 64 * 64) cost /= 1.8; // (the 2.0 of the unaligned chunks above hardly shows)
+        else if (v.bm * v.bn <= 64 * 64) cost /= pb.g.in_type == T_F32 ? 1.0 : per_cu <= 2 ? 0.75 : 0.5;
         else if (v.bm * v.bn <= 128 * 64) cost /= 0.8;
         // rank inside one tile shape: ping-pong kb64 x4 > ping-pong others > 8-wave > 4-wave (kb64 x4 first)
         int rank = v.pingpong ? (v.kb == 64 && v.stages == 4 ? 8 : 6) : (v.waves_m * v.waves_n == 8 ? 4 : 2);
@@ -513,7 +538,12 @@ bool streamed_b(const Problem& pb, int64_t least_bytes)
 int streamed_b_tile(const Problem& pb)
 {
     const GemmArgs& g = pb.g;
-    if (!streamed_b(pb, (int64_t)192 << 20)) return 0;
+    // (65 to 256 rows against 32 to 192 MB, 16-bit types: 128 x 128 tiles in slices, whatever of the cache holds B -- fp16
+    // 99x5312x14656 39.5 us in six slices, 86.9 on 64 x 64 tiles; bf16 80x2176x27648 32.1 / 50.8, 115x6464x4608 22.3 / 29.5,
+    // 185x3520x4800 with a K-contiguous B 17.9 / 21.9, fp16 194x2496x21504 45.2 / 74.4, 224x4224x5568 28.4 / 34.0; with tiles enough
+    // for the chip unsplit the general rule is ahead: 159x46976x1024 32.1 us on 256 x 256 tiles, 44.9)
+    if (!streamed_b(pb, (int64_t)192 << 20))
+        return pb.g.in_type != T_I8 && pb.g.M > 64 && streamed_b(pb, (int64_t)32 << 20) && (int64_t)((pb.g.M + 127) / 128) * ((pb.g.N + 127) / 128) < 160 ? 128 : 0;
     // (a tile that holds all rows of A: up to 64 rows the small tiles, up to 128 rows the 128 x 128 tiles, up to 256 the
     // 256 x 256 ones; with direct fills all take fewer rows than they have when A is row-major (the four-wave kernel, which
     // moves its last row of tiles instead, only from 256 rows on), else the register-staged edge forms apply -- of which
@@ -523,19 +553,22 @@ int streamed_b_tile(const Problem& pb)
 
 // K slices for the tile the rule above has taken: about 256 workgroups for the direct-fill kernels of the larger tiles (one
 // workgroup per CU), about 512 for the 64 x 64 tiles and the register-staged kernels (two per CU, fewer bytes in flight
-// each), a power of two, none from 160 tiles on with direct fills; a slice keeps at least 1024 elements of K, and the
+// each), none from 160 tiles on with direct fills; a slice keeps at least 960 elements of K, and the
 // partial sums (written and read once more) stay below a sixth of B's bytes (256x32000x4096: 74 us unsplit, 87 in two
-// slices with their 65 MB; 256x28672x8192 in two slices 132 against 165).
+// slices with their 65 MB; 256x28672x8192 in two slices 132 against 165).  Up to 128 x 128 tiles any number of slices, not powers of two only:
+// bf16 68x5376x23552 with a K-contiguous B 67.1 us in four / 54.2 in six, 11x6208x3904 18.1 in two / 13.4 in four of 976; but
+// 60x8640x1792 10.6 unsplit, 13.7 in two of 896.
 int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats)
 {
     const GemmArgs& g = pb.g;
     const int64_t tiles = (((int64_t)g.M + v.bm - 1) / v.bm) * (((int64_t)g.N + v.bn - 1) / v.bn);
     if (v.direct && tiles >= 160) return 1;
     const int64_t target = v.direct && v.bm * v.bn > 64 * 64 ? kComputeUnits : 2 * kComputeUnits;
-    int64_t want = 1;
-    while (want * 2 * tiles <= target && want < 32) want *= 2;
+    int64_t want = std::min<int64_t>(target / tiles, 32);
     const int64_t b_bytes = (int64_t)g.N * g.K * elem_size(g.in_type);
-    while (want > 1 && (g.K / want < 1024 || want * (int64_t)g.M * g.N * 4 > b_bytes / 6)) want /= 2;
+    while (want > 1 && (g.K / want < 960 || want * (int64_t)g.M * g.N * 4 > b_bytes / 6)) --want;
+    if (v.bm * v.bn > 128 * 128) // (the 256 x 256 tiles, whose partial sums weigh most: a power of two)
+        while (want & (want - 1)) want &= want - 1;
     if (want < 2) return 1;
     if ((size_t)want * (size_t)g.M * (size_t)g.N > ((size_t)1 << 24)) return 1; // 64 MiB of partial sums at most without being asked
     SplitPlan sp;
@@ -604,6 +637,22 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
     c->splits = 1;
     if (variant == ACC950_VARIANT_AUTO) {
         const int sv = auto_skinny_variant(pb);
+        // 17 to 32 rows against a B of 32 MB and more, 16-bit types: the streaming kernel fetches half as many bytes of A as of B
+        // by then; 64 x 64 tiles with direct fills are ahead while their slices fill the chip (us, streaming kernel / tiles: bf16
+        // 31x4416x9792 23.2 / 21.5, 31x20800x4544 58.0 / 39.5, 30x6336x30784 135.6 / 74.0, 29x10176x6656 33.5 / 27.9, fp16
+        // 26x21632x2048 26.2 / 19.7; a smaller B is not: 22x5056x1408 6.4 / 7.9, 18x3904x2752 8.8 / 9.4; nor are tiles too many to split and too few
+        // to fill the chip, or more than it holds: fp16 29x11712x7168 35.8 / 45.5, 25x37056x6912 104.5 / 115.3)
+        if (sv >= 0 && k_splits == 0 && pb.g.M > 16 && pb.g.in_type != T_I8 && streamed_b(pb, (int64_t)32 << 20) && !streamed_b(pb, (int64_t)768 << 20)) {
+            const int mv = auto_mfma_variant(pb, 64, true);
+            int n = 0;
+            const MfmaVariant* tab = mfma_table(pb.g.in_type, &n);
+            const int tiles = (pb.g.N + 63) / 64;
+            if (mv >= 0 && tab[mv].direct && (tiles < 160 || (tiles >= 300 && tiles <= 400 && pb.g.K <= 8192))) {
+                c->variant = mv;
+                c->splits = streamed_b_splits(tab[mv], pb, max_split_floats);
+                return ACC950_OK;
+            }
+        }
         if (sv >= 0) {
             c->variant = ACC950_VARIANT_SKINNY_BASE + sv;
             c->splits = k_splits > 0 ? k_splits : auto_skinny_splits(sv, pb.g);
@@ -642,6 +691,12 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
                     int n = 0;
                     const MfmaVariant& v = mfma_table(pb.g.in_type, &n)[mv];
                     streamed_splits = streamed_b_splits(v, pb, max_split_floats);
+                    // (a B below 192 MB: only with direct fills)
+                    if (!v.direct && !streamed_b(pb, (int64_t)192 << 20)) { mv = -1; streamed_splits = 0; }
+                }
+                if (mv >= 0) {
+                    int n = 0;
+                    const MfmaVariant& v = mfma_table(pb.g.in_type, &n)[mv];
                     // (too few workgroups to stream with, and no split to make more: the general rule's smaller tiles)
                     const int64_t tiles = (((int64_t)pb.g.M + v.bm - 1) / v.bm) * (((int64_t)pb.g.N + v.bn - 1) / v.bn);
                     if (tiles * streamed_splits < 100) { mv = -1; streamed_splits = 0; }
@@ -656,8 +711,8 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
             // column-major A 4.8 against 10.6 -- and on 6 of the 74 with a longer K, where the tiled kernels split K:
             // 64x192x1728 9.9 us in 16 slices against 18.5); with more blocks the tiled kernels with direct fills win
             // (768x576x1024: 17.1 in four slices against 26.3; 2048x192x1280: 17.3 against 27.4).  Against the
-            // register-staged tiled kernels (unaligned operands) the kernel of blocks also wins with a K up to 768, and with a
-            // longer one while the tiles x K slices leave half of the chip idle.
+            // register-staged tiled kernels (unaligned operands) the kernel of blocks also wins with two rounds and a K up to 768, and
+            // with a longer one while the tiles x K slices leave half of the chip idle.
             int slices = 1;
             if (mv >= 0) {
                 int n = 0;
@@ -668,9 +723,10 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
                 // (or more workgroups than there are 32 x 32 blocks: a small output with a long K, which only the tiled kernels split)
                 const int64_t blocks = (((int64_t)pb.g.M + 31) / 32) * (((int64_t)pb.g.N + 31) / 32);
                 const bool one_round = blocks <= kComputeUnits && pb.g.K <= 640;
-                // (against the register-staged kernels a short K is enough: 2304x256x196 with a column-major A, 576 blocks,
-                // 8.4 against 14.1 us; 4608x512x49, 2304 blocks, 16.8 against 19.0; but 1728x192x1225 24.1 against 19.8)
-                if (one_round || (!v.direct && (pb.g.K <= 768 || (tiles * slices * 2 < kComputeUnits && tiles * slices <= blocks)))) mv = -1;
+                // (with more blocks than two rounds the register-staged kernels are ahead however short K is: 4864x2752x648 170 us
+                // against 315, 4148x1439x128 26.6 / 44.4, 1472x674x576 18.5 / 28.2, 5037x376x32 8.0 / 11.9;
+                // 520x792x448, 425 blocks, 13.4 / 12.1)
+                if (one_round || (!v.direct && ((pb.g.K <= 768 && blocks <= 2 * kComputeUnits) || (tiles * slices * 2 < kComputeUnits && tiles * slices <= blocks)))) mv = -1;
             }
             if (mv < 0) { c->variant = ACC950_VARIANT_F32_MFMA; return ACC950_OK; }
         }
