@@ -540,10 +540,10 @@ int streamed_b_tile(const Problem& pb)
     const GemmArgs& g = pb.g;
     // (65 to 256 rows against 32 to 192 MB, 16-bit types: 128 x 128 tiles in slices, whatever of the cache holds B -- fp16
     // 99x5312x14656 39.5 us in six slices, 86.9 on 64 x 64 tiles; bf16 80x2176x27648 32.1 / 50.8, 115x6464x4608 22.3 / 29.5,
-    // 185x3520x4800 with a K-contiguous B 17.9 / 21.9, fp16 194x2496x21504 45.2 / 74.4, 224x4224x5568 28.4 / 34.0; with tiles enough
-    // for the chip unsplit the general rule is ahead: 159x46976x1024 32.1 us on 256 x 256 tiles, 44.9)
+    // 185x3520x4800 with a K-contiguous B 17.9 / 21.9, fp16 194x2496x21504 45.2 / 74.4, 224x4224x5568 28.4 / 34.0; while the
+    // chip takes three slices of every tile: 159x46976x1024, 734 tiles, is 32.1 us on the general rule's 256 x 256 ones, 44.9 this way)
     if (!streamed_b(pb, (int64_t)192 << 20))
-        return pb.g.in_type != T_I8 && pb.g.M > 64 && streamed_b(pb, (int64_t)32 << 20) && (int64_t)((pb.g.M + 127) / 128) * ((pb.g.N + 127) / 128) < 160 ? 128 : 0;
+        return pb.g.in_type != T_I8 && pb.g.M > 64 && streamed_b(pb, (int64_t)32 << 20) && (int64_t)((pb.g.M + 127) / 128) * ((pb.g.N + 127) / 128) * 3 <= kComputeUnits ? 128 : 0;
     // (a tile that holds all rows of A: up to 64 rows the small tiles, up to 128 rows the 128 x 128 tiles, up to 256 the
     // 256 x 256 ones; with direct fills all take fewer rows than they have when A is row-major (the four-wave kernel, which
     // moves its last row of tiles instead, only from 256 rows on), else the register-staged edge forms apply -- of which
