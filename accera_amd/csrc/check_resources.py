@@ -24,7 +24,8 @@ def kernels(text):
     """(function name, {field: value}) per kernel of the remarks text."""
     out, cur = [], None
     for line in text.splitlines():
-        m = re.search(r"remark:\s+(.*?)(?:\s+\[-Rpass-analysis=kernel-resource-usage\])?$", line)
+        # (the place in the source stands before "remark:" or after it, as the compiler's version has it)
+        m = re.search(r"remark:\s+(?:\S+:\d+:\d+:\s+)?(.*?)(?:\s+\[-Rpass-analysis=kernel-resource-usage\])?$", line)
         if not m:
             continue
         body = m.group(1).strip()
@@ -65,25 +66,26 @@ def agpr_uses_outside_asm(text):
 
 
 def main(paths):
-    bad, seen = [], 0
+    bad, seen = [], {}
     for path in [p for p in paths if p.endswith(".s")]:
-        uses, n = agpr_uses_outside_asm(open(path, errors="replace").read())
-        seen += n
+        uses, seen[path] = agpr_uses_outside_asm(open(path, errors="replace").read())
         for name, lines in uses.items():
             bad.append(f"{name}: the compiler uses accumulator registers outside the asm statements, e.g. `{lines[0]}` ({len(lines)} places)")
     for path in [p for p in paths if not p.endswith(".s")]:
+        seen[path] = 0
         for name, f in kernels(open(path, errors="replace").read()):
             if "gemm_mfma16w4_kernel" not in name:
                 continue
-            seen += 1
+            seen[path] += 1
             scratch = int(f.get("ScratchSize [bytes/lane]", "0"))
             if scratch:
                 bad.append(f"{name}: {scratch} bytes of scratch per lane (VGPRs spilled: {f.get('VGPRs Spill')}, SGPRs spilled: {f.get('SGPRs Spill')})")
     if bad:
         print("four-wave GEMM kernels must not use scratch memory, nor the compiler their accumulator registers:\n  " + "\n  ".join(bad), file=sys.stderr)
         return 1
-    if paths and not seen:
-        print("no four-wave GEMM kernel found in " + ", ".join(paths), file=sys.stderr)
+    unread = [path for path, n in seen.items() if not n] # (a file in which nothing is found is one that was not understood)
+    if unread:
+        print("no four-wave GEMM kernel found in " + ", ".join(unread), file=sys.stderr)
         return 1
     return 0
 

@@ -1,0 +1,43 @@
+"""The build's reader of the compiler's resource remarks (accera_amd/csrc/check_resources.py): what it has to notice, in
+the two forms in which compilers write the remarks, and that a file it does not understand is not taken for a clean one."""
+import importlib.util
+import os
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "accera_amd", "csrc")
+W4 = "_ZN6acc95020gemm_mfma16w4_kernelINS_14Mfma16W4ConfigILi0ELb1EEEEEvPKv"
+
+
+def _check():
+    spec = importlib.util.spec_from_file_location("check_resources", os.path.join(CSRC, "check_resources.py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+def _remarks(form, kernels):
+    lines = []
+    for name, scratch in kernels:
+        for body in (f"Function Name: {name}", "    VGPRs: 256", f"    ScratchSize [bytes/lane]: {scratch}", "    VGPRs Spill: 3"):
+            lines.append(form.format(body) + " [-Rpass-analysis=kernel-resource-usage]")
+    return "\n".join(lines) + "\n"
+
+
+@pytest.mark.parametrize("form", ["remark: ./gemm_mfma.h:512:0: {}", "./gemm_mfma.h:512:0: remark: {}"])
+def test_scratch_of_a_four_wave_kernel_fails_the_build(form, tmp_path, capsys):
+    check, path = _check(), tmp_path / "unit.resources.txt"
+    path.write_text(_remarks(form, [("_ZN6acc9505otherEv", 88), (W4, 0)]))
+    assert check.main([str(path)]) == 0
+    path.write_text(_remarks(form, [(W4, 16)]))
+    assert check.main([str(path)]) == 1
+    assert "16 bytes of scratch" in capsys.readouterr().err
+
+
+def test_a_file_without_a_known_kernel_fails_the_build(tmp_path, capsys):
+    check, path, listing = _check(), tmp_path / "unit.resources.txt", tmp_path / "unit.s"
+    listing.write_text(f"{W4}:\n\ts_endpgm\n.Lfunc_end0:\n")
+    path.write_text("remark made of something else\n")
+    assert check.main([str(listing)]) == 0
+    assert check.main([str(path), str(listing)]) == 1
+    assert "unit.resources.txt" in capsys.readouterr().err
