@@ -438,8 +438,12 @@ __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, i
 
 // Compile-time description of one kernel instantiation.
 template <int IN_, int BM_, int BN_, int WAVES_M_, int WAVES_N_, bool A_KC_, bool B_KC_, bool DIRECT_, bool EDGE_, int KB_, int STAGES_,
-          bool PINGPONG_ = false, bool TIMED_ = false, bool ANY_ = false>
+          bool PINGPONG_ = false, bool TIMED_ = false, bool ANY_ = false, bool CHECKED_ = false>
 struct MfmaConfig {
+    // CHECKED (an EDGE build): every chunk tested before it is fetched, see fills_checked
+    static constexpr bool CHECKED = CHECKED_;
+    static_assert(!CHECKED_ || EDGE_, "only the edge fill has tests");
+    using Checked = MfmaConfig<IN_, BM_, BN_, WAVES_M_, WAVES_N_, A_KC_, B_KC_, DIRECT_, EDGE_, KB_, STAGES_, PINGPONG_, TIMED_, ANY_, true>;
     // ANY (an EDGE build): operands of any size, leading dimension and alignment (see OperandTile::load_edge)
     static constexpr bool ANY = ANY_;
     static_assert(!ANY_ || EDGE_, "the any-shape fill is a form of the edge fill");
@@ -449,7 +453,8 @@ struct MfmaConfig {
     // end, and writes them to GemmArgs::stamps (phase times and the clock the engine ran at).
     static constexpr bool TIMED = TIMED_;
     // workgroups meant to share a CU: as many as the LDS allows, at most 2 waves per SIMD in all
-    static constexpr int WGS_PER_CU = (WAVES_M_ * WAVES_N_ <= 4 && 2 * STAGES_ * (BM_ + BN_) * KB_ <= 160 * 1024 && BM_ * BN_ <= 256 * 128) ? 2 : 1;
+    // (four of the 64 x 64 edge kernels, which is 128 registers each: asked for two, the compiler took up to 164)
+    static constexpr int WGS_PER_CU = EDGE_ && BM_ * BN_ <= 64 * 64 ? 4 : (WAVES_M_ * WAVES_N_ <= 4 && 2 * STAGES_ * (BM_ + BN_) * KB_ <= 160 * 1024 && BM_ * BN_ <= 256 * 128) ? 2 : 1;
     static constexpr int IN = IN_, BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, KB = KB_, STAGES = STAGES_;
     static constexpr bool A_KC = A_KC_, B_KC = B_KC_, DIRECT = DIRECT_, EDGE = EDGE_;
     static constexpr int NT = WAVES_M * WAVES_N * 64;
@@ -505,6 +510,33 @@ template <typename Cfg>
 constexpr bool mfma_takes_short_m()
 {
     return Cfg::DIRECT && !Cfg::EDGE && Cfg::A_KC && OperandTile<Cfg::IN, Cfg::BM, Cfg::A_KC, Cfg::NT, Cfg::KB>::EVEN_SPLIT;
+}
+
+// Register-staged fills: K tiles on their way in registers (see the kernel's loop).
+// (the checked build of the int8 64 x 64 tiles: with three its test of 16 chunks spilled at 128 registers, and 57 x (326x48x128)
+// took 4.7 us instead of 4.4)
+template <typename Cfg>
+constexpr int staged_ring()
+{
+    return !Cfg::EDGE ? 1 : Cfg::BM * Cfg::BN <= 64 * 64 ? (Cfg::CHECKED && Cfg::IN == IN_I8 ? 2 : 3) : Cfg::BM * Cfg::BN <= 128 * 128 ? 2 : 1;
+}
+
+// Edge kernels: whether a problem runs on the build that tests every chunk before it fetches it.  It has to where the rows of an
+// operand are shorter than a chunk (where K is split, in any slice); and the smallest problems do, K of no more tiles than are
+// fetched before the first is waited for, where no chunk straddles the end of a row and what is outside need not be fetched
+// (6016x16x128 bf16 3.3 us, 4.2 with the other loop; 80x128x48 3.4 / 4.3; where chunks do straddle the other is ahead
+// however short K is: 1280x6214x96 fp16 14.2 / 10.3).
+// (Kernels of their own: both loops in one kernel were the registers of the larger for either -- the int8 64 x 64 tiles took 132,
+// three workgroups to a CU, and the 256 x 256 ones spilled 132 bytes per lane instead of 68: 53 x (456x1961x256) fp16
+// 93.9 us together, 84.7 apart, 1024x50257x768 158 / 149, 57 x (326x48x128) int8 4.7 / 4.4, 6016x16x128 fp16 3.8 / 3.6.)
+template <typename Cfg>
+bool fills_checked(const GemmArgs& a)
+{
+    constexpr int ES = InTraits<Cfg::IN>::ES, VEC = 16 / ES, BK = Cfg::KB / ES;
+    const int k_least = a.k_last > 0 && a.k_last < a.K ? a.k_last : a.K;
+    if ((Cfg::A_KC ? k_least : a.M) < VEC || (Cfg::B_KC ? k_least : a.N) < VEC) return true;
+    const int ext_a = Cfg::A_KC ? a.K : a.M, ext_b = Cfg::B_KC ? a.K : a.N;
+    return (a.K + BK - 1) / BK <= staged_ring<typename Cfg::Checked>() && ext_a % VEC == 0 && ext_b % VEC == 0;
 }
 
 template <typename Cfg>
@@ -791,61 +823,80 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
         // multiplied in a fraction of the time its load takes: with one tile in flight a k-step costs the memory latency).
         // Tile t sits in slot t % RING; the slot of the tile that has just gone to LDS is refilled with tile t + RING.
         // The waits for memory count the loads that are younger than the ones waited for, and the compiler counts none that
-        // stand behind a branch: the loop that fetches without one keeps the ring full, the last tiles are a copy of it with tests.
-        constexpr int RING = EDGE ? (BM * BN <= 64 * 64 ? 3 : BM * BN <= 128 * 128 ? 2 : 1) : 1;
+        // stand behind a branch: the loop that fetches without one keeps the ring full, the last tiles (at most 2 RING - 1) come
+        // after it with tests, written out (as a loop they had a ring of registers of their own: 164 in all, not 110 to 125).
+        constexpr int RING = staged_ring<Cfg>();
+        constexpr bool CHECKED = Cfg::CHECKED;
         i32x4 ra[RING][TA::PER_THREAD], rb[RING][TB::PER_THREAD];
-        // (CHECKED: chunk by chunk, see OperandTile::load_checked)
-        auto staged_loop = [&](auto checked_tag) __attribute__((always_inline)) {
-            constexpr bool CHECKED = decltype(checked_tag)::value;
-            auto load = [&](int r, int kt) __attribute__((always_inline)) {
-                if constexpr (!EDGE) {
-                    TA::load_global(ra[r], Ab, m0, kt * BK, lda, tid);
-                    TB::load_global(rb[r], Bb, n0, kt * BK, ldb, tid);
-                } else if constexpr (CHECKED) {
-                    TA::template load_checked<Cfg::ANY>(ra[r], Ab, m0, kt * BK, lda, p.M, p.K, tid);
-                    TB::template load_checked<Cfg::ANY>(rb[r], Bb, n0, kt * BK, ldb, p.N, p.K, tid);
-                } else {
-                    TA::template load_edge<Cfg::ANY>(ra[r], Ab, m0, kt * BK, lda, p.M, p.K, tid);
-                    TB::template load_edge<Cfg::ANY>(rb[r], Bb, n0, kt * BK, ldb, p.N, p.K, tid);
+        auto load = [&](int r, int kt) __attribute__((always_inline)) {
+            if constexpr (!EDGE) {
+                TA::load_global(ra[r], Ab, m0, kt * BK, lda, tid);
+                TB::load_global(rb[r], Bb, n0, kt * BK, ldb, tid);
+            } else if constexpr (CHECKED) {
+                TA::template load_checked<Cfg::ANY>(ra[r], Ab, m0, kt * BK, lda, p.M, p.K, tid);
+                TB::template load_checked<Cfg::ANY>(rb[r], Bb, n0, kt * BK, ldb, p.N, p.K, tid);
+            } else {
+                TA::template load_edge<Cfg::ANY>(ra[r], Ab, m0, kt * BK, lda, p.M, p.K, tid);
+                TB::template load_edge<Cfg::ANY>(rb[r], Bb, n0, kt * BK, ldb, p.N, p.K, tid);
+            }
+        };
+        auto store = [&](int r, int kt) __attribute__((always_inline)) {
+            char* to = smem + (kt & 1) * STAGE_BYTES;
+            if constexpr (Cfg::ANY && !CHECKED) {
+                if (TA::straddles(m0, kt * BK, p.M, p.K)) TA::realign(ra[r], m0, kt * BK, p.M, p.K, tid);
+                if (TB::straddles(n0, kt * BK, p.N, p.K)) TB::realign(rb[r], n0, kt * BK, p.N, p.K, tid);
+            }
+            TA::store_lds(ra[r], to, tid);
+            TB::store_lds(rb[r], to + TA::TILE_BYTES, tid);
+            if constexpr (EDGE && !CHECKED) {
+                if ((kt + 1) * BK > p.K) {
+                    TA::zero_past_k(to, kt * BK, p.K, tid);
+                    TB::zero_past_k(to + TA::TILE_BYTES, kt * BK, p.K, tid);
                 }
-            };
-            auto store = [&](int r, int kt) __attribute__((always_inline)) {
-                char* to = smem + (kt & 1) * STAGE_BYTES;
-                if constexpr (Cfg::ANY && !CHECKED) {
-                    if (TA::straddles(m0, kt * BK, p.M, p.K)) TA::realign(ra[r], m0, kt * BK, p.M, p.K, tid);
-                    if (TB::straddles(n0, kt * BK, p.N, p.K)) TB::realign(rb[r], n0, kt * BK, p.N, p.K, tid);
-                }
-                TA::store_lds(ra[r], to, tid);
-                TB::store_lds(rb[r], to + TA::TILE_BYTES, tid);
-                if constexpr (EDGE && !CHECKED) {
-                    if ((kt + 1) * BK > p.K) {
-                        TA::zero_past_k(to, kt * BK, p.K, tid);
-                        TB::zero_past_k(to + TA::TILE_BYTES, kt * BK, p.K, tid);
-                    }
-                }
-            };
-            auto multiply = [&](int kt) __attribute__((always_inline)) {
-                const char* cur = smem + (kt & 1) * STAGE_BYTES;
-                load_first_frags(cur, cur + TA::TILE_BYTES);
-                mma_tile(cur, cur + TA::TILE_BYTES, cur, cur + TA::TILE_BYTES, std::false_type{}, std::false_type{}, 0, 0);
-            };
+            }
+        };
+        auto multiply = [&](int kt) __attribute__((always_inline)) {
+            const char* cur = smem + (kt & 1) * STAGE_BYTES;
+            load_first_frags(cur, cur + TA::TILE_BYTES);
+            mma_tile(cur, cur + TA::TILE_BYTES, cur, cur + TA::TILE_BYTES, std::false_type{}, std::false_type{}, 0, 0);
+        };
+        // (fp32: the first tiles without a branch as well, so that the first goes to LDS while the others are on their way:
+        // 1472x674x576 18.0 -> 17.1 us.  16-bit inputs gain 1 % that way and lose 1 % where K is short; int8 would spill.)
+        constexpr bool FULL_START = EDGE && !CHECKED && ES == 4 && RING > 1;
+        if (FULL_START && KT >= RING) {
+#pragma unroll
+            for (int r = 0; r < RING; ++r) load(r, r);
+        } else {
 #pragma unroll
             for (int r = 0; r < RING; ++r)
                 if (r < KT) load(r, r);
-            store(0, 0);
-            __syncthreads();
-            int kt0 = 0;
-            if constexpr (!CHECKED) {
-                for (; kt0 + 2 * RING <= KT; kt0 += RING) {
+            if constexpr (FULL_START) __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
+        }
+        store(0, 0);
+        __syncthreads();
+        int kt0 = 0;
+        if constexpr (!CHECKED) {
+            for (; kt0 + 2 * RING <= KT; kt0 += RING) {
 #pragma unroll
-                    for (int u = 0; u < RING; ++u) {
-                        load(u, kt0 + u + RING);
-                        multiply(kt0 + u);
-                        store((u + 1) % RING, kt0 + u + 1);
-                        __syncthreads();
-                    }
+                for (int u = 0; u < RING; ++u) {
+                    load(u, kt0 + u + RING);
+                    multiply(kt0 + u);
+                    store((u + 1) % RING, kt0 + u + 1);
+                    __syncthreads();
                 }
             }
+        }
+        if constexpr (EDGE && !CHECKED) {
+#pragma unroll
+            for (int u = 0; u < 2 * RING - 1; ++u) {
+                const int kt = kt0 + u;
+                if (kt >= KT) break;
+                if (u < RING - 1 && kt + RING < KT) load(u, kt + RING);
+                multiply(kt);
+                if (kt + 1 < KT) store((u + 1) % RING, kt + 1);
+                __syncthreads();
+            }
+        } else {
             for (; kt0 < KT; kt0 += RING) {
 #pragma unroll
                 for (int u = 0; u < RING; ++u) {
@@ -857,19 +908,11 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
                     __syncthreads();
                 }
             }
-        };
-        if constexpr (EDGE) {
-            // Chunk by chunk: rows shorter than a chunk; and the smallest problems, K of no more tiles than are fetched before
-            // the first is waited for, where no chunk straddles the end of a row and what is outside need not be fetched
-            // (6016x16x128 bf16 3.3 us, 4.2 with the other loop; 80x128x48 3.4 / 4.3; where chunks do straddle the other is ahead
-            // however short K is: 1280x6214x96 fp16 14.2 / 10.3).
-            constexpr int VEC = 16 / ES;
-            const int ext_a = A_KC ? p.K : p.M, ext_b = B_KC ? p.K : p.N;
-            if (ext_a < VEC || ext_b < VEC || (KT <= RING && ext_a % VEC == 0 && ext_b % VEC == 0)) staged_loop(std::true_type{});
-            else staged_loop(std::false_type{});
-        } else {
-            staged_loop(std::false_type{});
         }
+        // Nothing is in flight here; said for the compiler, which else takes registers of the ring for such, whatever it keeps in
+        // them by then, and waits for memory in front of every store of the write-back (190 waits in the int8 128 x 128 kernel, each
+        // of which also waits for the stores before: 190 x (320x960x32) 84.5 us, 61.4 without).
+        __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
     }
 
     stamp(2);
@@ -947,7 +990,14 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
                 return sum + __uint_as_float(bits) * c_mul;
             }
         };
-        auto offset_of = [&](int i, int r, int j) { return lane_off + ((unsigned)(i * 32 + (r >> 2) * 8 + (r & 3)) * row_bytes + ((unsigned)(j * 32) << sh)); };
+        // (edge kernels: the product in a scalar register.  As a 64-bit multiply-add of the vector unit, which is what the compiler makes of the
+        // sum else, it takes a register pair whose upper half, which nobody reads, may be the target of a load in flight -- and waits
+        // for it: 256x264x312 fp16 accumulating 8.2 us, 6.0 without)
+        auto offset_of = [&](int i, int r, int j) {
+            unsigned down = (unsigned)(i * 32 + (r >> 2) * 8 + (r & 3)) * row_bytes;
+            if constexpr (EDGE) asm("" : "+s"(down));
+            return lane_off + down + ((unsigned)(j * 32) << sh);
+        };
         if constexpr (TM * TN * 16 <= 64) {
             // A small wave tile (64 sums per lane) has the registers for a second copy: all of its loads are issued before the
             // first is used, so the tile of C costs one trip through memory instead of one per eight loads (left to the
@@ -1145,6 +1195,9 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
 template <typename Cfg>
 hipError_t launch_mfma(const GemmArgs& a, hipStream_t stream, LaunchGeom* geom, bool dry_run)
 {
+    if constexpr (Cfg::EDGE && !Cfg::CHECKED) {
+        if (fills_checked<Cfg>(a)) return launch_mfma<typename Cfg::Checked>(a, stream, geom, dry_run);
+    }
     auto kern = gemm_mfma_kernel<Cfg>;
     // an int8 C is written in 16-byte pieces of 16-byte aligned rows; no kernel here has a path for anything else
     if (a.out_type == T_I8 && (a.c_rs % 16 || ((size_t)a.C & 15) || (a.batch > 1 && a.c_bs % 16))) return hipErrorInvalidValue;

@@ -41,3 +41,20 @@ def test_a_file_without_a_known_kernel_fails_the_build(tmp_path, capsys):
     assert check.main([str(listing)]) == 0
     assert check.main([str(path), str(listing)]) == 1
     assert "unit.resources.txt" in capsys.readouterr().err
+
+
+def _staged(edge, any_alignment=True):
+    return (f"_ZN6acc95016gemm_mfma_kernelINS_10MfmaConfigILi2ELi{edge}ELi{edge}ELi2ELi2ELb1ELb0ELb0ELb1ELi128ELi2ELb0ELb0ELb{int(any_alignment)}ELb0EEEEEvPKv")
+
+
+@pytest.mark.parametrize("edge,vgprs,scratch,fails", [(64, 128, 0, False), (64, 132, 0, True), (64, 128, 8, True), (128, 222, 0, False), (128, 222, 16, True),
+                                                      (256, 256, 68, False), (256, 254, 132, True)])
+def test_registers_and_scratch_of_the_register_staged_kernels(edge, vgprs, scratch, fails, tmp_path, capsys):
+    """A CU holds four workgroups of the 64 x 64 tiles (the kernel choice counts on it), and none of these kernels may spill
+    more than they do."""
+    check, path = _check(), tmp_path / "unit.resources.txt"
+    form = "remark: ./gemm_mfma.h:512:0: {}"
+    own = _remarks(form, [(_staged(edge), scratch)]).replace("VGPRs: 256", f"VGPRs: {vgprs}")
+    path.write_text(_remarks(form, [(W4, 0)]) + own)
+    assert check.main([str(path)]) == int(fails)
+    assert not fails or f"{vgprs} vector registers" in capsys.readouterr().err
