@@ -638,19 +638,34 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
     if (variant == ACC950_VARIANT_AUTO) {
         const int sv = auto_skinny_variant(pb);
         // 17 to 32 rows against a B of 32 MB and more, 16-bit types: the streaming kernel fetches half as many bytes of A as of B
-        // by then; 64 x 64 tiles with direct fills are ahead while their slices fill the chip (us, streaming kernel / tiles: bf16
-        // 31x4416x9792 23.2 / 21.5, 31x20800x4544 58.0 / 39.5, 30x6336x30784 135.6 / 74.0, 29x10176x6656 33.5 / 27.9, fp16
-        // 26x21632x2048 26.2 / 19.7; a smaller B is not: 22x5056x1408 6.4 / 7.9, 18x3904x2752 8.8 / 9.4; nor are tiles too many to split and too few
-        // to fill the chip, or more than it holds: fp16 29x11712x7168 35.8 / 45.5, 25x37056x6912 104.5 / 115.3)
-        if (sv >= 0 && k_splits == 0 && pb.g.M > 16 && pb.g.in_type != T_I8 && streamed_b(pb, (int64_t)32 << 20) && !streamed_b(pb, (int64_t)768 << 20)) {
+        // by then; 64 x 64 tiles with direct fills are ahead where their slices stay long beside what the sums of the slices cost,
+        // which the streaming kernel's whole columns need not pay (us, streaming kernel / tiles, fp16, M rows: 32x64x262144 92 / 55
+        // in 32 slices, 17x4096x4096 11.8 / 11.5 in four, 24x5056x8192 23.9 / 19.7 in six; two slices or none lose, 31x9600x1792
+        // 8.9 / 9.7, 17x6400x2624 9.6 / 11.0, 24x9600x2048 9.3 / 11.7, and so do three short ones from 88 tiles on, 17x6080x3264 1.22
+        // times as long, 17x6400x3584 15.3 / 14.6; from 136 tiles on the streaming kernel has enough workgroups by itself while rows and K are
+        // few, 17x8960x5632 23.7 / 24.2, 24x8960x4096 20.0 / 19.8, 32x8960x4096 22.2 / 20.7, 17x9984x12288 level; rows of B a
+        // multiple of 16 KB apart cost the tiles a fifth, which fetch one line of 64 of them: 17x8128x3584 level, 17x8192x3584 15.9 / 18.9, 32x8192x8192 34.8 / 33.5).
+        // 300 to 400 tiles, unsplit, fill the chip by themselves (17 and 32 rows, K = 1024 to 8192, N = 19264 to 25600: 0.65 to 0.87 of
+        // the streaming kernel's time; 160 to 299 do not, 29x11712x7168 35.8 / 45.5, and more are a second round: 25x37056x6912 104.5 / 115.3),
+        // up to where that kernel's 256-column blocks in two slices do as well: 17x24576x8192 79.2 / 89.4.
+        // Not for an fp32 result: the streaming kernel sums K in four waves side by side, the tiles in one chain (2-norm of the
+        // error, 31x20800x4544 fp16: 2.2e-7 / 4.3e-7; see auto_skinny_splits).
+        // (a smaller B is not for the tiles: 22x5056x1408 6.4 / 7.9, 18x3904x2752 8.8 / 9.4)
+        if (sv >= 0 && k_splits == 0 && pb.g.M > 16 && pb.g.in_type != T_I8 && pb.g.out_type != T_F32 && streamed_b(pb, (int64_t)32 << 20) && !streamed_b(pb, (int64_t)768 << 20)) {
             const int mv = auto_mfma_variant(pb, 64, true);
             int n = 0;
             const MfmaVariant* tab = mfma_table(pb.g.in_type, &n);
             const int tiles = (pb.g.N + 63) / 64;
-            if (mv >= 0 && tab[mv].direct && (tiles < 160 || (tiles >= 300 && tiles <= 400 && pb.g.K <= 8192))) {
-                c->variant = mv;
-                c->splits = streamed_b_splits(tab[mv], pb, max_split_floats);
-                return ACC950_OK;
+            const int64_t k_rows = (int64_t)pb.g.K * pb.g.M;
+            bool pays = tiles >= 300 && (tiles <= 376 ? pb.g.K <= 8192 : tiles <= 400 && pb.g.K < 8192);
+            if (tiles < 160) pays = pb.g.b_rs % 8192 == 0 ? k_rows >= 250000 : tiles < 88 || (pb.g.K >= 3584 && (tiles < 136 || k_rows >= 120000));
+            if (pays && mv >= 0 && tab[mv].direct) {
+                const int slices = streamed_b_splits(tab[mv], pb, max_split_floats);
+                if (tiles >= 160 || slices >= 3) {
+                    c->variant = mv;
+                    c->splits = slices;
+                    return ACC950_OK;
+                }
             }
         }
         if (sv >= 0) {

@@ -210,6 +210,27 @@ def test_choices_of_the_cost_model():
     assert "64x64" in n and "fill=direct" in n and ks == 1                              # (90 MB: the general rule's tiles, 344 of them)
 
 
+@pytest.mark.parametrize("M,N,K,tile,slices", [
+    (31, 4416, 9792, "64x64", 7), (17, 4096, 4096, "64x64", 4), (32, 64, 262144, "64x64", 32), (24, 5056, 8192, "64x64", 6), (17, 6400, 3584, "64x64", 3),
+    (31, 20800, 4544, "64x64", 1),          # (325 tiles: unsplit, they fill the chip)
+    (31, 9600, 1792, None, 1), (24, 9600, 2048, None, 1), (17, 6400, 2624, None, 1),  # (two slices or none: the streaming kernel)
+    (17, 6080, 3264, None, None), (17, 8960, 5632, None, None), (32, 8960, 5632, "64x64", 3),
+    (18, 8192, 2048, None, None), (17, 8192, 8192, None, None), (32, 8192, 8192, "64x64", 4),   # (rows of B 16 KB apart)
+    (29, 11712, 7168, None, None), (25, 37056, 6912, None, None), (17, 24576, 8192, None, None),
+    (22, 5056, 1408, None, None),           # (a B of less than 32 MB)
+])
+def test_17_to_32_rows_against_a_large_b(M, N, K, tile, slices):
+    """Tiles in slices or the streaming kernel, as measured; an fp32 result and int8 keep the streaming kernel, whose sums are shorter chains."""
+    from accera_amd import tune
+    for t in (_lib.F16, _lib.BF16):
+        v, ks = tune.own_choice(t, t, M, N, K, False, False, 1.0, 0.0)
+        name = _lib.variant_name(v)
+        assert ("mfma 64x64" in name and "fill=direct" in name) if tile else "skinny" in name, name
+        assert slices is None or ks == slices, (name, ks)
+        assert "skinny" in _lib.variant_name(tune.own_choice(t, _lib.F32, M, N, K, False, False, 1.0, 0.0)[0])
+    assert "skinny" in _lib.variant_name(tune.own_choice(_lib.I8, _lib.I32, M, N, K, False, False, 1.0, 0.0)[0])
+
+
 def test_bound_call_handles_without_launching():
     """acc950_bind validates and chooses once; handles are reused after acc950_unbind; unknown handles
     are reported.  (No launch here: there is no GPU on the CPU test tier.)"""

@@ -543,6 +543,27 @@ def test_many_column_problems_with_few_rows_stream_b_once(in_type, out_type, M, 
     run_case(in_type, out_type, M, N, K, b_layout=b_layout, seed=M + N % 91, dist="normal", prologue=prologue)
 
 
+@pytest.mark.parametrize("in_type,M,N,K,slices,prologue", [
+    ("bf16", 31, 4416, 9792, 7, ora.PRO_SET0), ("f16", 17, 2048, 8192, 8, ora.PRO_NONE), ("f16", 32, 64, 262144, 32, ora.PRO_SET0),
+    ("f16", 25, 20800, 1024, 1, ora.PRO_NONE), ("bf16", 32, 6392, 3584, 3, ora.PRO_SET0),
+])
+def test_17_to_32_rows_on_tiles_in_slices(in_type, M, N, K, slices, prologue):
+    """The automatic choice and its results, through the allocating entry point and through the one that allocates nothing."""
+    import torch
+    from accera_amd import _lib, tune
+    t = getattr(_lib, in_type.upper())
+    v, ks = tune.own_choice(t, t, M, N, K, False, False, 1.0, 1.0 if prologue == ora.PRO_NONE else 0.0)
+    assert "mfma 64x64" in _lib.variant_name(v) and ks == slices, (_lib.variant_name(v), ks)
+    run_case(in_type, in_type, M, N, K, seed=M + N % 91, dist="normal", prologue=prologue)
+    rng = np.random.default_rng(N)
+    A, B, C0 = make_input(rng, (M, K), in_type, "normal"), make_input(rng, (K, N), in_type, "normal"), make_c0(rng, (M, N), in_type, "normal")
+    dA, dB, dC = to_device(A, in_type), to_device(B, in_type), to_device(C0, in_type)
+    _lib.check(_lib.lib().acc950_gemm_ops_static(t, t, M, N, K, dA.data_ptr(), K, 1, dB.data_ptr(), N, 1, dC.data_ptr(), N, 1, prologue, 0.0,
+                                                 _lib.EPILOGUE_RELU, 0.0, _lib.VARIANT_AUTO, 0, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert_matches(to_host(dC, in_type), ora.gemm_relu_exact(A, B, C0, in_type, in_type, prologue, ora.EPI_RELU), in_type, K)
+
+
 @pytest.mark.parametrize("out_type", ["i32", "i16", "i8"])
 def test_skinny_int8_streaming_kernels(out_type):
     """int8 rows of A against a large row-major int8 B on the streaming kernels of the matrix-core family
