@@ -303,21 +303,31 @@ int auto_skinny_splits(int variant, const GemmArgs& g)
     const int64_t all_blocks = (int64_t)skinny_column_blocks(variant, g.N) * (g.batch > 1 ? g.batch : 1);
     const int blocks = all_blocks > 4096 ? 4096 : (int)all_blocks;
     if (blocks >= 128) return 1;
-    // The fewest microseconds of: a slice of a block at the rate one CU streams such pieces (out of HBM 36 KB / us, int8 half
-    // lines 20; a B of less than 32 MB, mostly out of the Infinity Cache, 62 less half a KB per row, and 34), never less than all of B at the chip's rate (5.5, 4.2 MB / us), and for a split the second trip through
-    // memory, 3 us, 0.1 per row and 0.15 per slice.  Never more workgroups than CUs: a second round of a few costs as much as the first.
-    // (us, as many slices as gave at least 256 workgroups / this: fp16 22x5056x1408 11.1 in four / 6.4 unsplit, 18x3904x2752
-    // 11.8 in five / 8.8 unsplit, 16x1088x5440 11.1 in 16 / 9.4 in eight, bf16 8x3456x21952 42.2 in five / 28.9 in four, int8
-    // 15x5696x1536 8.8 in three / 5.1 unsplit)
+    const int max_splits = g.K / 256 > 0 ? g.K / 256 : 1;
+    // An fp32 result keeps about one workgroup per CU, whatever that costs: a slice is a chain of 32-bit additions, and the
+    // fewer there are the longer they get (2-norm of the error, 18x3904x2752 fp16: 1.0e-7 in five slices, 1.7e-7 unsplit; in a
+    // 16-bit result that is lost in its own rounding, 2e-4).
+    if (g.out_type == T_F32) return std::min((kComputeUnits + blocks - 1) / blocks, max_splits);
+    // The fewest microseconds of: a slice of a block at the rate one CU streams such pieces, never less than all of B at the
+    // chip's rate, which few workgroups do not reach; and for a split the second trip through memory.  Never more workgroups
+    // than CUs: a second round of a few costs as much as the first.  A CU's rate falls from what the Infinity Cache gives to
+    // what HBM gives while B grows from 24 to 60 MB (int8: 20 to 48, pieces of half a line); rows of B a multiple of 4 KB
+    // apart cost a tenth.  Fitted to 1078 problems of 1 to 32 rows, 256 to 7936 columns and K = 512 to 16384, each in one to 16 slices:
+    // 1.4 % off the best of them on average; as many slices as give 256 workgroups, 33 %
+    // (us, so many slices / this: fp16 22x5056x1408 11.1 in four / 6.4 unsplit, 18x3904x2752 11.8 in five / 8.8 unsplit, 16x1088x5440 11.1 in 16 / 9.4 in
+    // six, bf16 8x3456x21952 42.2 in five / 28.9 in four, int8 15x5696x1536 8.8 in three / 5.1 unsplit, 28x4096x6144 11.5 in four / 12.1 in three, 17.9 unsplit).
     const bool i8 = g.in_type == T_I8;
-    const bool cached = (int64_t)g.K * g.N * elem_size(g.in_type) * (g.batch > 1 ? g.batch : 1) < ((int64_t)32 << 20);
-    const double cu_rate = i8 ? (cached ? 34e3 : 20e3) : (cached ? 62e3 - 0.5e3 * g.M : 36e3);
-    const double k_us = (double)g.K * skinny_variant(variant).cols * elem_size(g.in_type) / cu_rate;
-    const double chip_us = (double)g.K * g.N * elem_size(g.in_type) * (g.batch > 1 ? g.batch : 1) / (i8 ? 4.2e6 : 5.5e6);
+    const double bytes = (double)g.K * g.N * elem_size(g.in_type) * (g.batch > 1 ? g.batch : 1), mb = bytes / (1 << 20);
+    const double uncached = std::min(1.0, std::max(0.0, i8 ? (mb - 20) / 28 : (mb - 24) / 36));
+    const double from_cache = i8 ? 32.5e3 : 61.5e3 - 430.0 * g.M, from_hbm = i8 ? 22e3 : 31e3; // bytes per us
+    const double pitch = g.b_rs * elem_size(g.in_type) % 4096 == 0 ? 0.9 : 1.0;
+    const double k_us = (double)g.K * skinny_variant(variant).cols * elem_size(g.in_type) / ((from_cache + (from_hbm - from_cache) * uncached) * pitch);
+    const double chip_us = bytes / ((i8 ? 5.5e6 : 6.1e6) * pitch);
     int best = 1;
     double best_us = 0;
-    for (int s = 1; s == 1 || (s * blocks <= kComputeUnits && g.K / s >= 256); ++s) {
-        const double us = std::max(k_us / s, chip_us) + (s > 1 ? 3.0 + 0.1 * g.M + 0.15 * s : 0.0);
+    for (int s = 1; s == 1 || (s * blocks <= kComputeUnits && s <= max_splits); ++s) {
+        const double full = 0.75 + 0.25 * s * blocks / kComputeUnits;
+        const double us = std::max(k_us / s, chip_us / full) + (s == 1 ? 0.0 : i8 ? 2.8 + 0.4 * s : 1.6 + 0.035 * g.M + 0.3 * s);
         if (s == 1 || us < best_us) { best = s; best_us = us; }
     }
     return best;

@@ -231,6 +231,24 @@ def test_17_to_32_rows_against_a_large_b(M, N, K, tile, slices):
     assert "skinny" in _lib.variant_name(tune.own_choice(_lib.I8, _lib.I32, M, N, K, False, False, 1.0, 0.0)[0])
 
 
+def test_slices_of_the_streaming_kernels():
+    """As many as pay, not as many as there are CUs for; an fp32 result keeps the many (its sums are shorter chains)."""
+    from accera_amd import tune
+    own = lambda *a: tune.own_choice(*a, False, False, 1.0, 0.0)
+    narrow = next(_lib.VARIANT_SKINNY_BASE + i for i in range(_lib.num_skinny_variants()) if "mfma cols/wg=64" in _lib.variant_name(_lib.VARIANT_SKINNY_BASE + i))
+    for (M, N, K), slices, many in [((22, 5056, 1408), 1, 4), ((18, 3904, 2752), 1, 5), ((28, 3144, 3904), 3, 6), ((16, 1088, 5440), 5, 16), ((26, 1752, 1984), 4, 7)]:
+        assert own(_lib.F16, _lib.F16, M, N, K) == (narrow, slices)
+        assert own(_lib.BF16, _lib.BF16, M, N, K) == (narrow, slices)
+        assert own(_lib.F16, _lib.F32, M, N, K) == (narrow, many)
+    assert own(_lib.I8, _lib.I32, 28, 4096, 6144)[1] in (3, 4)   # (17.9 us unsplit, 11.5 in four)
+    assert own(_lib.I8, _lib.I32, 15, 5696, 1536) == (narrow, 1)
+    # never more than a workgroup per CU, nor slices of less than 256 rows of B
+    for N in (64, 512, 1984, 4096, 8128):
+        for K in (256, 500 // 32 * 32, 4096, 32768):
+            s = own(_lib.F16, _lib.F16, 8, N, K)[1]
+            assert s == 1 or (s * -(-N // 64) <= 256 and K // s >= 256)
+
+
 def test_bound_call_handles_without_launching():
     """acc950_bind validates and chooses once; handles are reused after acc950_unbind; unknown handles
     are reported.  (No launch here: there is no GPU on the CPU test tier.)"""
