@@ -577,7 +577,9 @@ int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats
     int64_t want = std::min<int64_t>(target / tiles, 32);
     const int64_t b_bytes = (int64_t)g.N * g.K * elem_size(g.in_type);
     while (want > 1 && (g.K / want < 960 || want * (int64_t)g.M * g.N * 4 > b_bytes / 6)) --want;
-    if (v.bm * v.bn > 128 * 128) // (the 256 x 256 tiles, whose partial sums weigh most: a power of two)
+    // (the 256 x 256 tiles, whose partial sums weigh most: a power of two; and a K-contiguous B from 16 slices on:
+    // 48x768x23744 15.7 us in 16, 17.1 in 24, 2x1664x23744 20.6 in 16, 22.7 in 19)
+    if (v.bm * v.bn > 128 * 128 || (v.b_kc && want > 16))
         while (want & (want - 1)) want &= want - 1;
     if (want < 2) return 1;
     if ((size_t)want * (size_t)g.M * (size_t)g.N > ((size_t)1 << 24)) return 1; // 64 MiB of partial sums at most without being asked

@@ -249,6 +249,14 @@ def test_slices_of_the_streaming_kernels():
             assert s == 1 or (s * -(-N // 64) <= 256 and K // s >= 256)
 
 
+def test_slices_against_a_k_contiguous_b():
+    """Any number of slices up to 16, powers of two from there on."""
+    from accera_amd import tune
+    for (M, N, K), slices in [((48, 768, 23744), 16), ((2, 1664, 23744), 16), ((63, 2048, 6144), 6), ((48, 2560, 16384), 12), ((68, 5376, 23552), 6), ((11, 6208, 3904), 4)]:
+        v, ks = tune.own_choice(_lib.F16, _lib.F16, M, N, K, False, True, 1.0, 0.0)
+        assert "fill=direct" in _lib.variant_name(v) and ks == slices, (M, N, K, ks)
+
+
 def test_bound_call_handles_without_launching():
     """acc950_bind validates and chooses once; handles are reused after acc950_unbind; unknown handles
     are reported.  (No launch here: there is no GPU on the CPU test tier.)"""
