@@ -340,6 +340,30 @@ int auto_skinny_splits(int variant, const GemmArgs& g)
 // others in table order; partial tiles only fit the edge kernel.
 bool streamed_b(const Problem& pb, int64_t least_bytes);
 
+// Problems that only the register-staged kernels take, K of 64 (int8 128) to 2048 bytes: 64 x 64 or 128 x 128 tiles (the edge
+// length; 0: neither rule nor measurement is about such a problem).  Microseconds of a workgroup -- its start, its steps of 128 bytes
+// of K, its write-back, which weighs double for 32-bit results and four times where C is read as well -- times the rounds of them, of which a last one that is not
+// full costs in part: 512 of the small tiles, 256 of the large ones to a round.  Fitted to 520 problems, 100 tiles and more, batches among them; on the
+// 397 of this range 1.2 % off the better one on average, the small ones always 3.1 %
+// (us, 128 x 128 / 64 x 64: fp16 704x3136x48 6.1 / 4.2, 2112x973x448 11.1 / 9.5, 5808x384x496 11.2 / 10.2; but bf16 16 x (72x1144x848) 15.9 / 24.6,
+// fp16 5184x3972x73 with an fp32 result 26.5 / 35.7, 824x4072x888 16.0 / 20.8).
+int staged_short_k_tile(const Problem& pb, const MfmaVariant* tab, int n)
+{
+    const GemmArgs& g = pb.g;
+    const int64_t k_bytes = (int64_t)g.K * elem_size(g.in_type), batch = g.batch > 1 ? g.batch : 1;
+    const int64_t small = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch, large = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
+    if (g.in_type == T_F32 || k_bytes < (g.in_type == T_I8 ? 128 : 64) || k_bytes > 2048 || small * k_bytes > 3000000) return 0;
+    for (int i = 0; i < n; ++i)
+        if (tab[i].direct && (tab[i].w4 || g.M >= tab[i].bm || streamed_b(pb, (int64_t)16 << 20)) && mfma_can_take(tab[i], pb)) return 0;
+    const double steps = (double)((k_bytes + 127) / 128), out = (elem_size(g.out_type) == 4 ? 2 : 1) * (g.prologue == PRO_SET ? 1 : 4);
+    const auto rounds = [](int64_t tiles, int64_t slots, double whole) {
+        return tiles <= slots ? 1.0 : whole * (double)((tiles + slots - 1) / slots) + (1 - whole) * (double)tiles / (double)slots;
+    };
+    const double us64 = 1.6 + (1.0 + 0.65 * steps + 0.25 * out) * rounds(small, 2 * kComputeUnits, 0.7);
+    const double us128 = 2.4 + (2.0 + 0.85 * steps + 0.45 * out) * rounds(large, kComputeUnits, 0.5);
+    return us64 < us128 ? 64 : 128;
+}
+
 // only_tile: 0, or the edge length of the (square) tiles to choose among.  short_rows: also the 64-row tiles with direct fills
 // on fewer rows than they have, whatever the size of B.
 int auto_mfma_variant(const Problem& pb, int only_tile = 0, bool short_rows = false)
@@ -350,26 +374,20 @@ int auto_mfma_variant(const Problem& pb, int only_tile = 0, bool short_rows = fa
     int best = -1;
     double best_cost = 0;
     int best_rank = 0;
-    // Problems that only the register-staged kernels take, K of 64 (int8 128) to 2048 bytes: the 64 x 64 tiles, of which a CU holds four,
-    // hide each other's fetches and are ahead of the 128 x 128 ones whatever their number (us, 128 x 128 / 64 x 64: fp16
-    // 704x3136x48 8.5 / 5.4, 596x3840x696 18.6 / 15.0, 4936x640x112 7.6 / 6.1, 5808x384x496 11.5 / 10.7, bf16 2112x973x448 with
-    // a column-major A 14.5 / 11.6, 6688x768x933 36.1 / 31.8; int8 320x960x32, 190 of them, all write-back, 71.9 / 91.2)
-    // (not with many long tiles, where what the larger ones save in fetches counts: fp16 3712x5694x912 87 / 110)
-    const int64_t k_bytes = (int64_t)pb.g.K * elem_size(pb.g.in_type);
-    const int64_t small_tiles = (int64_t)((pb.g.M + 63) / 64) * ((pb.g.N + 63) / 64) * (pb.g.batch > 1 ? pb.g.batch : 1);
-    bool staged_short_k = k_bytes >= (pb.g.in_type == T_I8 ? 128 : 64) && k_bytes <= 2048 && small_tiles * k_bytes <= 3000000 && pb.g.in_type != T_F32;
-    for (int i = 0; i < n && staged_short_k; ++i)
-        if (tab[i].direct && (tab[i].w4 || pb.g.M >= tab[i].bm || streamed_b(pb, (int64_t)16 << 20)) && mfma_can_take(tab[i], pb)) staged_short_k = false;
+    const int staged_tile = only_tile ? 0 : staged_short_k_tile(pb, tab, n);
     for (int i = 0; i < n; ++i) {
         const MfmaVariant& v = tab[i];
         if (only_tile && (v.bm != only_tile || v.bn != only_tile)) continue;
+        if (staged_tile && v.edge && (v.bm * v.bn <= 64 * 64) != (staged_tile == 64)) continue;
         if (!mfma_can_take(v, pb)) continue;
         // (a tile with direct fills on fewer rows than it has: taken only where B has at least 16 MB, see streamed_b_tile --
         // elsewhere the choices stand as the sweeps of the reference's lists found them, none of whose rows is of this kind)
         if (!v.edge && !v.w4 && pb.g.M < v.bm && !short_rows && !streamed_b(pb, (int64_t)16 << 20)) continue;
-        // (the any-alignment form on 256 x 256 tiles pays where the K-contiguous operands' rows are 16 bytes aligned and the
-        // odd size is N or M -- 4096x50257x4096 with a row-major B: 2397 us on 128 x 128 tiles, 1832 on these -- and loses
-        // where every row of a K-contiguous operand starts unaligned: 4100^3 326 / 361, 1234x5678x4321 205 / 256)
+        // (the any-alignment form on 256 x 256 tiles pays where the K-contiguous operands' rows are 16 bytes aligned, the
+        // odd size is N or M and the tiles are many -- fp16, us, 128 x 128 tiles / these: 4096x50257x4096 with a row-major B 2124 / 1806,
+        // 2048x32003x2048 371 / 313, 3000x3001x3008 100 / 91, 53 x (456x1961x256) 88 / 86 -- and loses where every row of a K-contiguous operand
+        // starts unaligned: 4100^3 237 / 259, 1234x5678x4321 116 / 132.  With a K of 512 to 768 it is level or behind by now, which the
+        // costs below do not say: 1024x50257x768 134 / 151, 8000x3001x512 46 / 49)
         if (v.any && v.bm == 256) {
             const int vec_k = 16 / elem_size(pb.g.in_type);
             if ((v.a_kc && pb.g.a_rs % vec_k) || (v.b_kc && pb.g.b_cs % vec_k)) continue;
@@ -403,8 +421,7 @@ int auto_mfma_variant(const Problem& pb, int only_tile = 0, bool short_rows = fa
         // (measured, 64x64 against 128x128 tiles: fp32, bound by its slow MFMAs, 1024^3 20.7 against 63.7 us and 3072x1024x1024
         // 53 against 66; 8- and 16-bit inputs win while a CU has at most two of them -- fp16 1024^3 6.6 against 9.5 us,
         // 1536x1152x2048 14.4 against 17.0 -- and lose beyond: 3072x1024x1024 13.1 against 9.8, 2048^3 30.3 against 21.2)
-        if (staged_short_k && v.bm * v.bn <= 64 * 64) cost /= 1.8; // (the 2.0 of the unaligned chunks above hardly shows)
-        else if (v.bm * v.bn <= 64 * 64) cost /= pb.g.in_type == T_F32 ? 1.0 : per_cu <= 2 ? 0.75 : 0.5;
+        if (v.bm * v.bn <= 64 * 64) cost /= pb.g.in_type == T_F32 ? 1.0 : per_cu <= 2 ? 0.75 : 0.5;
         else if (v.bm * v.bn <= 128 * 64) cost /= 0.8;
         // rank inside one tile shape: ping-pong kb64 x4 > ping-pong others > 8-wave > 4-wave (kb64 x4 first)
         int rank = v.pingpong ? (v.kb == 64 && v.stages == 4 ? 8 : 6) : (v.waves_m * v.waves_n == 8 ? 4 : 2);

@@ -257,6 +257,19 @@ def test_slices_against_a_k_contiguous_b():
         assert "fill=direct" in _lib.variant_name(v) and ks == slices, (M, N, K, ks)
 
 
+def test_tiles_of_register_staged_problems_with_a_short_k():
+    """64 x 64 or 128 x 128 tiles by a model of both (unaligned operands, K of 64 to 2048 bytes), what reads C among it."""
+    from accera_amd import tune
+    tile = lambda v: re.search(r"mfma (\d+x\d+)", _lib.variant_name(v)).group(1)
+    F16, BF16, F32, I8, I32 = _lib.F16, _lib.BF16, _lib.F32, _lib.I8, _lib.I32
+    for (t, o, M, N, K, ta, beta), want in [
+            ((F16, F16, 704, 3136, 52, False, 0.0), "64x64"), ((F16, F16, 4936, 643, 112, False, 0.0), "64x64"),
+            ((F16, F32, 5184, 3972, 73, False, 0.0), "128x128"), ((BF16, BF16, 793, 5760, 547, True, 0.0), "128x128"),
+            ((F16, F16, 824, 4072, 888, False, 0.0), "128x128"), ((F16, F32, 600, 901, 100, False, 1.0), "64x64")]:
+        v, ks = tune.own_choice(t, o, M, N, K, ta, False, 1.0, beta)
+        assert "edge" in _lib.variant_name(v) and tile(v) == want and ks == 1, (M, N, K, _lib.variant_name(v), ks)
+
+
 def test_bound_call_handles_without_launching():
     """acc950_bind validates and chooses once; handles are reused after acc950_unbind; unknown handles
     are reported.  (No launch here: there is no GPU on the CPU test tier.)"""
