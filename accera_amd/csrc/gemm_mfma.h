@@ -535,8 +535,8 @@ bool fills_checked(const GemmArgs& a)
     constexpr int ES = InTraits<Cfg::IN>::ES, VEC = 16 / ES, BK = Cfg::KB / ES;
     const int k_least = a.k_last > 0 && a.k_last < a.K ? a.k_last : a.K;
     if ((Cfg::A_KC ? k_least : a.M) < VEC || (Cfg::B_KC ? k_least : a.N) < VEC) return true;
-    const int ext_a = Cfg::A_KC ? a.K : a.M, ext_b = Cfg::B_KC ? a.K : a.N;
-    return (a.K + BK - 1) / BK <= staged_ring<typename Cfg::Checked>() && ext_a % VEC == 0 && ext_b % VEC == 0;
+    const bool whole_k = a.K % VEC == 0 && (a.k_last <= 0 || a.k_last % VEC == 0);
+    return (a.K + BK - 1) / BK <= staged_ring<typename Cfg::Checked>() && (Cfg::A_KC ? whole_k : a.M % VEC == 0) && (Cfg::B_KC ? whole_k : a.N % VEC == 0);
 }
 
 template <typename Cfg>
