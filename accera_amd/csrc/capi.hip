@@ -755,8 +755,8 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
             // column-major A 4.8 against 10.6 -- and on 6 of the 74 with a longer K, where the tiled kernels split K:
             // 64x192x1728 9.9 us in 16 slices against 18.5); with more blocks the tiled kernels with direct fills win
             // (768x576x1024: 17.1 in four slices against 26.3; 2048x192x1280: 17.3 against 27.4).  Against the
-            // register-staged tiled kernels (unaligned operands) the kernel of blocks also wins with two rounds and a K up to 768, and
-            // with a longer one while the tiles x K slices leave half of the chip idle.
+            // register-staged tiled kernels (unaligned operands) the kernel of blocks also wins with up to two rounds and a K up to 768
+            // (see below), and with a longer one while the tiles x K slices leave half of the chip idle.
             int slices = 1;
             if (mv >= 0) {
                 int n = 0;
@@ -767,10 +767,19 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
                 // (or more workgroups than there are 32 x 32 blocks: a small output with a long K, which only the tiled kernels split)
                 const int64_t blocks = (((int64_t)pb.g.M + 31) / 32) * (((int64_t)pb.g.N + 31) / 32);
                 const bool one_round = blocks <= kComputeUnits && pb.g.K <= 640;
-                // (with more blocks than two rounds the register-staged kernels are ahead however short K is: 4864x2752x648 170 us
-                // against 315, 4148x1439x128 26.6 / 44.4, 1472x674x576 18.5 / 28.2, 5037x376x32 8.0 / 11.9;
-                // 520x792x448, 425 blocks, 13.4 / 12.1)
-                if (one_round || (!v.direct && ((pb.g.K <= 768 && blocks <= 2 * kComputeUnits) || (tiles * slices * 2 < kComputeUnits && tiles * slices <= blocks)))) mv = -1;
+                // Against the register-staged kernels, K up to 768: with more blocks than two rounds (those of a whole batch) the 64 x 64
+                // ones are ahead however short K is, while their tiles are not mostly empty (us, blocks / tiles: 4864x2752x648 315 / 181,
+                // 4148x1439x128 30.3 / 21.3, 1472x674x576 26.3 / 17.2, 5037x376x33 11.8 / 6.8, 160 x (888x329x80) 221 / 136, 104 x (80x192x301) 41.2 / 25.2;
+                // 520x792x448, 425 blocks, 13.4 / 12.1; 64 x (100x30x700), 256 blocks, 11.9 / 20.3).  They sum K in four chains, as the blocks do; never the
+                // 128 x 128 ones, which have one.
+                const bool staged_short = !v.direct && pb.g.K <= 768;
+                const int64_t all_blocks = blocks * (pb.g.batch > 1 ? pb.g.batch : 1);
+                const int64_t small = (((int64_t)pb.g.M + 63) / 64) * (((int64_t)pb.g.N + 63) / 64);
+                if (staged_short && k_splits <= 1 && all_blocks > 2 * kComputeUnits && 8 * small <= 3 * blocks) {
+                    mv = auto_mfma_variant(pb, 64);
+                    if (mv >= 0 && mfma_table(pb.g.in_type, &n)[mv].direct) mv = -1;
+                }
+                else if (one_round || staged_short || (!v.direct && tiles * slices * 2 < kComputeUnits && tiles * slices <= blocks)) mv = -1;
             }
             if (mv < 0) { c->variant = ACC950_VARIANT_F32_MFMA; return ACC950_OK; }
         }

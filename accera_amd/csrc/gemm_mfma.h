@@ -453,11 +453,17 @@ struct MfmaConfig {
     // end, and writes them to GemmArgs::stamps (phase times and the clock the engine ran at).
     static constexpr bool TIMED = TIMED_;
     // workgroups meant to share a CU: as many as the LDS allows, at most 2 waves per SIMD in all
-    // (four of the 64 x 64 edge kernels, which is 128 registers each: asked for two, the compiler took up to 164)
-    static constexpr int WGS_PER_CU = EDGE_ && BM_ * BN_ <= 64 * 64 ? 4 : (WAVES_M_ * WAVES_N_ <= 4 && 2 * STAGES_ * (BM_ + BN_) * KB_ <= 160 * 1024 && BM_ * BN_ <= 256 * 128) ? 2 : 1;
+    // (four of the 64 x 64 edge kernels, which is 128 registers each: asked for two, the compiler took up to 164; fp32 has two or three, see FOUR_SUMS)
+    static constexpr int WGS_PER_CU = EDGE_ && BM_ * BN_ <= 64 * 64 ? (IN_ == IN_F32 ? 2 : 4) : (WAVES_M_ * WAVES_N_ <= 4 && 2 * STAGES_ * (BM_ + BN_) * KB_ <= 160 * 1024 && BM_ * BN_ <= 256 * 128) ? 2 : 1;
     static constexpr int IN = IN_, BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, KB = KB_, STAGES = STAGES_;
     static constexpr bool A_KC = A_KC_, B_KC = B_KC_, DIRECT = DIRECT_, EDGE = EDGE_;
     static constexpr int NT = WAVES_M * WAVES_N * 64;
+    // FOUR_SUMS (fp32, 64 x 64 edge tiles): each of the four steps of a K tile has sums of its own, added up at the end.  These tiles
+    // take problems from the kernel of 32 x 32 blocks, whose four waves sum a quarter of K each: with one chain over all of K their
+    // error against float64 was twice that kernel's (1472x674x576 4.3e-7 of the 2-norm / 2.2e-7; 2.2e-7 with four).
+    // (Added to a total after every tile instead, K of less than 128 stayed worse, 5037x376x33 1.0e-7 / 6.8e-8; after every step the compiler
+    // spilled 500 bytes per lane.)
+    static constexpr bool FOUR_SUMS = IN_ == IN_F32 && EDGE_ && BM_ * BN_ <= 64 * 64;
     static constexpr int LDS_BYTES = STAGES * (BM + BN) * KB;
     static_assert(!(DIRECT && EDGE), "edge tiles are zero-filled through registers");
     static_assert(DIRECT || STAGES == 2, "the register-staged fill is double-buffered");
@@ -669,6 +675,8 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
 #pragma unroll
         for (int j = 0; j < TN; ++j) bf[0][j] = TB::read_frag(sb, wc0 + j * 32, 0, lane);
     };
+    [[maybe_unused]] acc_t step_sums[Cfg::FOUR_SUMS ? KSTEPS : 1] = {};
+    static_assert(!Cfg::FOUR_SUMS || (TM == 1 && TN == 1), "one 32x32 block per wave");
     auto mma_tile = [&](const char* sa, const char* sb, const char* next_sa, const char* next_sb, auto fill_tag,
                         auto cross_tag, int fill_stage, int fill_k0) {
         constexpr bool fill = decltype(fill_tag)::value;
@@ -684,7 +692,8 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     const int slot = i * TN + j;
-                    mfma32<IN>(af[ks & 1][i], bf[ks & 1][j], acc[i][j]);
+                    if constexpr (Cfg::FOUR_SUMS) mfma32<IN>(af[ks & 1][i], bf[ks & 1][j], step_sums[ks]);
+                    else mfma32<IN>(af[ks & 1][i], bf[ks & 1][j], acc[i][j]);
                     if (!last || cross) {
                         // B fragments first: the first MFMAs of the next step need bf[0] and af[0]
 #pragma unroll
@@ -913,6 +922,7 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
         // them by then, and waits for memory in front of every store of the write-back (190 waits in the int8 128 x 128 kernel, each
         // of which also waits for the stores before: 190 x (320x960x32) 84.5 us, 61.4 without).
         __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
+        if constexpr (Cfg::FOUR_SUMS) acc[0][0] = (step_sums[0] + step_sums[1]) + (step_sums[2] + step_sums[3]);
     }
 
     stamp(2);

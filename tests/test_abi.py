@@ -270,6 +270,33 @@ def test_tiles_of_register_staged_problems_with_a_short_k():
         assert "edge" in _lib.variant_name(v) and tile(v) == want and ks == 1, (M, N, K, _lib.variant_name(v), ks)
 
 
+def test_fp32_problems_with_unaligned_operands_and_a_short_k():
+    """More 32 x 32 blocks than two rounds: the 64 x 64 tiles, whose sums are four chains as well, never the 128 x 128 ones; fewer, or
+    tiles that would be mostly empty: the kernel of blocks."""
+    from accera_amd import tune
+    own = lambda *a: _lib.variant_name(tune.own_choice(_lib.F32, _lib.F32, *a, 1.0, 0.0)[0])
+    for a in [(4864, 2754, 648, False, False), (4148, 1439, 128, False, False), (1472, 674, 576, False, False), (5037, 376, 33, False, True), (700, 901, 766, True, True)]:
+        assert "mfma 64x64" in own(*a) and "edge" in own(*a), (a, own(*a))
+    for a in [(520, 793, 448, False, False), (512, 1024, 33, False, True), (20000, 24, 100, False, False), (300, 301, 301, False, False)]:
+        assert "fp32 mfma 32x32" in own(*a), (a, own(*a))
+    # a batch counts with all its blocks (grid: 64 x 64 tiles of one problem, or its 32 x 32 blocks)
+    geom = lambda batch: _batched_geometry(batch, 80, 192, 301)
+    assert geom(104) == (6, 104) and geom(8)[1] == 8 and geom(8)[0] != 6
+
+
+def _batched_geometry(batch, M, N, K):
+    L, h, v, ks, P = _lib.lib(), ctypes.c_int(-1), ctypes.c_int(), ctypes.c_int(), ctypes.c_void_p
+    _lib.check(L.acc950_bind(_lib.F32, _lib.F32, batch, M, N, K, P(1 << 32), M * K, K, 1, P(2 << 32), K * N, N, 1, P(3 << 32), M * N, N, 1,
+                             _lib.PROLOGUE_SET0, 0.0, _lib.EPILOGUE_NONE, 0.0, _lib.VARIANT_AUTO, 0, None, ctypes.byref(h)))
+    try:
+        _lib.check(L.acc950_bound_choice(h.value, ctypes.byref(v), ctypes.byref(ks)))
+    finally:
+        L.acc950_unbind(h.value)
+    if v.value == _lib.VARIANT_F32_MFMA:
+        return (-1, batch)
+    return _lib.launch_geometry(_lib.F32, _lib.F32, M, N, K, (K, 1), (N, 1), (N, 1), v.value)[0][0], batch
+
+
 def test_bound_call_handles_without_launching():
     """acc950_bind validates and chooses once; handles are reused after acc950_unbind; unknown handles
     are reported.  (No launch here: there is no GPU on the CPU test tier.)"""

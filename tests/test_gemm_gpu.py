@@ -1514,3 +1514,37 @@ def test_k_split_of_outputs_whose_rows_are_not_whole_vectors(in_type, out_type, 
                 want = A.astype(np.float64) @ B.astype(np.float64) + 2.0 * C0.astype(np.float64)
                 # (fp16's last rounding, 2^-11 of the value, and 32-bit sums of 1160 products of at most 1)
                 np.testing.assert_allclose(to_host(dC, out_type).astype(np.float64), want, rtol=2.0 ** -10, atol=1e-3)
+
+
+@pytest.mark.parametrize("M,N,K,batch", [(1472, 674, 576, 1), (5037, 376, 33, 1), (4148, 1439, 129, 1), (80, 192, 301, 104), (700, 901, 766, 1)])
+def test_fp32_tiles_are_as_close_to_float64_as_the_kernel_of_blocks(M, N, K, batch):
+    """The problems the 64 x 64 edge tiles take from the kernel of 32 x 32 blocks: their four chains of sums are as long as that
+    kernel's four waves' (one chain over all of K was twice as far off).  Every order of four such chains has the same expected
+    error; over 10^5 results and more the two measured ones differ by under 2 %."""
+    import accera_amd as acc
+    import torch
+    from accera_amd import _lib
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    lead = (batch,) if batch > 1 else ()
+    A = torch.empty(lead + (M, K), device="cuda").normal_(generator=g)
+    B = torch.empty(lead + (K, N), device="cuda").normal_(generator=g)
+    out = []
+    for variant in (_lib.VARIANT_AUTO, _lib.VARIANT_F32_MFMA):
+        C = torch.empty(lead + (M, N), device="cuda")
+        f = acc.GemmCall(A, B, C, epilogue=acc.EPILOGUE_NONE, variant=variant)
+        f()
+        assert ("mfma 64x64" in _lib.variant_name(f.chosen[0])) == (variant == _lib.VARIANT_AUTO), _lib.variant_name(f.chosen[0])
+        out.append(C.cpu().double().numpy())
+    want = np.matmul(A.cpu().double().numpy(), B.cpu().double().numpy())
+    tiles, blocks = (np.linalg.norm(x - want) / np.linalg.norm(want) for x in out)
+    assert tiles <= 1.03 * blocks and tiles < 4e-7, (tiles, blocks)
+
+
+@pytest.mark.parametrize("in_type", ["f16", "i8", "f32"])
+@pytest.mark.parametrize("K,splits", [(1532, 8), (1163, 3), (775, 2)])
+def test_k_split_whose_last_slice_ends_inside_a_chunk(in_type, K, splits):
+    """Any-alignment 64 x 64 tiles, K-contiguous operands: full slices of one to nine K tiles, a last one that is no whole chunk."""
+    out_type = {"f16": "f32", "i8": "i32", "f32": "f32"}[in_type]
+    v = next(v for v, n in _variants("col") if "mfma 64x64" in n and "any-alignment" in n and "A=col-major" not in n)
+    run_case(in_type, out_type, 67, 50, K, b_layout="col", variant=v, splits=splits, seed=K, dist="normal", prologue=ora.PRO_NONE)
