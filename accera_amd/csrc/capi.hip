@@ -216,6 +216,8 @@ int auto_skinny_variant(const Problem& pb)
 // ---- workspace of the skinny kernels' K split ------------------------------------------
 // Partial sums (fp32) and one arrival counter per column block.  One workspace per (device, stream): launches on one
 // stream run one after the other and may share it, launches on different streams may overlap and must not.  A
+// workspace that is missing or too small while its stream is being captured is not made (an allocation would end the
+// capture): the call runs unsplit then, as calls of the same shape did that had needed none.  A
 // workspace only grows, and an outgrown block stays allocated, because launches queued earlier may still be using
 // it, until acc950_release_workspaces frees everything on an idle device.  The pointers are copied out while the
 // lock is held.
@@ -237,6 +239,12 @@ hipError_t workspace_for(hipStream_t stream, size_t floats, size_t counters, flo
     if (e != hipSuccess) return e;
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     Workspace& w = g_ws[std::make_pair(dev, stream)];
+    if (floats > w.floats || counters > w.n_counters) {
+        // (no allocation while the stream is being captured: it would end the capture)
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
+        if (status == hipStreamCaptureStatusActive) return hipErrorStreamCaptureUnsupported;
+    }
     if (floats > w.floats) {
         const size_t want = floats < (1u << 20) ? (1u << 20) : floats + floats / 2;
         float* p = nullptr;
@@ -882,7 +890,10 @@ int run(const Problem& pb, const Choice& c, hipStream_t stream, LaunchGeom* geom
                 s.counters = (unsigned*)(base + kStaticFloats);
             } else {
                 e = workspace_for(stream, floats, counters, &s.scratch, &s.counters);
-                if (e != hipSuccess) return fail_hip(e, "workspace allocation");
+                if (e == hipErrorStreamCaptureUnsupported) { // (under capture, and no workspace yet: unsplit, no shared blocks)
+                    s.splits = 1;
+                    s.extra_phase = -1;
+                } else if (e != hipSuccess) return fail_hip(e, "workspace allocation");
             }
         }
         e = launch_skinny(sv, s, stream, geom, dry_run);
@@ -894,9 +905,9 @@ int run(const Problem& pb, const Choice& c, hipStream_t stream, LaunchGeom* geom
         const bool lean = g.prologue == PRO_SET && g.prologue_arg == 0.f && (g.epilogue == EPI_RELU || g.epilogue == EPI_NONE);
         SplitPlan sp;
         // (the choice was made for the workspace of this call: the same plan comes out again)
-        const bool split = c.splits > 1 && plan_split(mv, pb, c.splits, &sp, static_ws ? kStaticFloats : kMaxSplitFloats);
+        bool split = c.splits > 1 && plan_split(mv, pb, c.splits, &sp, static_ws ? kStaticFloats : kMaxSplitFloats);
+        float* ws = nullptr;
         if (split) {
-            float* ws = nullptr;
             if (!dry_run) {
                 const size_t floats = (size_t)sp.splits * (size_t)g.M * (size_t)g.N + 3; // (the reduction reads whole pieces of four; the built-in array has its counters behind)
                 unsigned* unused = nullptr;
@@ -905,9 +916,12 @@ int run(const Problem& pb, const Choice& c, hipStream_t stream, LaunchGeom* geom
                     if (e != hipSuccess) return fail_hip(e, "address of the built-in workspace");
                 } else {
                     e = workspace_for(stream, floats, 0, &ws, &unused);
-                    if (e != hipSuccess) return fail_hip(e, "workspace allocation");
+                    if (e == hipErrorStreamCaptureUnsupported) split = false; // (under capture, and no workspace yet: unsplit)
+                    else if (e != hipSuccess) return fail_hip(e, "workspace allocation");
                 }
             }
+        }
+        if (split) {
             e = mv.launch(split_first_step(g, sp, ws), stream, geom, dry_run); // partial products: C = A*B, nothing else
             if (e == hipSuccess && !dry_run) e = launch_splitk_reduce(g, ws, sp.splits, stream);
         } else {

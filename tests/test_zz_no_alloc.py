@@ -135,3 +135,40 @@ def test_static_workspace_entry_point_under_graph_capture():
         if replay == 1:                                  # the same entry point eagerly, between replays: the array is shared
             step(L.acc950_gemm_ops_static, hid_e, out_e, sq_e, torch.cuda.current_stream().cuda_stream)
             torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("M,N,K", [(99, 5312, 7168), (32, 9600, 4096), (8, 2048, 4096), (8, 11008, 4096)])
+def test_a_captured_call_without_a_workspace_runs_unsplit(M, N, K):
+    """The allocating entry points on a stream that is being captured and has no workspace yet: problems that are split over K
+    (or share column blocks) elsewhere run unsplit -- nothing is allocated, nothing refused -- and every replay gives the same
+    result; once the stream has its workspace a capture uses it."""
+    import accera_amd as acc
+    import torch
+    from accera_amd import _lib
+    _lib.check(_lib.lib().acc950_init(0))
+    rng = np.random.default_rng(M)
+    A, B = make_input(rng, (M, K), "f16", "normal"), (make_input(rng, (K, N), "f16", "normal").astype(np.float32) * 0.03).astype(np.float16)
+    dA, dB, dC = to_device(A, "f16"), to_device(B, "f16"), to_device(np.zeros((M, N), np.float16), "f16")
+    want = ora.gemm_relu_exact(A, B, out_zeros(M, N, "f16"), "f16", "f16", ora.PRO_SET0, ora.EPI_RELU)
+    acc.gemm_relu(dA, dB, dC)  # (eager, on another stream: loads the kernels' code)
+    torch.cuda.synchronize()
+    assert_matches(to_host(dC, "f16"), want, "f16", K)
+    for warm in (False, True):
+        side = torch.cuda.Stream()
+        _lib.check(_lib.lib().acc950_release_workspaces())
+        if warm:
+            acc.gemm_relu(dA, dB, dC, stream=side.cuda_stream)
+            torch.cuda.synchronize()
+        before = _lib.allocation_probe()
+        graph = torch.cuda.CUDAGraph()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            with torch.cuda.graph(graph, stream=side):
+                acc.gemm_relu(dA, dB, dC, stream=side.cuda_stream)
+        assert _lib.allocation_probe() == before
+        for replay in range(3):
+            dC.fill_(3)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_matches(to_host(dC, "f16"), want, "f16", K)
