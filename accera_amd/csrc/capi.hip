@@ -576,7 +576,9 @@ int streamed_b_tile(const Problem& pb)
     // (65 to 256 rows against 32 to 192 MB, 16-bit types: 128 x 128 tiles in slices, whatever of the cache holds B -- fp16
     // 99x5312x14656 39.5 us in six slices, 86.9 on 64 x 64 tiles; bf16 80x2176x27648 32.1 / 50.8, 115x6464x4608 22.3 / 29.5,
     // 185x3520x4800 with a K-contiguous B 17.9 / 21.9, fp16 194x2496x21504 45.2 / 74.4, 224x4224x5568 28.4 / 34.0; while the
-    // chip takes three slices of every tile: 159x46976x1024, 734 tiles, is 32.1 us on the general rule's 256 x 256 ones, 44.9 this way)
+    // chip takes three slices of every tile: 159x46976x1024, 734 tiles, is 32.1 us on the general rule's 256 x 256 ones, 44.9 this way.
+    // Of 86 to 128 tiles it takes two, 100x11008x4096 43.1 us unsplit on 64 x 64 tiles, 28.7 so, 128x14336x4096 49.7 / 35.2, 100x16384x4096
+    // 47.9 / 43.4, and int8 gains as much, 128x4096x16384 41.0 / 27.6 in six slices, 115x6464x4608 18.5 / 15.7 in three: not in this rule yet)
     if (!streamed_b(pb, (int64_t)192 << 20))
         return pb.g.in_type != T_I8 && pb.g.M > 64 && streamed_b(pb, (int64_t)32 << 20) && (int64_t)((pb.g.M + 127) / 128) * ((pb.g.N + 127) / 128) * 3 <= kComputeUnits ? 128 : 0;
     // (a tile that holds all rows of A: up to 64 rows the small tiles, up to 128 rows the 128 x 128 tiles, up to 256 the
@@ -679,8 +681,9 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
         // which the streaming kernel's whole columns need not pay (us, streaming kernel / tiles, fp16, M rows: 32x64x262144 92 / 55
         // in 32 slices, 17x4096x4096 11.8 / 11.5 in four, 24x5056x8192 23.9 / 19.7 in six; two slices or none lose, 31x9600x1792
         // 8.9 / 9.7, 17x6400x2624 9.6 / 11.0, 24x9600x2048 9.3 / 11.7, and so do three short ones from 88 tiles on, 17x6080x3264 1.22
-        // times as long, 17x6400x3584 15.3 / 14.6; from 136 tiles on the streaming kernel has enough workgroups by itself while rows and K are
-        // few, 17x8960x5632 23.7 / 24.2, 24x8960x4096 20.0 / 19.8, 32x8960x4096 22.2 / 20.7, 17x9984x12288 level; rows of B a
+        // times as long, 17x6400x3584 15.3 / 14.6; from 136 tiles on, where the streaming kernel shares its slow blocks between two workgroups, it is ahead while rows
+        // and K are few, 17x8960x5632 23.7 / 24.2, 17x9984x8192 32.8 / 34.3, 32x8960x5632 28.9 / 26.0, and where it does not share them it is not: 17x9600x3584
+        // 17.8 / 17.0, 32x9600x3584 21.5 / 18.7; rows of B a
         // multiple of 16 KB apart cost the tiles a fifth, which fetch one line of 64 of them: 17x8128x3584 level, 17x8192x3584 15.9 / 18.9, 32x8192x8192 34.8 / 33.5).
         // 300 to 400 tiles, unsplit, fill the chip by themselves (17 and 32 rows, K = 1024 to 8192, N = 19264 to 25600: 0.65 to 0.87 of
         // the streaming kernel's time; 160 to 299 do not, 29x11712x7168 35.8 / 45.5, and more are a second round: 25x37056x6912 104.5 / 115.3),
@@ -695,7 +698,7 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
             const int tiles = (pb.g.N + 63) / 64;
             const int64_t k_rows = (int64_t)pb.g.K * pb.g.M;
             bool pays = tiles >= 300 && (tiles <= 376 ? pb.g.K <= 8192 : tiles <= 400 && pb.g.K < 8192);
-            if (tiles < 160) pays = pb.g.b_rs % 8192 == 0 ? k_rows >= 250000 : tiles < 88 || (pb.g.K >= 3584 && (tiles < 136 || k_rows >= 120000));
+            if (tiles < 160) pays = pb.g.b_rs % 8192 == 0 ? k_rows >= 250000 : tiles < 88 || (pb.g.K >= 3584 && (tiles < 136 || (pb.g.b_rs * 2) % 512 != 0 || k_rows >= 150000));
             if (pays && mv >= 0 && tab[mv].direct) {
                 const int slices = streamed_b_splits(tab[mv], pb, max_split_floats);
                 if (tiles >= 160 || slices >= 3) {

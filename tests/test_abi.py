@@ -214,7 +214,7 @@ def test_choices_of_the_cost_model():
     (31, 4416, 9792, "64x64", 7), (17, 4096, 4096, "64x64", 4), (32, 64, 262144, "64x64", 32), (24, 5056, 8192, "64x64", 6), (17, 6400, 3584, "64x64", 3),
     (31, 20800, 4544, "64x64", 1),          # (325 tiles: unsplit, they fill the chip)
     (31, 9600, 1792, None, 1), (24, 9600, 2048, None, 1), (17, 6400, 2624, None, 1),  # (two slices or none: the streaming kernel)
-    (17, 6080, 3264, None, None), (17, 8960, 5632, None, None), (32, 8960, 5632, "64x64", 3),
+    (17, 6080, 3264, None, None), (17, 8960, 5632, None, None), (32, 8960, 5632, "64x64", 3), (17, 9984, 8192, None, None), (17, 9600, 3584, "64x64", 3),
     (18, 8192, 2048, None, None), (17, 8192, 8192, None, None), (32, 8192, 8192, "64x64", 4),   # (rows of B 16 KB apart)
     (29, 11712, 7168, None, None), (25, 37056, 6912, None, None), (17, 24576, 8192, None, None),
     (22, 5056, 1408, None, None),           # (a B of less than 32 MB)
