@@ -1059,21 +1059,23 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
         }
     }
 
-    // ---- pass B (ReLU after a SET-0 prologue is the fused hot path: one max per element; every other
-    // combination shares one copy with wave-uniform selects)
-    if (p.epilogue == EPI_RELU && !(p.prologue == PRO_SET && p.prologue_arg != 0.f)) {
-        for_each_acc([&](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); });
-    } else if (p.epilogue != EPI_NONE || (p.prologue == PRO_SET && p.prologue_arg != 0.f)) {
-        const scalar_t set_value = p.prologue == PRO_SET ? (scalar_t)p.prologue_arg : scalar_t(0);
+    // ---- pass B: a SET constant, then the epilogue op, each a loop of its own with the one or two instructions per element it needs.
+    // (As one loop with wave-uniform selects over all ops it was about twelve: 32 x (2048x2048x128) fp16 scaled by alpha 111 us on
+    // 128 x 128 tiles, 79 without an epilogue.)
+    if (p.prologue == PRO_SET && p.prologue_arg != 0.f) {
+        const scalar_t set_value = (scalar_t)p.prologue_arg;
+        for_each_acc([&](scalar_t v) { return wrap_add(v, set_value); });
+    }
+    if (p.epilogue == EPI_RELU) for_each_acc([&](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); });
+    else if (p.epilogue == EPI_SCALE) {
         const scalar_t epi_arg = (scalar_t)p.epilogue_arg;
-        const bool is_relu = p.epilogue == EPI_RELU, is_nocond = p.epilogue == EPI_RELU_NOCOND, is_scale = p.epilogue == EPI_SCALE,
-                   is_set = p.epilogue == EPI_SET;
+        for_each_acc([&](scalar_t v) { return wrap_mul(v, epi_arg); });
+    } else if (p.epilogue != EPI_NONE) {
+        const scalar_t epi_arg = (scalar_t)p.epilogue_arg;
+        const bool is_set = p.epilogue == EPI_SET; // (else ReLU_NoConditional)
         for_each_acc([&](scalar_t v) {
-            v = wrap_add(v, set_value);
-            const scalar_t r = v > scalar_t(0) ? v : scalar_t(0);
             const scalar_t n = v * (v > scalar_t(0) ? scalar_t(1) : scalar_t(0));
-            const scalar_t m = wrap_mul(v, epi_arg);
-            return is_relu ? r : (is_nocond ? n : (is_scale ? m : (is_set ? epi_arg : v)));
+            return is_set ? epi_arg : n;
         });
     }
     };
