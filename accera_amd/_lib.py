@@ -19,7 +19,7 @@ F32, F16, BF16, I8, I32, I16 = 0, 1, 2, 3, 4, 5
 PROLOGUE_NONE, PROLOGUE_SET0, PROLOGUE_SET, PROLOGUE_SCALE = 0, 1, 1, 2
 EPILOGUE_NONE, EPILOGUE_RELU, EPILOGUE_RELU_NOCOND, EPILOGUE_SCALE, EPILOGUE_SET = 0, 1, 2, 3, 4
 OK, INVALID_ARGUMENT, UNSUPPORTED, HIP_ERROR = 0, 1, 2, 3
-VARIANT_AUTO, VARIANT_SKINNY_BASE, VARIANT_GENERIC, VARIANT_F32_MFMA = -1, 100, 200, 201
+VARIANT_AUTO, VARIANT_SKINNY_BASE, VARIANT_GENERIC, VARIANT_F32_MFMA, VARIANT_SHORT_K = -1, 100, 200, 201, 202
 
 EXPORTS = [
     "acc950_init", "acc950_gemm_relu", "acc950_gemm_relu_ex", "acc950_gemm_relu_host", "acc950_gemm_ops", "acc950_gemm_ops_host", "acc950_gemm_ops_static",

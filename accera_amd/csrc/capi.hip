@@ -184,6 +184,27 @@ bool mfma_can_take(const MfmaVariant& v, const Problem& pb)
     return true;
 }
 
+// The short-K kernel (gemm_short_k.h): K in one to four whole k-steps of 64 bytes; C only written, in 16-byte pieces of aligned rows,
+// with no op or one of the usual ones behind it.
+bool short_k_can_take(const Problem& pb)
+{
+    const GemmArgs& g = pb.g;
+    if ((g.in_type != T_F16 && g.in_type != T_BF16 && g.in_type != T_I8) || g.M <= 0 || g.N <= 0 || g.K <= 0 || g.K > 256) return false;
+    if (g.prologue != PRO_SET || (g.epilogue != EPI_NONE && g.epilogue != EPI_RELU && g.epilogue != EPI_SCALE)) return false;
+    const int es = elem_size(g.in_type), os = elem_size(g.out_type), vec = 16 / es, k_bytes = g.K * es;
+    if (k_bytes > 256 || k_bytes % 64) return false;
+    if (g.c_cs != 1 || (g.a_cs != 1 && g.a_rs != 1) || (g.b_rs != 1 && g.b_cs != 1)) return false;
+    const bool a_kc = g.a_cs == 1, b_kc = g.b_rs == 1; // (as its launcher tells them apart)
+    const int64_t lda = a_kc ? g.a_rs : g.a_cs, ldb = b_kc ? g.b_cs : g.b_rs;
+    if (lda % vec || ldb % vec || (!a_kc && g.M % vec) || (!b_kc && g.N % vec)) return false;
+    if ((g.c_rs * os) % 16 || (g.N * os) % 16) return false;
+    if (g.batch > 1 && (g.a_bs % vec || g.b_bs % vec || (g.c_bs * os) % 16)) return false;
+    if (pb.have_pointers && (!aligned16(g.A) || !aligned16(g.B) || !aligned16(g.C))) return false;
+    // 32-bit offsets inside a tile: 64 rows of C, 64 / 256 rows of A / B or one staged sub-tile of K of them
+    const int bk = 128 / es;
+    return 64 * g.c_rs * os < (1ll << 31) && (a_kc ? 64 : bk) * lda * es < (1ll << 31) && (b_kc ? 256 : bk) * ldb * es < (1ll << 31);
+}
+
 bool skinny_can_take(const Problem& pb, int sv)
 {
     const GemmArgs& g = pb.g;
@@ -614,6 +635,23 @@ int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats
     return plan_split(v, pb, (int)want, &sp, max_floats) ? sp.splits : 1;
 }
 
+// K of one to four whole k-steps and many tiles of C: the short-K kernel (gemm_short_k.h), if it pays.  Against the other
+// kernels' choice on 220 problems of K = 64 to 256 bytes, 1 to 600 MB of C, every type, layout and ops of this range (geometric mean of the
+// time it saves): more than two of its 64 x 256 tiles per CU and these mostly full 1.8 (us, fp16 32 x (2048x2048x128) scaled 85 / 57, 8192x8192x64
+// 39 / 29, bf16 6352x2952x96 with an fp32 result 54 / 28, int8 47 x (128x4816x128) 105 / 29); with rows of C that end inside a line from one per CU on 1.4,
+// where the others store parts of lines; fewer tiles, a workgroup has nothing to walk along: 0.9 (5136x384x64 3.0 / 4.4), and so where tiles stick
+// out by half (195 x (4608x128x32) 58 / 84).
+bool short_k_pays(const Problem& pb)
+{
+    const GemmArgs& g = pb.g;
+    if (!short_k_can_take(pb)) return false;
+    // (int8, all four k-steps, a row-major B: the four-wave kernel is level -- 8192x6144x256 43.2 us, 42.6 here; 8192x8192x256 60.8 / 63.5 -- and keeps them)
+    if (g.in_type == T_I8 && g.K == 256 && g.a_cs == 1 && g.b_cs == 1 && g.batch <= 1 && g.M >= 256 && g.N >= 256) return false;
+    const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 255) / 256), batch = g.batch > 1 ? g.batch : 1;
+    const bool part_lines = (g.c_rs * elem_size(g.out_type)) % 128 != 0;
+    return (double)g.M * g.N >= 0.6 * 64 * 256 * (double)tiles && tiles * batch > (part_lines ? 1 : 2) * kComputeUnits;
+}
+
 struct Choice {
     int variant;
     int splits;
@@ -675,6 +713,7 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
 {
     c->splits = 1;
     if (variant == ACC950_VARIANT_AUTO) {
+        if (k_splits <= 1 && short_k_pays(pb)) { c->variant = ACC950_VARIANT_SHORT_K; return ACC950_OK; }
         const int sv = auto_skinny_variant(pb);
         // 17 to 32 rows against a B of 32 MB and more, 16-bit types: the streaming kernel fetches half as many bytes of A as of B
         // by then; 64 x 64 tiles with direct fills are ahead where their slices stay long beside what the sums of the slices cost,
@@ -817,6 +856,14 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
         c->variant = variant;
         return ACC950_OK;
     }
+    if (variant == ACC950_VARIANT_SHORT_K) {
+        if (!short_k_can_take(pb))
+            return fail(ACC950_UNSUPPORTED, "the short-K kernel needs 8- or 16-bit inputs, K of one to four times 64 bytes, a C that is only written, with no epilogue, a ReLU or a "
+                                            "scale, and 16-byte aligned rows of A, B and C in whole 16-byte pieces");
+        if (k_splits > 1) return fail(ACC950_UNSUPPORTED, "the short-K kernel does not split K");
+        c->variant = variant;
+        return ACC950_OK;
+    }
     if (variant >= ACC950_VARIANT_SKINNY_BASE && variant < ACC950_VARIANT_SKINNY_BASE + skinny_num_variants()) {
         const int sv = variant - ACC950_VARIANT_SKINNY_BASE;
         if (!skinny_can_take(pb, sv))
@@ -855,6 +902,8 @@ int run(const Problem& pb, const Choice& c, hipStream_t stream, LaunchGeom* geom
         e = launch_generic(g, stream, geom, dry_run);
     } else if (c.variant == ACC950_VARIANT_F32_MFMA) {
         e = launch_f32(g, stream, geom, dry_run);
+    } else if (c.variant == ACC950_VARIANT_SHORT_K) {
+        e = launch_short_k(g, stream, geom, dry_run);
     } else if (c.variant >= ACC950_VARIANT_SKINNY_BASE) {
         const int sv = c.variant - ACC950_VARIANT_SKINNY_BASE;
         SkinnyArgs s{};
@@ -1222,6 +1271,10 @@ int acc950_variant_name(int variant, char* buf, size_t buf_len)
     }
     if (variant == ACC950_VARIANT_F32_MFMA) {
         std::snprintf(buf, buf_len, "fp32 mfma 32x32 tile, K split over 4 waves");
+        return ACC950_OK;
+    }
+    if (variant == ACC950_VARIANT_SHORT_K) {
+        std::snprintf(buf, buf_len, "mfma 64x256 short K, A in registers, walking column tiles");
         return ACC950_OK;
     }
     if (variant >= ACC950_VARIANT_SKINNY_BASE && variant < ACC950_VARIANT_SKINNY_BASE + skinny_num_variants()) {

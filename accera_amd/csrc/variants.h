@@ -31,6 +31,8 @@ hipError_t launch_splitk_reduce(const GemmArgs& g, const void* ws, int splits, h
 
 bool f32_can_take(const GemmArgs& g);
 hipError_t launch_f32(const GemmArgs& a, hipStream_t stream, LaunchGeom* geom, bool dry_run);
+// a short K and a large C (gemm_short_k.h); the caller has checked sizes, types and alignments (short_k_can_take)
+hipError_t launch_short_k(const GemmArgs& a, hipStream_t stream, LaunchGeom* geom, bool dry_run);
 hipError_t launch_generic(const GemmArgs& a, hipStream_t stream, LaunchGeom* geom, bool dry_run);
 
 } // namespace acc950

@@ -61,7 +61,7 @@ def candidates(in_id, out_id, M, N, K, sa, sb, sc, splits_for_skinny=(0, 2, 4, 8
     small beside B): elsewhere the partial sums cost more than the idle compute units."""
     L = _lib.lib()
     ids = list(range(_lib.num_variants())) + [_lib.VARIANT_SKINNY_BASE + i for i in range(_lib.num_skinny_variants())]
-    ids += [_lib.VARIANT_F32_MFMA, _lib.VARIANT_GENERIC]
+    ids += [_lib.VARIANT_F32_MFMA, _lib.VARIANT_SHORT_K, _lib.VARIANT_GENERIC]
     out = []
     for v in ids:
         if _lib.VARIANT_SKINNY_BASE <= v < _lib.VARIANT_GENERIC:

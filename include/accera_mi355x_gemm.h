@@ -60,6 +60,7 @@ extern "C" {
 #define ACC950_VARIANT_SKINNY_BASE 100 /* 100 + i : streaming kernel i for M <= 8 */
 #define ACC950_VARIANT_GENERIC 200     /* thread-bound kernel, any shape / stride / type */
 #define ACC950_VARIANT_F32_MFMA 201    /* fp32 MFMA kernel (fp32 inputs) */
+#define ACC950_VARIANT_SHORT_K 202     /* K of 64 to 256 bytes, C only written: A's rows in registers, walking along column tiles */
 
 /*
  * Selects the device and checks that it is a gfx950 part.  Optional: the other entry
@@ -91,7 +92,7 @@ int acc950_gemm_relu(int in_type, int out_type, int M, int N, int K,
  * point of the reference's tuning space (tile sizes, cache strategy, double buffering:
  * /root/reference/tools/benchmarkers/accera_gemm.py:187-348).  `variant` is
  * ACC950_VARIANT_AUTO, an index < acc950_num_variants() into the MFMA table,
- * ACC950_VARIANT_SKINNY_BASE + i, ACC950_VARIANT_F32_MFMA or ACC950_VARIANT_GENERIC.  `k_splits` splits K
+ * ACC950_VARIANT_SKINNY_BASE + i, ACC950_VARIANT_F32_MFMA, ACC950_VARIANT_SHORT_K or ACC950_VARIANT_GENERIC.  `k_splits` splits K
  * over workgroups (skinny and MFMA kernels; 0 = the library decides -- for a named MFMA variant: no split --,
  * 1 = no split, n > 1 = at most n slices).  The slices are added in a fixed order, so a split result does not
  * vary from run to run; an MFMA kernel's split goes through a workspace of 4 * slices * M * N bytes (held per

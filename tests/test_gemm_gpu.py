@@ -1548,3 +1548,68 @@ def test_k_split_whose_last_slice_ends_inside_a_chunk(in_type, K, splits):
     out_type = {"f16": "f32", "i8": "i32", "f32": "f32"}[in_type]
     v = next(v for v, n in _variants("col") if "mfma 64x64" in n and "any-alignment" in n and "A=col-major" not in n)
     run_case(in_type, out_type, 67, 50, K, b_layout="col", variant=v, splits=splits, seed=K, dist="normal", prologue=ora.PRO_NONE)
+
+
+@pytest.mark.parametrize("in_type,out_type", [("f16", "f16"), ("bf16", "bf16"), ("f16", "f32"), ("bf16", "f16"), ("i8", "i32"), ("i8", "i16"), ("i8", "i8")])
+@pytest.mark.parametrize("a_layout", ["row", "col"])
+@pytest.mark.parametrize("b_layout", ["row", "col"])
+def test_short_k_kernel(in_type, out_type, a_layout, b_layout):
+    """The kernel that keeps its rows of A and walks along column tiles: one to four k-steps of 64 bytes, tiles partly outside
+    C in both directions, rows of C that end inside a line, several tiles per workgroup, a batch, padded rows of C.  Integers bit for
+    bit, floats against the float64 product: half a unit in the last place of the output type (11 and 8 bits: 2^-11, 2^-8; fp32: K roundings of
+    2^-24 each) on sums of order one."""
+    import torch
+    import accera_amd as acc
+    from accera_amd import _lib
+    variant = _lib.VARIANT_SHORT_K
+    es = 1 if in_type == "i8" else 2
+    vec = 16 // es
+    for steps in (1, 2, 3, 4):
+        K = steps * 64 // es
+        for n, (batch, M, N, pad) in enumerate(((1, 16, 16, 0), (3, 80, 272, 0), (2, 64, 256, 64), (20, 48 + (0 if a_layout == "col" else 5), 2896, 0), (1, 176, 512 * 25 + 16, 16))):
+            epi, arg = ((ora.EPI_NONE, 0.0), (ora.EPI_RELU, 0.0), (ora.EPI_SCALE, 3.0))[(n + steps) % 3]
+            print(in_type, out_type, a_layout, b_layout, K, batch, M, N, pad, epi, flush=True)
+            assert (M % vec == 0 or a_layout == "row") and N % vec == 0
+            rng = np.random.default_rng(31 * steps + n)
+            A = np.stack([make_input(rng, (M, K), in_type, "normal") for _ in range(batch)])
+            B = np.stack([make_input(rng, (K, N), in_type, "normal") for _ in range(batch)])
+            dA = torch.stack([to_device(np.asfortranarray(a) if a_layout == "col" else a, in_type) for a in A]) if a_layout == "row" else \
+                torch.stack([to_device(np.ascontiguousarray(a.T), in_type) for a in A]).transpose(1, 2)
+            dB = torch.stack([to_device(b, in_type) for b in B]) if b_layout == "row" else \
+                torch.stack([to_device(np.ascontiguousarray(b.T), in_type) for b in B]).transpose(1, 2)
+            full = torch.stack([to_device(np.full((M, N + pad), 3, ora.NP_STORAGE[out_type]), out_type) for _ in range(batch)])
+            call = acc.GemmCall(dA, dB, full[:, :, :N], epilogue=epi, epilogue_arg=arg, variant=variant, k_splits=1)
+            assert call.chosen == (variant, 1)
+            call()
+            torch.cuda.synchronize()
+            wide = [ora.widen(x, in_type).astype(np.float64) for x in (A, B)]
+            want = wide[0] @ wide[1]
+            if epi == ora.EPI_RELU:
+                want = np.maximum(want, 0)
+            elif epi == ora.EPI_SCALE:
+                want = want * 3
+            for z in range(batch):
+                got = to_host(full[z], out_type)
+                assert (got[:, N:] == 3).all()
+                if in_type == "i8":
+                    assert (got[:, :N] == want[z].astype(np.int64).astype(ora.NP_STORAGE[out_type])).all()
+                else:
+                    eps = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8, "f32": 0}[out_type] * np.abs(want[z]) + K * 2.0 ** -24 * 3 * (np.abs(wide[0][z]) @ np.abs(wide[1][z])) + 2.0 ** -25
+                    assert (np.abs(ora.widen(got[:, :N], out_type).astype(np.float64) - want[z]) <= eps).all()
+
+
+def test_short_k_problems_run_on_the_short_k_kernel():
+    """The automatic choice on both sides of its lines, against the float64 product."""
+    import torch
+    import accera_amd as acc
+    from accera_amd import _lib
+    for batch, M, N, K, short in ((16, 1024, 1024, 128, True), (16, 1024, 512, 128, False), (8, 1024, 1032, 128, True), (16, 1024, 1024, 160, False), (60, 64, 2048, 64, False), (130, 64, 1024, 64, True)):
+        g = torch.Generator(device="cuda").manual_seed(M + N)
+        A = torch.randn(batch, M, K, device="cuda", generator=g).half()
+        B = torch.randn(batch, K, N, device="cuda", generator=g).half()
+        C = torch.empty(batch, M, N, device="cuda", dtype=torch.float16)
+        call = acc.GemmCall(A, B, C)
+        assert ("short K" in _lib.variant_name(call.chosen[0])) == short, (batch, M, N, K, _lib.variant_name(call.chosen[0]))
+        call()
+        want = (A.double() @ B.double()).relu()
+        assert ((C.double() - want).norm() / want.norm()).item() < 2.0 ** -11
