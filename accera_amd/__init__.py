@@ -19,7 +19,8 @@ def __getattr__(name):
     # torch and the DSL are imported on first use so that `import accera_amd` stays light
     if name in ("gemm_relu", "GemmCall"):
         from . import gemm
-        return getattr(gemm, name)
+        value = globals()[name] = getattr(gemm, name)  # (found in the module itself from now on)
+        return value
     if name == "hat":
         import importlib
         return importlib.import_module(".hat", __name__)

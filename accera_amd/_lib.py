@@ -23,7 +23,7 @@ VARIANT_AUTO, VARIANT_SKINNY_BASE, VARIANT_GENERIC, VARIANT_F32_MFMA, VARIANT_SH
 
 EXPORTS = [
     "acc950_init", "acc950_gemm_relu", "acc950_gemm_relu_ex", "acc950_gemm_relu_host", "acc950_gemm_ops", "acc950_gemm_ops_host", "acc950_gemm_ops_static",
-    "acc950_gemm_batched", "acc950_gemm_batched_host", "acc950_bind", "acc950_launch", "acc950_unbind",
+    "acc950_gemm_batched", "acc950_gemm_packed", "acc950_gemm_batched_host", "acc950_bind", "acc950_launch", "acc950_unbind",
     "acc950_launch_geometry", "acc950_num_variants", "acc950_num_skinny_variants",
     "acc950_variant_name", "acc950_last_error",
     "acc950_bound_choice", "acc950_workspace_probe", "acc950_allocation_probe", "acc950_release_workspaces",
@@ -64,6 +64,7 @@ def lib():
     L.acc950_gemm_ops_host.argtypes = [ci, ci, ci, ci, ci] + mat * 3 + [ci, cd, ci, cd]
     bmat = [vp, i64, i64, i64]
     L.acc950_gemm_batched.argtypes = [ci, ci, ci, ci, ci, ci] + bmat * 3 + [ci, cd, ci, cd, ci, ci, vp]
+    L.acc950_gemm_packed.argtypes = [vp]
     L.acc950_gemm_batched_host.argtypes = [ci, ci, ci, ci, ci, ci] + bmat * 3 + [ci, cd, ci, cd, ci, ci]
     L.acc950_bind.argtypes = [ci, ci, ci, ci, ci, ci] + bmat * 3 + [ci, cd, ci, cd, ci, ci, vp, ctypes.POINTER(ci)]
     L.acc950_launch.argtypes = [ci]

@@ -1058,6 +1058,16 @@ int acc950_gemm_batched(int in_type, int out_type, int batch, int M, int N, int 
     return run(pb, c, (hipStream_t)stream, nullptr, false);
 }
 
+int acc950_gemm_packed(const acc950_gemm_call* c)
+{
+    if (!c) return fail(ACC950_INVALID_ARGUMENT, "null call");
+    for (int64_t v : {c->in_type, c->out_type, c->batch, c->M, c->N, c->K, c->prologue, c->epilogue, c->variant, c->k_splits})
+        if (v != (int)v) return fail(ACC950_INVALID_ARGUMENT, "sizes, types, ops and kernel choices are 32-bit numbers");
+    return acc950_gemm_batched((int)c->in_type, (int)c->out_type, (int)c->batch, (int)c->M, (int)c->N, (int)c->K, c->A, c->a_batch_stride, c->a_row_stride,
+                               c->a_col_stride, c->B, c->b_batch_stride, c->b_row_stride, c->b_col_stride, c->C, c->c_batch_stride, c->c_row_stride, c->c_col_stride,
+                               (int)c->prologue, c->prologue_arg, (int)c->epilogue, c->epilogue_arg, (int)c->variant, (int)c->k_splits, c->stream);
+}
+
 // ---- bound calls: validate and choose once, launch many times -------------------------
 struct BoundCall {
     Problem pb;

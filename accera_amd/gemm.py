@@ -1,10 +1,11 @@
 """Device-tensor front end of the C ABI: torch supplies device memory and streams,
 every computation happens in the HIP kernels of libaccera_mi355x.so."""
 import ctypes
+import struct
 
 import torch
 
-from . import _lib
+from . import _lib, tuned
 
 _TORCH_TYPES = {
     torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16,
@@ -13,31 +14,44 @@ _TORCH_TYPES = {
 
 
 def _mat(t, name):
-    if t.dim() not in (2, 3):
+    strides = t.stride()
+    if len(strides) not in (2, 3):
         raise ValueError(f"{name} must be 2-D, or 3-D for a batch")
     if not t.is_cuda:
         raise ValueError(f"{name} must live on the GPU (there is no CPU path)")
-    if t.dim() == 3:
-        return t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)
-    return t.data_ptr(), 0, t.stride(0), t.stride(1)
+    return (t.data_ptr(), *strides) if len(strides) == 3 else (t.data_ptr(), 0, *strides)
 
 
 def _problem(A, B, C):
     """(in type, out type, batch, M, N, K, A ptr + strides, B ..., C ...) of a 2-D call or of a batch
     (3-D tensors (batch, rows, cols); a 2-D A or B is shared by every problem of the batch)."""
-    batch = C.shape[0] if C.dim() == 3 else 1
-    if C.dim() == 2 and (A.dim() == 3 or B.dim() == 3):
-        raise ValueError("a batched A or B needs a 3-D C")
-    for t, name in ((A, "A"), (B, "B")):
-        if t.dim() == 3 and t.shape[0] != batch:
-            raise ValueError(f"{name} has {t.shape[0]} matrices, C has {batch}")
-    M, K = A.shape[-2:]
-    K2, N = B.shape[-2:]
-    if K2 != K or tuple(C.shape[-2:]) != (M, N):
+    a_shape, b_shape, c_shape = A.shape, B.shape, C.shape
+    batch = 1
+    if len(a_shape) != 2 or len(b_shape) != 2 or len(c_shape) != 2:
+        batch = c_shape[0] if len(c_shape) == 3 else 1
+        if len(c_shape) == 2 and (len(a_shape) == 3 or len(b_shape) == 3):
+            raise ValueError("a batched A or B needs a 3-D C")
+        for t, name in ((A, "A"), (B, "B")):
+            if t.dim() == 3 and t.shape[0] != batch:
+                raise ValueError(f"{name} has {t.shape[0]} matrices, C has {batch}")
+        a_shape, b_shape, c_shape = a_shape[-2:], b_shape[-2:], c_shape[-2:]
+    M, K = a_shape
+    K2, N = b_shape
+    if K2 != K or c_shape != (M, N):
         raise ValueError(f"shape mismatch: A {tuple(A.shape)}, B {tuple(B.shape)}, C {tuple(C.shape)}")
-    if A.dtype != B.dtype or A.dtype not in _TORCH_TYPES or C.dtype not in _TORCH_TYPES:
+    dtype = A.dtype
+    in_type, out_type = _TORCH_TYPES.get(dtype), _TORCH_TYPES.get(C.dtype)
+    if B.dtype != dtype or in_type is None or out_type is None:
         raise ValueError(f"unsupported dtypes {A.dtype}, {B.dtype}, {C.dtype}")
-    return (_TORCH_TYPES[A.dtype], _TORCH_TYPES[C.dtype], batch, M, N, K, *_mat(A, "A"), *_mat(B, "B"), *_mat(C, "C"))
+    return (in_type, out_type, batch, M, N, K, *_mat(A, "A"), *_mat(B, "B"), *_mat(C, "C"))
+
+
+def _current_stream(C):
+    """Raw hipStream_t of the stream that is current on C's device."""
+    return torch._C._cuda_getCurrentRawStream(C.get_device())
+
+
+_pack = struct.Struct("19qdqd3q").pack  # acc950_gemm_call
 
 
 class GemmCall:
@@ -52,13 +66,12 @@ class GemmCall:
         hit = None
         if variant == _lib.VARIANT_AUTO and k_splits == 0 and problem[2] == 1:
             # a recorded choice for this very shape (accera_amd.tune --save) goes before the library's cost model
-            from . import tuned
             hit = tuned.lookup(problem[0], problem[1], problem[3], problem[4], problem[5], problem[8:10], problem[12:14], problem[16:18],
                                tuned.ops_class(prologue, prologue_arg, epilogue))
             if hit:
                 variant, k_splits = hit
         if stream is None:
-            stream = torch.cuda.current_stream(C.device).cuda_stream
+            stream = _current_stream(C)
         self.variant, self.k_splits = variant, k_splits  # as asked of the library (after the table look-up)
         self.tensors = (A, B, C)
         L = _lib.lib()
@@ -107,5 +120,20 @@ def gemm_relu(A, B, C, prologue=_lib.PROLOGUE_SET0, epilogue=_lib.EPILOGUE_RELU,
     fp32 -> fp32.  Mirrors calling one function of an Accera package on (A, B, C)
     (/root/reference/README.md:124-130), on device memory.
     """
-    GemmCall(A, B, C, prologue, epilogue, variant, k_splits, stream, prologue_arg, epilogue_arg)()
+    problem = _problem(A, B, C)
+    hit = None
+    if variant == _lib.VARIANT_AUTO and k_splits == 0 and problem[2] == 1:
+        # a recorded choice, as for a GemmCall; if the library refuses it for this call, its own choice runs
+        in_type, out_type, _, M, N, K, _, _, a_rs, a_cs, _, _, b_rs, b_cs, _, _, c_rs, c_cs = problem
+        hit = tuned.recorded(in_type, out_type, M, N, K, a_rs, a_cs, b_rs, b_cs, c_rs, c_cs, tuned.ops_class(prologue, prologue_arg, epilogue))
+        if hit:
+            variant, k_splits = hit
+    if stream is None:
+        stream = _current_stream(C)
+    run = _lib.lib().acc950_gemm_packed
+    rc = run(_pack(*problem, prologue, prologue_arg, epilogue, epilogue_arg, variant, k_splits, stream))
+    if rc and hit:
+        rc = run(_pack(*problem, prologue, prologue_arg, epilogue, epilogue_arg, _lib.VARIANT_AUTO, 0, stream))
+    if rc:
+        _lib.check(rc)
     return C

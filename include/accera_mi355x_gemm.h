@@ -175,6 +175,27 @@ int acc950_gemm_batched_host(int in_type, int out_type, int batch, int M, int N,
                              int variant, int k_splits);
 
 /*
+ * acc950_gemm_batched with its arguments in memory, for callers that pay for every argument they pass through a foreign-function
+ * interface (27 of them cost a Python program more than the launch does).  Read before the function returns.
+ */
+typedef struct acc950_gemm_call {
+    int64_t in_type, out_type, batch, M, N, K;
+    const void* A;
+    int64_t a_batch_stride, a_row_stride, a_col_stride;
+    const void* B;
+    int64_t b_batch_stride, b_row_stride, b_col_stride;
+    void* C;
+    int64_t c_batch_stride, c_row_stride, c_col_stride;
+    int64_t prologue;
+    double prologue_arg;
+    int64_t epilogue;
+    double epilogue_arg;
+    int64_t variant, k_splits;
+    void* stream;
+} acc950_gemm_call;
+int acc950_gemm_packed(const acc950_gemm_call* call);
+
+/*
  * Bound call: validates the problem and chooses the kernel once, then acc950_launch(handle)
  * only launches (asynchronously on the stream given at bind time).  This is what a function
  * of a package is to its caller, a fixed kernel for fixed shapes, with the arrays fixed too;

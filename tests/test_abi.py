@@ -1,6 +1,7 @@
 """The C-ABI library loads without a GPU and exports every symbol the header declares;
 argument checking and the launch-geometry query run on the host alone."""
 import ctypes
+import json
 import os
 import re
 
@@ -360,3 +361,44 @@ def test_tuned_table_is_consulted_by_name_and_validated(tmp_path, monkeypatch):
     assert tuned.lookup(_lib.F16, _lib.F32, 512, 512, 512, (512, 1), (512, 1), (512, 1), True) is None
     assert tuned.lookup(_lib.F16, _lib.F32, 4096, 4096, 4096, (4096, 1), (4096, 1), (4100, 1), True) is None  # padded C: not a table shape
     tuned.reset()
+
+
+def test_recorded_choices_without_asking_the_library(tmp_path, monkeypatch):
+    """tuned.recorded, which an eager call uses, finds what tuned.lookup finds wherever the library takes the recorded kernel."""
+    from accera_amd import tuned
+    F, name = _lib.F16, _lib.variant_name(7)
+    col = next(_lib.variant_name(v) for v in range(_lib.num_variants()) if "A=col-major" in _lib.variant_name(v) and "edge" in _lib.variant_name(v))
+    path = tmp_path / "table.json"
+    path.write_text(json.dumps({
+        tuned.key(F, F, 256, 512, 128, False, False, "lean"): {"kernel": name, "k_splits": 1},
+        tuned.key(F, F, 256, 512, 128, True, False, "acc"): {"kernel": col, "k_splits": 0},
+        tuned.key(F, F, 1, 512, 128, False, False, "lean"): {"kernel": "no such kernel", "k_splits": 0},
+        "not a key": {"kernel": name}}))
+    monkeypatch.setenv("ACCERA_AMD_TUNED", str(path))
+    tuned.reset()
+    try:
+        for M, a, c, ops in ((256, (128, 1), (512, 1), "lean"), (256, (1, 256), (512, 1), "acc"), (256, (1, 256), (512, 1), "lean"), (256, (136, 1), (512, 1), "lean"),
+                             (256, (128, 1), (520, 1), "lean"), (1, (128, 1), (512, 1), "lean"), (257, (128, 1), (512, 1), "lean")):
+            want = tuned.lookup(F, F, M, 512, 128, a, (512, 1), c, ops)
+            assert tuned.recorded(F, F, M, 512, 128, *a, 512, 1, *c, ops) == want, (M, a, c, ops)
+        assert tuned.recorded(F, F, 256, 512, 128, 128, 1, 512, 1, 512, 1, "lean") == (7, 1)
+    finally:
+        monkeypatch.undo()
+        tuned.reset()
+
+
+def test_packed_call_checks_its_numbers():
+    import struct
+    pack = struct.Struct("19qdqd3q").pack
+    L = _lib.lib()
+    head = [_lib.F16, _lib.F16, 1, 64, 64, 64] + [0, 0, 64, 1] * 3
+    assert L.acc950_gemm_packed(None) == _lib.INVALID_ARGUMENT
+    assert L.acc950_gemm_packed(pack(*head, 1, 0.0, 1, 0.0, -1, 0, 0)) == _lib.INVALID_ARGUMENT  # (null matrices)
+    assert "null" in L.acc950_last_error().decode()
+    for i in (0, 2, 3, 5):
+        wide = list(head)
+        wide[i] += 1 << 32
+        assert L.acc950_gemm_packed(pack(*wide, 1, 0.0, 1, 0.0, -1, 0, 0)) == _lib.INVALID_ARGUMENT and "32-bit" in L.acc950_last_error().decode()
+    empty = list(head)
+    empty[3] = 0
+    assert L.acc950_gemm_packed(pack(*empty, 1, 0.0, 1, 0.0, -1, 0, 0)) == _lib.OK  # (nothing to do)
