@@ -1059,23 +1059,26 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
         }
     }
 
-    // ---- pass B: a SET constant, then the epilogue op, each a loop of its own with the one or two instructions per element it needs.
-    // (As one loop with wave-uniform selects over all ops it was about twelve: 32 x (2048x2048x128) fp16 scaled by alpha 111 us on
-    // 128 x 128 tiles, 79 without an epilogue.)
-    if (p.prologue == PRO_SET && p.prologue_arg != 0.f) {
-        const scalar_t set_value = (scalar_t)p.prologue_arg;
-        for_each_acc([&](scalar_t v) { return wrap_add(v, set_value); });
-    }
-    if (p.epilogue == EPI_RELU) for_each_acc([&](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); });
-    else if (p.epilogue == EPI_SCALE) {
-        const scalar_t epi_arg = (scalar_t)p.epilogue_arg;
-        for_each_acc([&](scalar_t v) { return wrap_mul(v, epi_arg); });
-    } else if (p.epilogue != EPI_NONE) {
-        const scalar_t epi_arg = (scalar_t)p.epilogue_arg;
-        const bool is_set = p.epilogue == EPI_SET; // (else ReLU_NoConditional)
+    // ---- pass B: ReLU after a SET-0 prologue is the fused hot path, one max per element; every other combination shares one copy
+    // without a select: (v + constant) * factor, times 0 where ReLU_NoConditional cuts, max with itself or 0, the SET operand over it -- nine instructions
+    // per element.  (With wave-uniform selects over the ops it was about fourteen: 32 x (2048x2048x128) fp16 scaled by alpha 110 us on
+    // 128 x 128 tiles, 82 this way.  Loops of their own per op, two instructions each, are as fast where they fit, but the sums on either side of each
+    // branch are as many registers again: a kilobyte of scratch per lane on 256 x 256 tiles.)
+    if (p.epilogue == EPI_RELU && !(p.prologue == PRO_SET && p.prologue_arg != 0.f)) {
+        for_each_acc([&](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); });
+    } else if (p.epilogue != EPI_NONE || (p.prologue == PRO_SET && p.prologue_arg != 0.f)) {
+        const scalar_t set_value = p.prologue == PRO_SET ? (scalar_t)p.prologue_arg : scalar_t(0);
+        const scalar_t factor = p.epilogue == EPI_SCALE ? (scalar_t)p.epilogue_arg : scalar_t(1); // (x 1 is exact)
+        [[maybe_unused]] const scalar_t cut = scalar_t(p.epilogue == EPI_RELU_NOCOND ? 0 : 1);
+        const unsigned floor_mask = p.epilogue == EPI_RELU || (IN == IN_I8 && p.epilogue == EPI_RELU_NOCOND) ? 0u : ~0u; // lower bound: the value itself, or 0
+        const unsigned keep = p.epilogue == EPI_SET ? 0u : ~0u, put = p.epilogue == EPI_SET ? __builtin_bit_cast(unsigned, (scalar_t)p.epilogue_arg) : 0u;
         for_each_acc([&](scalar_t v) {
-            const scalar_t n = v * (v > scalar_t(0) ? scalar_t(1) : scalar_t(0));
-            return is_set ? epi_arg : n;
+            v = wrap_mul(wrap_add(v, set_value), factor);
+            if constexpr (IN != IN_I8) v = v * (v > scalar_t(0) ? scalar_t(1) : cut); // (of integers it is ReLU)
+            const scalar_t lo = __builtin_bit_cast(scalar_t, __builtin_bit_cast(unsigned, v) & floor_mask);
+            if constexpr (IN == IN_I8) v = v > lo ? v : lo;
+            else v = __builtin_fmaxf(v, lo);
+            return __builtin_bit_cast(scalar_t, (__builtin_bit_cast(unsigned, v) & keep) | put);
         });
     }
     };
