@@ -109,7 +109,11 @@ __device__ __forceinline__ T apply_prologue(T sum, int pro, float arg, LoadC&& l
 // kernel, whose stores are the last thing a 9 us launch does, loses 2.6 us waiting for them to reach memory, and the
 // four-wave kernels (a C far larger than the L2, lines gone before the kernel ends) keep `nt` alone: with `sc1` they
 // measured 1 % slower when C is only written and 0 - 1 % faster when it is read.
+// Not where rows of C do not start on 64-byte boundaries (c_part_lines): two tiles then write parts of the same 64 bytes, and past the L2 each
+// part is a read-modify-write in memory (us, with / without: bf16 2048x2056x512 with an fp32 result 19.7 / 12.2, 8192x1000x512 24.9 / 15.9, fp16 2000x2008x128
+// 7.9 / 5.9, 256x264x256 4.1 / 3.3; with rows on odd multiples of 64 bytes the other way round: int8 2000x2016x128 5.6 / 6.5).
 constexpr int C_STORE_AUX = 16 | 2;
+__device__ __forceinline__ bool c_part_lines(const void* C, int64_t c_rs, unsigned os) { return (((unsigned)c_rs * os) | (unsigned)(size_t)C) % 64 != 0; }
 
 // Store one float accumulator as the output element type.
 __device__ __forceinline__ void store_out(void* C, int out_type, int64_t idx, float v)

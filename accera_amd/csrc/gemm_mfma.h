@@ -938,8 +938,10 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
     // is one 32-bit register, the row of the access a scalar offset and the column block an
     // immediate, so no address registers compete with the live accumulators.
     const int row_in_tile = wr0 + (lane >> 5) * 4, col_in_tile = wc0 + (lane & 31);
-    // fn(descriptor, lane offset, row offset, acc element) -> acc element, for every element of the wave tile
-    auto for_each_element = [&](auto out_tag, auto&& fn) {
+    // fn(descriptor, lane offset, row offset, acc element) -> the same element, for every element of the wave tile
+    // (edge kernels write it back where it came from: without, the compiler moved the narrowing of all sums ahead of the tests, 132 bytes of scratch
+    // for 68 on 256 x 256 tiles; with it, two copies of the loop in the others were a second copy of the sums)
+    auto for_each_element = [&](auto out_tag, auto&& fn) __attribute__((always_inline)) {
         using out_t = decltype(out_tag);
         constexpr unsigned OS = sizeof(out_t);
         const CTile tile = c_tile(p, m0, n0, OS); // uniform
@@ -955,7 +957,8 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     if (EDGE && n0 + col_in_tile + j * 32 >= p.N) continue;
-                    acc[i][j][r] = fn(tile, lane_off + j * 32 * OS, soff, acc[i][j][r]);
+                    const scalar_t same = fn(tile, lane_off + j * 32 * OS, soff, acc[i][j][r]);
+                    if constexpr (EDGE) acc[i][j][r] = same;
                 }
                 if ((r & 3) == 3) __builtin_amdgcn_sched_barrier(0); // keep loads of pass A near their use: no second copy of the tile in registers
             }
@@ -1092,8 +1095,8 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
     constexpr int PITCH_B = PITCH_DW * 4;
     constexpr bool CAN_STAGE = !EDGE && (NT / 64) * 32 * PITCH_B <= Cfg::LDS_BYTES;
     // the wave's slab of 32 rows leaves as 16-byte pieces: rows i*32 .. i*32+31 of the wave tile
-    auto stream_slab = [&](auto out_tag, const char* slab, int i) {
-        constexpr int OS = sizeof(decltype(out_tag));
+    auto stream_slab = [&](auto out_tag, auto aux_tag, const char* slab, int i) __attribute__((always_inline)) {
+        constexpr int OS = sizeof(decltype(out_tag)), AUX = decltype(aux_tag)::value;
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
         const CTile tile = c_tile(p, m0 + (wave_u / WAVES_N) * WTM, n0 + (wave_u % WAVES_N) * WTN, OS);
         const unsigned row_bytes = (unsigned)p.c_rs * OS;
@@ -1106,11 +1109,11 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
             const int row = id / CPRW, cc = id % CPRW;
             const i32x4 v = *(const i32x4*)(slab + row * PITCH_B + cc * 16);
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), tile.rsrc, (unsigned)row * row_bytes + cc * 16,
-                                                   (unsigned)(i * 32) * row_bytes, C_STORE_AUX);
+                                                   (unsigned)(i * 32) * row_bytes, AUX);
         }
     };
     // fp16 / bf16: two columns packed per dword after a swap with the neighbouring lane
-    auto store_staged = [&](auto out_tag, auto relu_tag) {
+    auto store_staged = [&](auto out_tag, auto relu_tag, auto aux_tag) __attribute__((always_inline)) {
         auto fin = [&](float v) { return decltype(relu_tag)::value ? (v > 0.f ? v : 0.f) : v; };
         using out_t = decltype(out_tag);
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
@@ -1141,7 +1144,7 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
                     const int row = (t >> 1) * 8 + (t & 1) * 2 + wrow;
                     slab[row * PITCH_DW + j * 16 + wcol] = __builtin_amdgcn_perm(nbr, own, sel);
                 }
-            stream_slab(uint16_t{}, (const char*)slab, i);
+            stream_slab(uint16_t{}, aux_tag, (const char*)slab, i);
         }
     };
     // int16 / int8: the low bits of the int32 sums, written into the slab at their row-major place
@@ -1160,31 +1163,42 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
                     const int row = (r >> 2) * 8 + (r & 3) + srow;
                     *(out_t*)(slab + row * PITCH_B + (j * 32 + scol) * OS) = (out_t)acc[i][j][r];
                 }
-            stream_slab(out_tag, slab, i);
+            stream_slab(out_tag, std::integral_constant<int, C_STORE_AUX>{}, slab, i);
         }
     };
-    auto store_all = [&](auto relu_tag) {
+    auto store_all = [&](auto relu_tag) __attribute__((always_inline)) {
         auto fin = [&](scalar_t v) { return decltype(relu_tag)::value ? (v > scalar_t(0) ? v : scalar_t(0)) : v; };
         const unsigned os = p.out_type == T_I8 ? 1 : (p.out_type == T_F32 || p.out_type == T_I32) ? 4 : 2;
         // (whole 16-byte pieces of rows: rows 16 bytes apart, and a tile -- a moved last one may start at any column when B is K-contiguous -- on a 16-byte boundary)
         const bool staged = CAN_STAGE && (p.c_rs * os) % 16 == 0 && ((size_t)p.C & 15) == 0 && ((unsigned)n0 * os) % 16 == 0;
-        if constexpr (IN == IN_I8) {
-            if (p.out_type == T_I32) for_each_element(int{}, [&](CTile t, unsigned vo, unsigned so, int v) { c_store<int, EDGE ? 0 : C_STORE_AUX>(t, vo, so, fin(v)); return v; });
-            else if (CAN_STAGE && staged) {
-                if constexpr (CAN_STAGE) {
-                    __syncthreads(); // every wave is done reading the tile buffers
-                    if (p.out_type == T_I16) store_staged_int(int16_t{});
-                    else store_staged_int(int8_t{});
-                }
-            } else if (p.out_type == T_I16) for_each_element(int16_t{}, [&](CTile t, unsigned vo, unsigned so, int v) { c_store<int16_t>(t, vo, so, (int16_t)fin(v)); return v; });
-            else for_each_element(int8_t{}, [&](CTile t, unsigned vo, unsigned so, int v) { c_store<int8_t>(t, vo, so, (int8_t)fin(v)); return v; });
-        } else if (p.out_type == T_F32) for_each_element(float{}, [&](CTile t, unsigned vo, unsigned so, float v) { c_store<float, EDGE ? 0 : C_STORE_AUX>(t, vo, so, fin(v)); return v; });
-        else if (CAN_STAGE && staged) {
+        // Rows of C that do not start on 64-byte boundaries have a copy of the stores of their own, out of the way of the others (with a branch at every
+        // store int8 2048x2064x512 took 9.9 us for 9.0).
+        [[maybe_unused]] const bool part_lines = !EDGE && c_part_lines(p.C, p.c_rs, os);
+        using aux_lines = std::integral_constant<int, EDGE ? 0 : C_STORE_AUX>;
+        [[maybe_unused]] typedef std::integral_constant<int, 0> aux_parts;
+        auto store_32 = [&](auto aux_tag) __attribute__((always_inline)) { for_each_element(scalar_t{}, [&](CTile t, unsigned vo, unsigned so, scalar_t v) { c_store<scalar_t, decltype(aux_tag)::value>(t, vo, so, fin(v)); return v; }); };
+        if (os == 4) {
+            if constexpr (IN == IN_I8) store_32(aux_lines{}); // (one copy, here and below: with two the 256 x 256 kernels use half a kilobyte of scratch)
+            else if (__builtin_expect(part_lines && p.K * ES < 2048, 0)) store_32(aux_parts{}); // (longer: bf16 4096x4104x1024 with an fp32 result 75 us past the L2, 80 through it)
+            else store_32(aux_lines{});
+        } else if (CAN_STAGE && staged) {
             if constexpr (CAN_STAGE) {
                 __syncthreads(); // every wave is done reading the tile buffers
-                if (p.out_type == T_F16) store_staged(_Float16{}, relu_tag);
-                else store_staged(uint16_t{}, relu_tag);
+                if constexpr (IN == IN_I8) {
+                    if (p.out_type == T_I16) store_staged_int(int16_t{});
+                    else store_staged_int(int8_t{});
+                } else if constexpr (IN != IN_F32) {
+                    auto narrow = [&](auto aux_tag) __attribute__((always_inline)) {
+                        if (p.out_type == T_F16) store_staged(_Float16{}, relu_tag, aux_tag);
+                        else store_staged(uint16_t{}, relu_tag, aux_tag);
+                    };
+                    if (__builtin_expect(part_lines, 0)) narrow(aux_parts{});
+                    else narrow(aux_lines{});
+                }
             }
+        } else if constexpr (IN == IN_I8) {
+            if (p.out_type == T_I16) for_each_element(int16_t{}, [&](CTile t, unsigned vo, unsigned so, int v) { c_store<int16_t>(t, vo, so, (int16_t)fin(v)); return v; });
+            else for_each_element(int8_t{}, [&](CTile t, unsigned vo, unsigned so, int v) { c_store<int8_t>(t, vo, so, (int8_t)fin(v)); return v; });
         } else if (p.out_type == T_F16) for_each_element(_Float16{}, [&](CTile t, unsigned vo, unsigned so, float v) { c_store<_Float16>(t, vo, so, (_Float16)fin(v)); return v; }); // RNE
         else for_each_element(uint16_t{}, [&](CTile t, unsigned vo, unsigned so, float v) { c_store<uint16_t>(t, vo, so, float_to_bf16_bits(fin(v))); return v; });
     };

@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256, 2) gemm_short_k_kernel(ACC950_HEAD_PARAMS
     // Descriptor of the workgroup's rows of C: an offset past it is dropped.
     const int rows = p.M - m0 < BM ? p.M - m0 : BM;
     const auto c_rsrc = __builtin_amdgcn_make_buffer_rsrc((char*)p.C + (int64_t)m0 * p.c_rs * OS, 0, (int)((unsigned)(rows - 1) * row_bytes + (unsigned)p.N * OS), 0x00020000);
-    const bool whole_lines = row_bytes % 128 == 0 && ((size_t)p.C & 127) == 0;
+    const bool whole_lines = !c_part_lines(p.C, p.c_rs, OS);
     constexpr unsigned kOutside = 0x80000000u; // (C's rows of a tile span less than 2 GiB)
     const scalar_t set_value = (scalar_t)p.prologue_arg;
     const scalar_t epi_arg = (scalar_t)p.epilogue_arg;
