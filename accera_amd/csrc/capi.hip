@@ -635,12 +635,12 @@ int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats
     return plan_split(v, pb, (int)want, &sp, max_floats) ? sp.splits : 1;
 }
 
-// K of one to four whole k-steps and many tiles of C: the short-K kernel (gemm_short_k.h), if it pays.  Against the other
-// kernels' choice on 220 problems of K = 64 to 256 bytes, 1 to 600 MB of C, every type, layout and ops of this range (geometric mean of the
-// time it saves): more than two of its 64 x 256 tiles per CU and these mostly full 1.8 (us, fp16 32 x (2048x2048x128) scaled 85 / 57, 8192x8192x64
-// 39 / 29, bf16 6352x2952x96 with an fp32 result 54 / 28, int8 47 x (128x4816x128) 105 / 29); with rows of C that end inside a line from one per CU on 1.4,
-// where the others store parts of lines; fewer tiles, a workgroup has nothing to walk along: 0.9 (5136x384x64 3.0 / 4.4), and so where tiles stick
-// out by half (195 x (4608x128x32) 58 / 84).
+// K of one to four whole k-steps and many tiles of C: does the short-K kernel (gemm_short_k.h) pay?  Against the other kernels' choice on 220
+// problems of K = 64 to 256 bytes, 1 to 600 MB of C, every type, layout and ops of this range: with more than three of its 64 x 256 tiles per
+// CU, and these mostly full, it takes 0.6 of the time on average (us, fp16 32 x (2048x2048x128) scaled 85 / 57, 8192x8192x64 39 / 29, bf16 6352x2952x96 with an
+// fp32 result 54 / 28, int8 47 x (128x4816x128) 105 / 29); where rows of C end inside 64 bytes, parts of which the stores of most other kernels send to memory, from one
+// per CU on 0.7; fewer, and a workgroup has nothing to walk along (us, other / this: 5136x384x64 3.0 / 4.4, bf16 4 x (2704x608x96), 516 tiles, with an fp32 result
+// 7.7 / 10.1), and so where tiles stick out by half (195 x (4608x128x32) 58 / 84).
 bool short_k_pays(const Problem& pb)
 {
     const GemmArgs& g = pb.g;
@@ -648,8 +648,8 @@ bool short_k_pays(const Problem& pb)
     // (int8, all four k-steps, a row-major B: the four-wave kernel is level -- 8192x6144x256 43.2 us, 42.6 here; 8192x8192x256 60.8 / 63.5 -- and keeps them)
     if (g.in_type == T_I8 && g.K == 256 && g.a_cs == 1 && g.b_cs == 1 && g.batch <= 1 && g.M >= 256 && g.N >= 256) return false;
     const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 255) / 256), batch = g.batch > 1 ? g.batch : 1;
-    const bool part_lines = (g.c_rs * elem_size(g.out_type)) % 128 != 0;
-    return (double)g.M * g.N >= 0.6 * 64 * 256 * (double)tiles && tiles * batch > (part_lines ? 1 : 2) * kComputeUnits;
+    const bool part_lines = (g.c_rs * elem_size(g.out_type)) % 64 != 0;
+    return (double)g.M * g.N >= 0.6 * 64 * 256 * (double)tiles && tiles * batch > (part_lines ? 1 : 3) * kComputeUnits;
 }
 
 struct Choice {
@@ -1176,7 +1176,7 @@ int acc950_release_workspaces(void)
         it = g_ws_retired.erase(it);
     }
     if (first != hipSuccess) return fail_hip(first, "hipFree");
-    // the host-pointer path's idle contexts: device copies of the largest operands they have carried, 16 MiB of pinned staging each
+    // the host-pointer path's idle contexts: device copies of the largest operands they have carried, 24 or 48 MiB of pinned staging each
     e = host_path_release_idle(dev);
     if (e != hipSuccess) return fail_hip(e, "releasing the host-pointer path's buffers");
     return ACC950_OK;
@@ -1254,7 +1254,44 @@ int acc950_gemm_batched_host(int in_type, int out_type, int batch, int M, int N,
     (void)counted;
     HostOperands h{A, B, C, a_bytes, b_bytes, c_bytes, prologue != PRO_SET || !c_dense};
     int status = ACC950_OK;
-    const hipError_t e = host_path_run(h, [&](void* dA, void* dB, void* dC, hipStream_t stream) {
+    // A large product goes in parts of whole rows of a row-major A and C, so that the first rows of C travel back while later rows of A travel
+    // in: with the kernel that the whole product would run on, unsplit, so that every element is summed as it would be in one piece
+    // (whole rows of 256-row tiles, the remainder with the last part); at least 4 MB of A and C to a part, eight parts at most, from 16 MB on (1024^3 fp16 with an fp32
+    // result, 6 MB, 320 us in one piece, 350 in two).
+    Choice whole{};
+    std::vector<int> first_row; // of every part
+    const auto part_problem = [&](int r0, int rows, void* dA, void* dB, void* dC, Problem* pb) {
+        return make_problem(in_type, out_type, rows, N, K, (const char*)dA + (int64_t)r0 * a_rs * elem_size(in_type), a_rs, a_cs, dB, b_rs, b_cs,
+                            (char*)dC + (int64_t)r0 * c_rs * elem_size(out_type), c_rs, c_cs, prologue, epilogue, true, pb, prologue_arg, epilogue_arg);
+    };
+    const auto rows_of = [&](size_t i) { return (i + 1 < first_row.size() ? first_row[i + 1] : M) - first_row[i]; };
+    const auto plan = [&](void* dA, void* dB, void* dC) {
+        std::vector<HostPart> parts;
+        const size_t part_bytes = (size_t)4 << 20, bytes = a_bytes + c_bytes;
+        if (batch != 1 || h.send_c || c_cs != 1 || a_cs != 1 || a_rs < K || K < 1 || M < 512 || bytes < 4 * part_bytes) return parts;
+        const int blocks = M / 256, n = (int)std::min<size_t>(std::min<size_t>(8, bytes / part_bytes), (size_t)blocks);
+        if (n < 2) return parts;
+        Problem pb;
+        if (part_problem(0, M, dA, dB, dC, &pb) || choose(pb, variant, k_splits, &whole) || whole.splits > 1) return parts;
+        int tables = 0;
+        mfma_table(in_type, &tables);
+        if (whole.variant != ACC950_VARIANT_SHORT_K && (whole.variant < 0 || whole.variant >= tables)) return parts;
+        for (int i = 0; i < n; ++i) first_row.push_back(256 * (int)((int64_t)blocks * i / n));
+        for (size_t i = 0; i < first_row.size(); ++i) {
+            Choice c;
+            if (part_problem(first_row[i], rows_of(i), dA, dB, dC, &pb) || choose(pb, whole.variant, 1, &c)) { first_row.clear(); parts.clear(); return parts; }
+            const size_t r0 = (size_t)first_row[i], rows = (size_t)rows_of(i), es = elem_size(in_type), os = elem_size(out_type);
+            const bool last = i + 1 == first_row.size();
+            parts.push_back(HostPart{r0 * a_rs * es, (last ? a_bytes : (r0 + rows) * a_rs * es) - r0 * a_rs * es, r0 * c_rs * os, rows * c_rs * os});
+        }
+        return parts;
+    };
+    const hipError_t e = host_path_run(h, plan, [&](int part, void* dA, void* dB, void* dC, hipStream_t stream) {
+        if (!first_row.empty()) {
+            Problem pb;
+            const int rc = part_problem(first_row[part], rows_of(part), dA, dB, dC, &pb);
+            return rc ? rc : run(pb, Choice{whole.variant, 1}, stream, nullptr, false);
+        }
         return acc950_gemm_batched(in_type, out_type, batch, M, N, K, dA, a_bs, a_rs, a_cs, dB, b_bs, b_rs, b_cs, dC, c_bs, c_rs, c_cs,
                                    prologue, prologue_arg, epilogue, epilogue_arg, variant, k_splits, stream);
     }, &status);

@@ -10,13 +10,17 @@
 //   * host to device: the caller's bytes are copied into a staging slot by a few worker threads, the slot is sent with
 //     an asynchronous copy, and the next slot is filled meanwhile (a slot is reused once its copy's event has passed);
 //   * the kernel runs on the context's stream behind the copies;
+//   * a large product in several parts (rows of A and C): kernels and copies back have streams and a ring of their own, so that a part
+//     is computed as soon as B and its rows of A are there, and travels back while the next rows travel in;
 //   * device to host: the same ring the other way round -- the copies of the first slots are queued at once, each slot is
 //     copied out to the caller's array when its event has passed and then queued again for a later piece.
 #include "host_path.h"
 
+#include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <immintrin.h>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -25,79 +29,128 @@ namespace acc950 {
 
 namespace {
 
-constexpr size_t kSlotBytes = (size_t)4 << 20; // one staging slot
-constexpr int kSlots = 4;
+// One staging slot, and how many a ring has.  (A copy costs its call about 10 us besides the bytes; 134 MB in parts: 2.44 ms with
+// three slots of 8 MB, 2.65 with four of 4, 2.95 with eight of 2.)
+constexpr size_t kSlotBytes = (size_t)8 << 20;
+constexpr int kSlots = 3;
 constexpr int kCopyThreads = 6;               // workers that move bytes between the caller's arrays and the staging slots
 constexpr size_t kParallelFrom = (size_t)256 << 10; // smaller pieces are copied by the calling thread alone
 
-// ---- worker threads for the copies on the host ------------------------------------------------
+// ---- copies on the host ------------------------------------------------------------------------
+// Stores that go past the caches: neither side of these copies is read again by this program soon, and an ordinary store would
+// first fetch the line it is about to overwrite, half as much memory traffic again.
+__attribute__((target("avx2"))) void stream_copy(char* dst, const char* src, size_t bytes)
+{
+    const size_t head = (32 - ((size_t)dst & 31)) & 31;
+    if (bytes < 4096 + head) { std::memcpy(dst, src, bytes); return; }
+    std::memcpy(dst, src, head);
+    dst += head; src += head; bytes -= head;
+    for (; bytes >= 128; bytes -= 128, dst += 128, src += 128) {
+        const __m256i a = _mm256_loadu_si256((const __m256i*)src), b = _mm256_loadu_si256((const __m256i*)(src + 32)),
+                      c = _mm256_loadu_si256((const __m256i*)(src + 64)), d = _mm256_loadu_si256((const __m256i*)(src + 96));
+        _mm256_stream_si256((__m256i*)dst, a);
+        _mm256_stream_si256((__m256i*)(dst + 32), b);
+        _mm256_stream_si256((__m256i*)(dst + 64), c);
+        _mm256_stream_si256((__m256i*)(dst + 96), d);
+    }
+    std::memcpy(dst, src, bytes);
+    _mm_sfence();
+}
+void copy_bytes(char* dst, const char* src, size_t bytes)
+{
+    static const bool wide = __builtin_cpu_supports("avx2");
+    if (wide) stream_copy(dst, src, bytes);
+    else std::memcpy(dst, src, bytes);
+}
+
 // A fixed set of threads, started at the first large copy.  One copy at a time is dealt out (callers take turns);
-// the calling thread takes a share itself.  The threads live until the process ends.
+// the calling thread takes a share itself.  While a large call is under way (Busy) the threads wait for the next copy without
+// sleeping: a call is a dozen or two copies of 1 to 8 MB, 15 to 100 us each, and waking six sleeping threads takes half as long again.
+// The threads live until the process ends, asleep between calls.
 class CopyPool {
 public:
+    class Busy {
+    public:
+        Busy(CopyPool& pool, bool large) : pool_(large ? &pool : nullptr) { if (pool_) pool_->busy(1); }
+        ~Busy() { if (pool_) pool_->busy(-1); }
+        Busy(const Busy&) = delete;
+        Busy& operator=(const Busy&) = delete;
+
+    private:
+        CopyPool* pool_;
+    };
     void copy(char* dst, const char* src, size_t bytes)
     {
         if (bytes < kParallelFrom) { std::memcpy(dst, src, bytes); return; }
         std::lock_guard<std::mutex> turn(turn_);
         start_workers();
-        const size_t parts = kCopyThreads + 1;
-        const size_t per = ((bytes + parts - 1) / parts + 4095) & ~(size_t)4095;
-        {
-            std::lock_guard<std::mutex> lock(m_);
-            dst_ = dst; src_ = src; bytes_ = bytes; per_ = per;
-            next_part_ = 0; parts_left_ = 0;
-            for (size_t off = 0; off < bytes; off += per) ++parts_left_;
-            ++generation_;
-        }
-        wake_.notify_all();
-        work(); // the caller's share
-        std::unique_lock<std::mutex> lock(m_);
-        done_.wait(lock, [&] { return parts_left_ == 0; });
+        Busy awake(*this, true);
+        Job job;
+        job.dst = dst; job.src = src; job.bytes = bytes;
+        job.per = ((bytes + kCopyThreads) / (kCopyThreads + 1) + 4095) & ~(size_t)4095;
+        job.left = (bytes + job.per - 1) / job.per;
+        job_ = &job;
+        ++generation_;
+        work(job); // the caller's share
+        while (job.left) __builtin_ia32_pause();
+        // (a thread that is still looking at the job counts itself in before it does: none is once the count is zero)
+        job_ = nullptr;
+        while (inside_) __builtin_ia32_pause();
     }
 
 private:
+    struct Job {
+        char* dst;
+        const char* src;
+        size_t bytes, per;
+        std::atomic<size_t> next{0}, left{0};
+    };
     void start_workers()
     {
         if (started_) return;
         started_ = true;
         for (int i = 0; i < kCopyThreads; ++i) std::thread([this] { loop(); }).detach();
     }
-    // takes pieces of the current copy until none is left
-    void work()
+    void busy(int change)
+    {
+        {
+            std::lock_guard<std::mutex> lock(m_);
+            busy_ += change;
+        }
+        if (change > 0) wake_.notify_all();
+    }
+    // takes pieces of the job until none is left
+    static void work(Job& job)
     {
         for (;;) {
-            size_t off;
-            {
-                std::lock_guard<std::mutex> lock(m_);
-                off = next_part_ * per_;
-                if (off >= bytes_) return;
-                ++next_part_;
-            }
-            const size_t n = bytes_ - off < per_ ? bytes_ - off : per_;
-            std::memcpy(dst_ + off, src_ + off, n);
-            std::lock_guard<std::mutex> lock(m_);
-            if (--parts_left_ == 0) done_.notify_all();
+            const size_t off = job.next++ * job.per;
+            if (off >= job.bytes) return;
+            copy_bytes(job.dst + off, job.src + off, job.bytes - off < job.per ? job.bytes - off : job.per);
+            --job.left;
         }
     }
     void loop()
     {
         unsigned long long seen = 0;
         for (;;) {
-            {
+            if (generation_ == seen) {
+                if (busy_) { __builtin_ia32_pause(); continue; }
                 std::unique_lock<std::mutex> lock(m_);
-                wake_.wait(lock, [&] { return generation_ != seen; });
-                seen = generation_;
+                wake_.wait(lock, [&] { return busy_ != 0; });
+                continue;
             }
-            work();
+            seen = generation_;
+            ++inside_;
+            if (Job* job = job_) work(*job);
+            --inside_;
         }
     }
     std::mutex turn_, m_;
-    std::condition_variable wake_, done_;
+    std::condition_variable wake_;
     bool started_ = false;
-    char* dst_ = nullptr;
-    const char* src_ = nullptr;
-    size_t bytes_ = 0, per_ = 1, next_part_ = 0, parts_left_ = 0;
-    unsigned long long generation_ = 0;
+    std::atomic<Job*> job_{nullptr};
+    std::atomic<unsigned long long> generation_{0};
+    std::atomic<int> inside_{0}, busy_{0};
 };
 
 CopyPool& copy_pool()
@@ -118,6 +171,10 @@ struct HostContext {
     DevBuf a, b, c;
     char* slot[kSlots] = {};
     hipEvent_t event[kSlots] = {};
+    // calls in several parts only (made by the first of them)
+    hipStream_t compute = nullptr, back = nullptr;
+    char* back_slot[kSlots] = {};
+    hipEvent_t back_event[kSlots] = {}, arrived = nullptr, computed = nullptr;
 };
 
 std::mutex g_pool_mutex;
@@ -144,6 +201,20 @@ hipError_t make_context(int device, HostContext** out)
     }
     *out = c;
     return hipSuccess;
+}
+
+hipError_t prepare_parts(HostContext& c)
+{
+    hipError_t e = hipSuccess;
+    for (hipStream_t* s : {&c.compute, &c.back})
+        if (e == hipSuccess && !*s) e = hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+    for (hipEvent_t* ev : {&c.arrived, &c.computed})
+        if (e == hipSuccess && !*ev) e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
+    for (int i = 0; i < kSlots; ++i) {
+        if (e == hipSuccess && !c.back_slot[i]) e = hipHostMalloc((void**)&c.back_slot[i], kSlotBytes, hipHostMallocDefault);
+        if (e == hipSuccess && !c.back_event[i]) e = hipEventCreateWithFlags(&c.back_event[i], hipEventDisableTiming);
+    }
+    return e; // (what was made stays with the context, and goes with it)
 }
 
 hipError_t acquire(HostContext** out)
@@ -186,14 +257,23 @@ hipError_t reserve(DevBuf& b, size_t bytes)
     return e;
 }
 
+// Bytes of a piece of a transfer: four pieces, so that one is copied on the host while another is on the bus, but
+// not less than two megabytes (1024^3 fp16 with an fp32 result 367 us with one), and never more than a slot.
+size_t piece_bytes(size_t bytes)
+{
+    const size_t quarter = (bytes / 4 + 65535) & ~(size_t)65535;
+    return std::min(std::max(quarter, (size_t)2 << 20), kSlotBytes);
+}
+
 // caller's array -> device buffer, through the staging ring
 hipError_t upload(HostContext& c, void* dev, const void* host, size_t bytes)
 {
     const char* src = (const char*)host;
+    const size_t step = piece_bytes(bytes);
     size_t piece = 0;
-    for (size_t off = 0; off < bytes; off += kSlotBytes, ++piece) {
+    for (size_t off = 0; off < bytes; off += step, ++piece) {
         const int s = (int)(piece % kSlots);
-        const size_t n = bytes - off < kSlotBytes ? bytes - off : kSlotBytes;
+        const size_t n = std::min(bytes - off, step);
         // (the slot's last copy to the device -- of this call or an earlier one -- has read it)
         hipError_t e = hipEventSynchronize(c.event[s]);
         if (e != hipSuccess) return e;
@@ -209,9 +289,10 @@ hipError_t upload(HostContext& c, void* dev, const void* host, size_t bytes)
 hipError_t download(HostContext& c, void* host, const void* dev, size_t bytes)
 {
     char* dst = (char*)host;
-    const size_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
+    const size_t step = piece_bytes(bytes);
+    const size_t pieces = (bytes + step - 1) / step;
     auto queue = [&](size_t piece) {
-        const size_t off = piece * kSlotBytes, n = bytes - off < kSlotBytes ? bytes - off : kSlotBytes;
+        const size_t off = piece * step, n = std::min(bytes - off, step);
         const int s = (int)(piece % kSlots);
         hipError_t e = hipMemcpyAsync(c.slot[s], (const char*)dev + off, n, hipMemcpyDeviceToHost, c.stream);
         if (e == hipSuccess) e = hipEventRecord(c.event[s], c.stream);
@@ -221,13 +302,93 @@ hipError_t download(HostContext& c, void* host, const void* dev, size_t bytes)
     for (size_t piece = 0; piece < pieces && piece < (size_t)kSlots; ++piece)
         if (hipError_t e = queue(piece); e != hipSuccess) return e;
     for (size_t piece = 0; piece < pieces; ++piece) {
-        const size_t off = piece * kSlotBytes, n = bytes - off < kSlotBytes ? bytes - off : kSlotBytes;
+        const size_t off = piece * step, n = std::min(bytes - off, step);
         const int s = (int)(piece % kSlots);
         hipError_t e = hipEventSynchronize(c.event[s]);
         if (e != hipSuccess) return e;
         copy_pool().copy(dst + off, c.slot[s], n);
         if (piece + kSlots < pieces)
             if (e = queue(piece + kSlots); e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+// Has the event passed?  (A query that answers "not yet" also leaves that as the thread's last error, which the next
+// kernel launch would report.)
+hipError_t passed(hipEvent_t event, bool* yes)
+{
+    const hipError_t e = hipEventQuery(event);
+    *yes = e == hipSuccess;
+    if (e != hipErrorNotReady) return e;
+    (void)hipGetLastError();
+    return hipSuccess;
+}
+
+// A call in several parts: all of B and the first part's bytes of A go in; then every part is launched as its bytes of A have
+// arrived, and its bytes of C come back on a stream of their own while later bytes of A go in.  One thread deals out the copies between
+// the caller's arrays and both rings: whatever slot is ready next, results first.  fp16 4096^3 with an fp32 result, 134 MB over the
+// bus: 3.1 ms one after the other, 2.45 in eight parts.
+hipError_t run_parts(HostContext& c, const HostOperands& h, const std::vector<HostPart>& parts, const HostLaunchFn& launch, int* launch_status)
+{
+    struct Piece { char* dev; char* host; size_t bytes; int part; bool first, last; };
+    std::vector<Piece> in, back;
+    const auto cut = [](std::vector<Piece>& to, char* dev, char* host, size_t bytes, int part) {
+        const size_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes, step = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095; // (equal ones)
+        for (size_t off = 0; off < bytes; off += step) {
+            const size_t n = std::min(bytes - off, step);
+            to.push_back(Piece{dev + off, host + off, n, part, off == 0, off + n == bytes});
+        }
+    };
+    cut(in, (char*)c.b.p, (char*)h.B, h.b_bytes, -1);
+    for (int i = 0; i < (int)parts.size(); ++i) {
+        cut(in, (char*)c.a.p + parts[i].a_off, (char*)h.A + parts[i].a_off, parts[i].a_bytes, i);
+        cut(back, (char*)c.c.p + parts[i].c_off, (char*)h.C + parts[i].c_off, parts[i].c_bytes, i);
+    }
+    size_t sent = 0, queued = 0, drained = 0;
+    int launched = 0;
+    hipError_t e = hipSuccess;
+    while (drained < back.size()) {
+        bool ready = false;
+        if (drained < queued) {
+            if ((e = passed(c.back_event[drained % kSlots], &ready)) != hipSuccess) return e;
+            // (nothing left to send: there is nothing else to do than wait)
+            if (!ready && sent == in.size()) {
+                if ((e = hipEventSynchronize(c.back_event[drained % kSlots])) != hipSuccess) return e;
+                ready = true;
+            }
+            if (ready) {
+                const Piece& p = back[drained];
+                copy_pool().copy(p.host, c.back_slot[drained % kSlots], p.bytes);
+                ++drained;
+            }
+        }
+        if (!ready && sent < in.size()) {
+            const Piece& p = in[sent];
+            const int s = (int)(sent % kSlots);
+            bool free_slot = false;
+            if ((e = passed(c.event[s], &free_slot)) != hipSuccess) return e;
+            // (neither ring has a slot ready: four pieces are on their way in, the oldest is next)
+            if (!free_slot && (e = hipEventSynchronize(c.event[s])) != hipSuccess) return e;
+            copy_pool().copy(c.slot[s], p.host, p.bytes);
+            if ((e = hipMemcpyAsync(p.dev, c.slot[s], p.bytes, hipMemcpyHostToDevice, c.stream)) != hipSuccess) return e;
+            if ((e = hipEventRecord(c.event[s], c.stream)) != hipSuccess) return e;
+            ++sent;
+            if (p.part >= 0 && p.last) {
+                // (a wait takes the event as it was last recorded when the wait is queued: one event serves all parts)
+                if ((e = hipEventRecord(c.arrived, c.stream)) != hipSuccess) return e;
+                if ((e = hipStreamWaitEvent(c.compute, c.arrived, 0)) != hipSuccess) return e;
+                if ((*launch_status = launch(p.part, c.a.p, c.b.p, c.c.p, c.compute)) != 0) return hipSuccess;
+                if ((e = hipEventRecord(c.computed, c.compute)) != hipSuccess) return e;
+                if ((e = hipStreamWaitEvent(c.back, c.computed, 0)) != hipSuccess) return e;
+                ++launched;
+            }
+        }
+        for (; queued < back.size() && queued < drained + kSlots && back[queued].part < launched; ++queued) {
+            const Piece& p = back[queued];
+            const int s = (int)(queued % kSlots);
+            if ((e = hipMemcpyAsync(c.back_slot[s], p.dev, p.bytes, hipMemcpyDeviceToHost, c.back)) != hipSuccess) return e;
+            if ((e = hipEventRecord(c.back_event[s], c.back)) != hipSuccess) return e;
+        }
     }
     return hipSuccess;
 }
@@ -254,34 +415,53 @@ hipError_t host_path_release_idle(int device)
         for (DevBuf* b : {&c->a, &c->b, &c->c})
             if (b->p) note(hipFree(b->p));
         for (int i = 0; i < kSlots; ++i) {
-            if (c->event[i]) note(hipEventDestroy(c->event[i]));
-            if (c->slot[i]) note(hipHostFree(c->slot[i]));
+            for (hipEvent_t ev : {c->event[i], c->back_event[i]})
+                if (ev) note(hipEventDestroy(ev));
+            for (char* p : {c->slot[i], c->back_slot[i]})
+                if (p) note(hipHostFree(p));
         }
-        if (c->stream) note(hipStreamDestroy(c->stream));
+        for (hipEvent_t ev : {c->arrived, c->computed})
+            if (ev) note(hipEventDestroy(ev));
+        for (hipStream_t s : {c->stream, c->compute, c->back})
+            if (s) note(hipStreamDestroy(s));
         delete c;
     }
     return first;
 }
 
-hipError_t host_path_run(const HostOperands& h, const HostLaunchFn& launch, int* launch_status)
+hipError_t host_path_run(const HostOperands& h, const HostPlanFn& plan, const HostLaunchFn& launch, int* launch_status)
 {
     HostContext* c = nullptr;
     hipError_t e = acquire(&c);
     if (e != hipSuccess) return e;
     *launch_status = 0;
+    bool in_parts = false;
+    CopyPool::Busy awake(copy_pool(), h.a_bytes + h.b_bytes + h.c_bytes >= ((size_t)4 << 20));
     do {
         if ((e = reserve(c->a, h.a_bytes ? h.a_bytes : 16)) != hipSuccess) break;
         if ((e = reserve(c->b, h.b_bytes ? h.b_bytes : 16)) != hipSuccess) break;
         if ((e = reserve(c->c, h.c_bytes ? h.c_bytes : 16)) != hipSuccess) break;
+        const std::vector<HostPart> parts = plan(c->a.p, c->b.p, c->c.p);
+        if (parts.size() > 1) {
+            if ((e = prepare_parts(*c)) != hipSuccess) break;
+            in_parts = true;
+            e = run_parts(*c, h, parts, launch, launch_status);
+            break;
+        }
         if ((e = upload(*c, c->a.p, h.A, h.a_bytes)) != hipSuccess) break;
         if ((e = upload(*c, c->b.p, h.B, h.b_bytes)) != hipSuccess) break;
         if (h.send_c && (e = upload(*c, c->c.p, h.C, h.c_bytes)) != hipSuccess) break;
-        *launch_status = launch(c->a.p, c->b.p, c->c.p, c->stream);
+        *launch_status = launch(0, c->a.p, c->b.p, c->c.p, c->stream);
         if (*launch_status != 0) break;
         if ((e = download(*c, h.C, c->c.p, h.c_bytes)) != hipSuccess) break;
     } while (false);
-    // whatever happened, the stream is idle and the slots are free when the context goes back
+    // whatever happened, the streams are idle and the slots are free when the context goes back
     hipError_t e2 = hipStreamSynchronize(c->stream);
+    if (in_parts)
+        for (hipStream_t s : {c->compute, c->back}) {
+            const hipError_t e3 = hipStreamSynchronize(s);
+            if (e2 == hipSuccess) e2 = e3;
+        }
     release(c);
     return e != hipSuccess ? e : e2;
 }

@@ -1603,7 +1603,7 @@ def test_short_k_problems_run_on_the_short_k_kernel():
     import torch
     import accera_amd as acc
     from accera_amd import _lib
-    for batch, M, N, K, short in ((16, 1024, 1024, 128, True), (16, 1024, 512, 128, False), (8, 1024, 1032, 128, True), (16, 1024, 1024, 160, False), (60, 64, 2048, 64, False), (130, 64, 1024, 64, True)):
+    for batch, M, N, K, short in ((16, 1024, 1024, 128, True), (24, 1024, 512, 128, False), (8, 1024, 1032, 128, True), (16, 1024, 1024, 160, False), (96, 64, 2048, 64, False), (200, 64, 1024, 64, True)):
         g = torch.Generator(device="cuda").manual_seed(M + N)
         A = torch.randn(batch, M, K, device="cuda", generator=g).half()
         B = torch.randn(batch, K, N, device="cuda", generator=g).half()
@@ -1613,3 +1613,38 @@ def test_short_k_problems_run_on_the_short_k_kernel():
         call()
         want = (A.double() @ B.double()).relu()
         assert ((C.double() - want).norm() / want.norm()).item() < 2.0 ** -11
+
+
+@pytest.mark.parametrize("in_type,out_type,M,N,K,b_layout,pad", [
+    ("f16", "f32", 2048, 2048, 512, "row", 0),     # four parts of 512 rows
+    ("bf16", "bf16", 1111, 8192, 512, "col", 0),   # a last part with the remainder
+    ("i8", "i32", 1536, 3000, 333, "row", 0),      # nothing aligned
+    ("f32", "f32", 1024, 4096, 512, "row", 8),     # rows of A further apart than they are long
+    ("f16", "f16", 4100, 3000, 128, "col", 0),     # pieces of C that are no multiple of anything
+    ("f16", "f16", 511, 16384, 256, "row", 0),     # too few rows: one piece
+])
+def test_host_call_in_parts_gives_the_bits_of_the_device_call(in_type, out_type, M, N, K, b_layout, pad):
+    """A large product on host arrays goes through the device in parts of whole rows; every element comes out as from one call on
+    device memory, twice in a row on the same context."""
+    import ctypes
+    import torch
+    import accera_amd as acc
+    from accera_amd import _lib
+    rng = np.random.default_rng(M)
+    A = make_input(rng, (M, K + pad), in_type, "normal")
+    B = make_input(rng, (K, N), in_type, "normal")
+    if b_layout == "col":
+        B = np.asfortranarray(B)
+    dA, dB = to_device(A, in_type)[:, :K], to_device(B, in_type)
+    dC = to_device(np.zeros((M, N), ora.NP_STORAGE[out_type]), out_type)
+    acc.GemmCall(dA, dB, dC, variant=acc.VARIANT_AUTO, k_splits=1)()
+    torch.cuda.synchronize()
+    want = to_host(dC, out_type)
+    ids = {"f32": _lib.F32, "f16": _lib.F16, "bf16": _lib.BF16, "i8": _lib.I8, "i32": _lib.I32}
+    strides = (N, 1) if b_layout == "row" else (1, K)
+    for n in range(2):
+        C = np.full((M, N), 3, ora.NP_STORAGE[out_type])
+        _lib.check(_lib.lib().acc950_gemm_ops_host(ids[in_type], ids[out_type], M, N, K, A.ctypes.data_as(ctypes.c_void_p), K + pad, 1,
+                                                   B.ctypes.data_as(ctypes.c_void_p), *strides, C.ctypes.data_as(ctypes.c_void_p), N, 1,
+                                                   _lib.PROLOGUE_SET0, 0.0, _lib.EPILOGUE_RELU, 0.0))
+        assert (C.view(np.uint8) == want.view(np.uint8)).all(), n
