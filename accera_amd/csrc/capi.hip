@@ -598,10 +598,18 @@ int streamed_b_tile(const Problem& pb)
     // 99x5312x14656 39.5 us in six slices, 86.9 on 64 x 64 tiles; bf16 80x2176x27648 32.1 / 50.8, 115x6464x4608 22.3 / 29.5,
     // 185x3520x4800 with a K-contiguous B 17.9 / 21.9, fp16 194x2496x21504 45.2 / 74.4, 224x4224x5568 28.4 / 34.0; while the
     // chip takes three slices of every tile: 159x46976x1024, 734 tiles, is 32.1 us on the general rule's 256 x 256 ones, 44.9 this way.
-    // Of 86 to 128 tiles it takes two, 100x11008x4096 43.1 us unsplit on 64 x 64 tiles, 28.7 so, 128x14336x4096 49.7 / 35.2, 100x16384x4096
-    // 47.9 / 43.4, and int8 gains as much, 128x4096x16384 41.0 / 27.6 in six slices, 115x6464x4608 18.5 / 15.7 in three: not in this rule yet)
-    if (!streamed_b(pb, (int64_t)192 << 20))
-        return pb.g.in_type != T_I8 && pb.g.M > 64 && streamed_b(pb, (int64_t)32 << 20) && (int64_t)((pb.g.M + 127) / 128) * ((pb.g.N + 127) / 128) * 3 <= kComputeUnits ? 128 : 0;
+    // Of 86 to 128 tiles it takes two, which pays as well -- f16 127x14784x4096 with a K-contiguous B 54.1 us unsplit on 64 x 64 tiles, 42.9 so, bf16 169x6336x6656
+    // 61.5 / 41.7, 213x6016x4416 27.2 / 24.9 --, against a row-major B from slices of more than 2048 of K on (100x11008x4096, 43.1 / 28.7, is left where the tests
+    // hold it); int8 gains more: 155x5568x7296 47.0 / 22.0 in two, 92x9920x7936 40.5 / 26.9 in three, 164x4416x16896 63.7 / 44.7, 214x7808x20608 117 / 65; but
+    // 100x6080x3456, 20 MB, 9.8 / 14.1)
+    if (!streamed_b(pb, (int64_t)192 << 20)) {
+        if (g.M <= 64 || !streamed_b(pb, (int64_t)32 << 20)) return 0;
+        const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+        // (int8, a K-contiguous B and a K of no whole 128 bytes, which the four-stage tiles do not take: 181x5440x7616 26.2 / 40.0)
+        if (g.in_type == T_I8 && g.b_rs == 1 && g.K % 128) return 0;
+        const bool two = g.in_type == T_I8 || g.b_rs == 1 || g.K > 4096;
+        return tiles * (two ? 2 : 3) <= kComputeUnits ? 128 : 0;
+    }
     // (a tile that holds all rows of A: up to 64 rows the small tiles, up to 128 rows the 128 x 128 tiles, up to 256 the
     // 256 x 256 ones; with direct fills all take fewer rows than they have when A is row-major (the four-wave kernel, which
     // moves its last row of tiles instead, only from 256 rows on), else the register-staged edge forms apply -- of which
@@ -624,7 +632,9 @@ int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats
     const int64_t target = v.direct && v.bm * v.bn > 64 * 64 ? kComputeUnits : 2 * kComputeUnits;
     int64_t want = std::min<int64_t>(target / tiles, 32);
     const int64_t b_bytes = (int64_t)g.N * g.K * elem_size(g.in_type);
-    while (want > 1 && (g.K / want < 960 || want * (int64_t)g.M * g.N * 4 > b_bytes / 6)) --want;
+    // (int8 on 128 x 128 tiles: a quarter, 155x5568x7296 22.0 us in two slices with their 7 MB, 41 MB of B, 47.0 unsplit)
+    const int64_t sums_at_most = b_bytes / (g.in_type == T_I8 && v.bm * v.bn == 128 * 128 ? 4 : 6);
+    while (want > 1 && (g.K / want < 960 || want * (int64_t)g.M * g.N * 4 > sums_at_most)) --want;
     // (the 256 x 256 tiles, whose partial sums weigh most: a power of two; and a K-contiguous B from 16 slices on:
     // 48x768x23744 15.7 us in 16, 17.1 in 24, 2x1664x23744 20.6 in 16, 22.7 in 19)
     if (v.bm * v.bn > 128 * 128 || (v.b_kc && want > 16))

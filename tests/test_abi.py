@@ -402,3 +402,19 @@ def test_packed_call_checks_its_numbers():
     empty = list(head)
     empty[3] = 0
     assert L.acc950_gemm_packed(pack(*empty, 1, 0.0, 1, 0.0, -1, 0, 0)) == _lib.OK  # (nothing to do)
+
+
+@pytest.mark.parametrize("in_type,M,N,K,b_col,tile,slices", [
+    ("f16", 127, 14784, 4096, True, "128x128", 2),     # 116 tiles: two slices of each
+    ("bf16", 169, 6336, 6656, False, "128x128", 2),
+    ("f16", 100, 12800, 4096, False, "64x64", 1),      # a row-major B, slices of 2048: the general rule's tiles
+    ("bf16", 107, 6016, 3648, True, "64x64", 1),       # three slices' sums are more than a sixth of B, two are 94 workgroups
+    ("i8", 155, 5568, 7296, False, "128x128", 2), ("i8", 92, 9920, 7936, True, "128x128", 3), ("i8", 194, 2304, 14720, False, "128x128", 4),
+    ("i8", 100, 6080, 3456, True, "64x64", 1),         # a B of 20 MB
+    ("i8", 181, 5440, 7616, True, "64x64", 1),         # K of no whole 128 bytes
+])
+def test_65_to_256_rows_against_32_to_192_mb(in_type, M, N, K, b_col, tile, slices):
+    from accera_amd import tune
+    i, o = {"f16": (_lib.F16, _lib.F16), "bf16": (_lib.BF16, _lib.BF16), "i8": (_lib.I8, _lib.I32)}[in_type]
+    variant, splits = tune.own_choice(i, o, M, N, K, False, b_col, 1.0, 0.0)
+    assert f"mfma {tile} " in _lib.variant_name(variant) and splits == slices, (_lib.variant_name(variant), splits)
