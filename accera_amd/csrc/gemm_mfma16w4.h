@@ -500,9 +500,6 @@ __global__ void __launch_bounds__(256, 1) gemm_mfma16w4_kernel(ACC950_HEAD_PARAM
                 const unsigned mine = smem_addr + slab_off + (unsigned)((lane_wb & 15) * PITCH + (lane_wb >> 4) * 16);
                 const CTile tile = c_tile(p, m0 + (wave_u / WAVES_N) * WTM, n0 + (wave_u % WAVES_N) * WTN, OS);
                 const unsigned row_bytes = (unsigned)p.c_rs * OS;
-                // (not where tiles write parts of the same 64 bytes, see C_STORE_AUX: 16 x (1000x1008x256) fp16 21.4 us with, 19.2 without; where C is read as
-                // well, with: 4096x4104x1024 bf16 50.9 / 58.8)
-                const bool part_lines = p.prologue == PRO_SET && c_part_lines(p.C, p.c_rs, OS);
                 // A tile that was moved up / left to end at M / N, of a problem that reads C: its first rows / columns belong
                 // to the neighbouring tile, which may or may not have written them yet -- they are not stored from here.
                 // (first row / column of the wave tile this workgroup owns; 0 wherever nothing is shared)
@@ -530,9 +527,7 @@ __global__ void __launch_bounds__(256, 1) gemm_mfma16w4_kernel(ACC950_HEAD_PARAM
                         acc_t v[VPL / 4];
 #pragma unroll
                         for (int q = 0; q < VPL / 4; ++q) v[q] = finish(*(const acc_t*)(slab + r * PITCH + g * (VPL * 4) + q * 16));
-                        if (part_lines) // (nothing is shared: C is not read)
-                            __builtin_amdgcn_raw_buffer_store_b128(pack(v), tile.rsrc, (unsigned)r * row_bytes + g * 16, (unsigned)(i.value * 16) * row_bytes, 0);
-                        else if (i.value * 16 + r >= own_row && g * VPL >= own_col)
+                        if (i.value * 16 + r >= own_row && g * VPL >= own_col)
                             __builtin_amdgcn_raw_buffer_store_b128(pack(v), tile.rsrc, (unsigned)r * row_bytes + g * 16,
                                                                    (unsigned)(i.value * 16) * row_bytes, AUX);
                     }
