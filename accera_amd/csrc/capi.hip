@@ -662,6 +662,32 @@ bool short_k_pays(const Problem& pb)
     return (double)g.M * g.N >= 0.6 * 64 * 256 * (double)tiles && tiles * batch > (part_lines ? 1 : 3) * kComputeUnits;
 }
 
+// Problems of any alignment with a long K and 30 to 128 tiles of 256 x 256: these tiles fetch half as much per MFMA as the 128 x 128 ones the
+// general rule takes, which unaligned operands pay for dearly, and in as many K slices as the chip holds of them (six at most) they
+// fill it; the sums of the slices need a K of about 3800, int8, with twice as many to a byte, 5000 and fewer tiles (us, 128 x 128 unsplit / so: fp16 1234x5678x4321
+// 122.9 / 104.9 in two, 3913x893x6825 108 / 86 in four, bf16 5060x941x3879 105 / 75 in three, 703x3293x5909 86 / 62 in six, int8 644x7700x5155 86 / 66; but fp16 2140x1916x3269
+// 54.4 / 59.8, int8 2287x1790x4547 47 / 54, 2576x2645x4099, 121 tiles, 67.7 / 70.5).  Moves *mv to that kernel and returns the slices, or 1.
+int staged_large_slices(const Problem& pb, int* mv, size_t max_floats)
+{
+    const GemmArgs& g = pb.g;
+    int n = 0;
+    const MfmaVariant* tab = mfma_table(g.in_type, &n);
+    if (!tab[*mv].any || g.in_type == T_F32 || g.batch > 1) return 1;
+    const bool i8 = g.in_type == T_I8;
+    const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
+    if (g.K < (i8 ? 5000 : 3800) || tiles < 30 || tiles > (i8 ? 100 : 128) || (double)g.M * g.N < 0.75 * 65536.0 * (double)tiles) return 1;
+    const int want = (int)std::min<int64_t>(6, kComputeUnits / tiles);
+    if ((size_t)want * (size_t)g.M * (size_t)g.N > ((size_t)1 << 24)) return 1; // 64 MiB of partial sums at most without being asked
+    for (int i = 0; i < n; ++i) {
+        if (!tab[i].any || tab[i].bm != 256 || !mfma_can_take(tab[i], pb)) continue;
+        SplitPlan sp;
+        if (!plan_split(tab[i], pb, want, &sp, max_floats)) return 1;
+        *mv = i;
+        return sp.splits;
+    }
+    return 1;
+}
+
 struct Choice {
     int variant;
     int splits;
@@ -842,6 +868,10 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
                 else if (one_round || staged_short || (!v.direct && tiles * slices * 2 < kComputeUnits && tiles * slices <= blocks)) mv = -1;
             }
             if (mv < 0) { c->variant = ACC950_VARIANT_F32_MFMA; return ACC950_OK; }
+        }
+        if (mv >= 0 && k_splits == 0) {
+            const int slices = staged_large_slices(pb, &mv, max_split_floats);
+            if (slices > 1) { c->variant = mv; c->splits = slices; return ACC950_OK; }
         }
         c->variant = mv >= 0 ? mv : ACC950_VARIANT_GENERIC;
         if (mv >= 0) {

@@ -418,3 +418,17 @@ def test_65_to_256_rows_against_32_to_192_mb(in_type, M, N, K, b_col, tile, slic
     i, o = {"f16": (_lib.F16, _lib.F16), "bf16": (_lib.BF16, _lib.BF16), "i8": (_lib.I8, _lib.I32)}[in_type]
     variant, splits = tune.own_choice(i, o, M, N, K, False, b_col, 1.0, 0.0)
     assert f"mfma {tile} " in _lib.variant_name(variant) and splits == slices, (_lib.variant_name(variant), splits)
+
+
+@pytest.mark.parametrize("in_type,M,N,K,tile,slices", [
+    ("f16", 1234, 5678, 4321, "256x256", 2), ("f16", 3913, 893, 6825, "256x256", 4), ("bf16", 703, 3293, 5909, "256x256", 6), ("i8", 644, 7700, 5155, "256x256", 2),
+    ("f16", 1234, 5678, 3333, "128x128", 1),      # K too short for the sums of the slices
+    ("f16", 2600, 2900, 4321, "128x128", 1),      # 132 tiles: no two slices of each
+    ("i8", 2576, 2645, 6001, "128x128", 1),
+    ("f16", 520, 8001, 4321, "128x128", 1),       # a last row of tiles that is nearly empty
+])
+def test_large_tiles_in_slices_for_unaligned_problems_with_a_long_k(in_type, M, N, K, tile, slices):
+    from accera_amd import tune
+    i, o = {"f16": (_lib.F16, _lib.F16), "bf16": (_lib.BF16, _lib.BF16), "i8": (_lib.I8, _lib.I32)}[in_type]
+    variant, splits = tune.own_choice(i, o, M, N, K, False, False, 1.0, 0.0)
+    assert f"mfma {tile} " in _lib.variant_name(variant) and "any-alignment" in _lib.variant_name(variant) and splits == slices, (_lib.variant_name(variant), splits)
