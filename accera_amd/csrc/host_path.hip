@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <exception>
 #include <cstring>
 #include <immintrin.h>
 #include <mutex>
@@ -437,6 +438,7 @@ hipError_t host_path_run(const HostOperands& h, const HostPlanFn& plan, const Ho
     *launch_status = 0;
     bool in_parts = false;
     CopyPool::Busy awake(copy_pool(), h.a_bytes + h.b_bytes + h.c_bytes >= ((size_t)4 << 20));
+    try {
     do {
         if ((e = reserve(c->a, h.a_bytes ? h.a_bytes : 16)) != hipSuccess) break;
         if ((e = reserve(c->b, h.b_bytes ? h.b_bytes : 16)) != hipSuccess) break;
@@ -455,6 +457,9 @@ hipError_t host_path_run(const HostOperands& h, const HostPlanFn& plan, const Ho
         if (*launch_status != 0) break;
         if ((e = download(*c, h.C, c->c.p, h.c_bytes)) != hipSuccess) break;
     } while (false);
+    } catch (const std::exception&) { // (the lists of parts and pieces, or a copying thread: no memory for them)
+        e = hipErrorOutOfMemory;
+    }
     // whatever happened, the streams are idle and the slots are free when the context goes back
     hipError_t e2 = hipStreamSynchronize(c->stream);
     if (in_parts)
