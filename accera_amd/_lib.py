@@ -26,7 +26,7 @@ EXPORTS = [
     "acc950_gemm_batched", "acc950_gemm_packed", "acc950_gemm_batched_host", "acc950_bind", "acc950_launch", "acc950_unbind",
     "acc950_launch_geometry", "acc950_num_variants", "acc950_num_skinny_variants",
     "acc950_variant_name", "acc950_last_error",
-    "acc950_bound_choice", "acc950_workspace_probe", "acc950_allocation_probe", "acc950_release_workspaces",
+    "acc950_bound_choice", "acc950_host_parts", "acc950_workspace_probe", "acc950_allocation_probe", "acc950_release_workspaces",
 ]
 # measurement aids (include/accera_mi355x_probes.h, libaccera_mi355x_probes.so): not part of the product
 PROBE_EXPORTS = ["acc950_mfma_ceiling", "acc950_mfma_traffic_probe", "acc950_mfma_phase_probe", "acc950_copy_probe", "acc950_stream_read_probe",
@@ -74,6 +74,7 @@ def lib():
     L.acc950_variant_name.argtypes = [ci, ctypes.c_char_p, ctypes.c_size_t]
     L.acc950_allocation_probe.argtypes = [ctypes.POINTER(ctypes.c_ulonglong)]
     L.acc950_workspace_probe.argtypes = [vp, ctypes.POINTER(vp), ctypes.POINTER(vp)]
+    L.acc950_host_parts.argtypes = [vp, ctypes.POINTER(ci)]
     L.acc950_bound_choice.argtypes = [ci, ctypes.POINTER(ci), ctypes.POINTER(ci)]
     L.acc950_release_workspaces.argtypes = []
     L.acc950_last_error.restype = ctypes.c_char_p

@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <string>
@@ -1030,6 +1031,79 @@ size_t extent_elems(int rows, int cols, int64_t rs, int64_t cs)
     return (size_t)(1 + (int64_t)(rows - 1) * rs + (int64_t)(cols - 1) * cs);
 }
 
+// ---- host arrays ------------------------------------------------------------------------
+// The caller's arrays of a call on host memory, and whether C has to travel in (it is read, or has gaps that the copy back must keep).
+HostOperands host_operands(const acc950_gemm_call& c)
+{
+    const size_t nb = (size_t)(c.batch - 1);
+    const int es = elem_size((int)c.in_type), os = elem_size((int)c.out_type);
+    const size_t a = extent_elems((int)c.M, (int)c.K, c.a_row_stride, c.a_col_stride), b = extent_elems((int)c.K, (int)c.N, c.b_row_stride, c.b_col_stride),
+                 cc = extent_elems((int)c.M, (int)c.N, c.c_row_stride, c.c_col_stride);
+    const bool c_dense = cc == (size_t)c.M * (size_t)c.N && (c.batch == 1 || (size_t)c.c_batch_stride == cc);
+    return HostOperands{c.A, c.B, c.C, (a ? nb * c.a_batch_stride + a : 0) * es, (b ? nb * c.b_batch_stride + b : 0) * es, (nb * c.c_batch_stride + cc) * os,
+                        c.prologue != PRO_SET || !c_dense};
+}
+
+// Rows [r0, r0 + rows) of an unbatched call, on device copies of its operands.
+int host_part_problem(const acc950_gemm_call& c, int r0, int rows, void* dA, void* dB, void* dC, Problem* pb)
+{
+    return make_problem((int)c.in_type, (int)c.out_type, rows, (int)c.N, (int)c.K, (const char*)dA + (int64_t)r0 * c.a_row_stride * elem_size((int)c.in_type), c.a_row_stride, c.a_col_stride,
+                        dB, c.b_row_stride, c.b_col_stride, (char*)dC + (int64_t)r0 * c.c_row_stride * elem_size((int)c.out_type), c.c_row_stride, c.c_col_stride,
+                        (int)c.prologue, (int)c.epilogue, true, pb, c.prologue_arg, c.epilogue_arg);
+}
+
+struct HostPlan {
+    Choice whole{};
+    std::vector<int> first_row; // of every part
+    std::vector<HostPart> parts; // empty: the call goes in one piece
+    int rows(size_t part, int M) const { return (part + 1 < first_row.size() ? first_row[part + 1] : M) - first_row[part]; }
+};
+
+// A large product goes in parts of whole rows of a row-major A and C, so that the first rows of C travel back while later rows of A travel
+// in: with the kernel that the whole product would run on, unsplit, so that every element is summed as it would be in one piece
+// (whole rows of 256-row tiles, the remainder with the last part); at least 4 MB of A and C to a part, eight parts at most, from 16 MB on (1024^3 fp16 with an fp32
+// result, 6 MB, 320 us in one piece, 350 in two).
+// Not where a part's rows of C lie over bytes of A that a later part has yet to read (A and C as shifted views of one array): in one piece all of A is
+// read before anything is written.  (C over B, which is all read first, and C over its own part's or earlier rows of A may stay.)
+bool plan_host_parts_of(const acc950_gemm_call& c, const HostOperands& h, HostPlan* plan)
+{
+    const int M = (int)c.M;
+    const size_t part_bytes = (size_t)4 << 20, bytes = h.a_bytes + h.c_bytes;
+    if (c.batch != 1 || h.send_c || c.c_col_stride != 1 || c.a_col_stride != 1 || c.a_row_stride < c.K || c.K < 1 || M < 512 || bytes < 4 * part_bytes) return false;
+    const int blocks = M / 256, n = (int)std::min<size_t>(std::min<size_t>(8, bytes / part_bytes), (size_t)blocks);
+    if (n < 2) return false;
+    // (addresses of the device copies do not matter beyond their alignment, which is an allocation's)
+    void* const at = (void*)(uintptr_t)4096;
+    Problem pb;
+    if (host_part_problem(c, 0, M, at, at, at, &pb) || choose(pb, (int)c.variant, (int)c.k_splits, &plan->whole) || plan->whole.splits > 1) return false;
+    int tables = 0;
+    mfma_table((int)c.in_type, &tables);
+    if (plan->whole.variant != ACC950_VARIANT_SHORT_K && (plan->whole.variant < 0 || plan->whole.variant >= tables)) return false;
+    for (int i = 0; i < n; ++i) plan->first_row.push_back(256 * (int)((int64_t)blocks * i / n));
+    const size_t a_row = (size_t)c.a_row_stride * elem_size((int)c.in_type), c_row = (size_t)c.c_row_stride * elem_size((int)c.out_type);
+    for (size_t i = 0; i < plan->first_row.size(); ++i) {
+        Choice same;
+        if (host_part_problem(c, plan->first_row[i], plan->rows(i, M), at, at, at, &pb) || choose(pb, plan->whole.variant, 1, &same)) return false;
+        const size_t r0 = (size_t)plan->first_row[i], rows = (size_t)plan->rows(i, M);
+        const bool last = i + 1 == plan->first_row.size();
+        plan->parts.push_back(HostPart{r0 * a_row, (last ? h.a_bytes : (r0 + rows) * a_row) - r0 * a_row, r0 * c_row, rows * c_row});
+    }
+    for (size_t i = 0; i + 1 < plan->parts.size(); ++i) {
+        const uintptr_t written = (uintptr_t)h.C + plan->parts[i].c_off, unread = (uintptr_t)h.A + plan->parts[i + 1].a_off, end = (uintptr_t)h.A + h.a_bytes;
+        if (written < end && unread < written + plan->parts[i].c_bytes) return false;
+    }
+    return true;
+}
+void plan_host_parts(const acc950_gemm_call& c, const HostOperands& h, HostPlan* plan)
+{
+    try {
+        if (plan_host_parts_of(c, h, plan)) return;
+    } catch (const std::exception&) { // (no memory for the lists)
+    }
+    plan->first_row.clear();
+    plan->parts.clear();
+}
+
 } // namespace
 
 extern "C" {
@@ -1281,62 +1355,46 @@ int acc950_gemm_batched_host(int in_type, int out_type, int batch, int M, int N,
                           prologue_arg, epilogue_arg, bt);
     if (rc) return rc;
     if (M == 0 || N == 0 || batch == 0) return ACC950_OK;
-    const size_t nb = (size_t)(batch - 1);
-    const size_t a_elems = extent_elems(M, K, a_rs, a_cs), b_elems = extent_elems(K, N, b_rs, b_cs), c_elems = extent_elems(M, N, c_rs, c_cs);
-    const size_t a_bytes = (a_elems ? nb * a_bs + a_elems : 0) * elem_size(in_type);
-    const size_t b_bytes = (b_elems ? nb * b_bs + b_elems : 0) * elem_size(in_type);
-    const size_t c_bytes = (nb * c_bs + c_elems) * elem_size(out_type);
-    const bool c_dense = c_elems == (size_t)M * (size_t)N && (batch == 1 || (size_t)c_bs == c_elems);
-
     // Through pinned staging on a context of this call's own (host_path.hip): calls from different host threads do not
     // wait for each other.
     static const bool counted = (host_path_count_allocations(&g_device_allocations), true);
     (void)counted;
-    HostOperands h{A, B, C, a_bytes, b_bytes, c_bytes, prologue != PRO_SET || !c_dense};
+    const acc950_gemm_call call{in_type, out_type, batch, M, N, K, A, a_bs, a_rs, a_cs, B, b_bs, b_rs, b_cs, C, c_bs, c_rs, c_cs,
+                                prologue, prologue_arg, epilogue, epilogue_arg, variant, k_splits, nullptr};
+    const HostOperands h = host_operands(call);
     int status = ACC950_OK;
-    // A large product goes in parts of whole rows of a row-major A and C, so that the first rows of C travel back while later rows of A travel
-    // in: with the kernel that the whole product would run on, unsplit, so that every element is summed as it would be in one piece
-    // (whole rows of 256-row tiles, the remainder with the last part); at least 4 MB of A and C to a part, eight parts at most, from 16 MB on (1024^3 fp16 with an fp32
-    // result, 6 MB, 320 us in one piece, 350 in two).
-    Choice whole{};
-    std::vector<int> first_row; // of every part
-    const auto part_problem = [&](int r0, int rows, void* dA, void* dB, void* dC, Problem* pb) {
-        return make_problem(in_type, out_type, rows, N, K, (const char*)dA + (int64_t)r0 * a_rs * elem_size(in_type), a_rs, a_cs, dB, b_rs, b_cs,
-                            (char*)dC + (int64_t)r0 * c_rs * elem_size(out_type), c_rs, c_cs, prologue, epilogue, true, pb, prologue_arg, epilogue_arg);
-    };
-    const auto rows_of = [&](size_t i) { return (i + 1 < first_row.size() ? first_row[i + 1] : M) - first_row[i]; };
-    const auto plan = [&](void* dA, void* dB, void* dC) {
-        std::vector<HostPart> parts;
-        const size_t part_bytes = (size_t)4 << 20, bytes = a_bytes + c_bytes;
-        if (batch != 1 || h.send_c || c_cs != 1 || a_cs != 1 || a_rs < K || K < 1 || M < 512 || bytes < 4 * part_bytes) return parts;
-        const int blocks = M / 256, n = (int)std::min<size_t>(std::min<size_t>(8, bytes / part_bytes), (size_t)blocks);
-        if (n < 2) return parts;
-        Problem pb;
-        if (part_problem(0, M, dA, dB, dC, &pb) || choose(pb, variant, k_splits, &whole) || whole.splits > 1) return parts;
-        int tables = 0;
-        mfma_table(in_type, &tables);
-        if (whole.variant != ACC950_VARIANT_SHORT_K && (whole.variant < 0 || whole.variant >= tables)) return parts;
-        for (int i = 0; i < n; ++i) first_row.push_back(256 * (int)((int64_t)blocks * i / n));
-        for (size_t i = 0; i < first_row.size(); ++i) {
-            Choice c;
-            if (part_problem(first_row[i], rows_of(i), dA, dB, dC, &pb) || choose(pb, whole.variant, 1, &c)) { first_row.clear(); parts.clear(); return parts; }
-            const size_t r0 = (size_t)first_row[i], rows = (size_t)rows_of(i), es = elem_size(in_type), os = elem_size(out_type);
-            const bool last = i + 1 == first_row.size();
-            parts.push_back(HostPart{r0 * a_rs * es, (last ? a_bytes : (r0 + rows) * a_rs * es) - r0 * a_rs * es, r0 * c_rs * os, rows * c_rs * os});
-        }
-        return parts;
-    };
-    const hipError_t e = host_path_run(h, plan, [&](int part, void* dA, void* dB, void* dC, hipStream_t stream) {
-        if (!first_row.empty()) {
+    HostPlan plan;
+    plan_host_parts(call, h, &plan);
+    const hipError_t e = host_path_run(h, plan.parts, [&](int part, void* dA, void* dB, void* dC, hipStream_t stream) {
+        if (part >= 0) {
             Problem pb;
-            const int rc = part_problem(first_row[part], rows_of(part), dA, dB, dC, &pb);
-            return rc ? rc : run(pb, Choice{whole.variant, 1}, stream, nullptr, false);
+            const int rc = host_part_problem(call, plan.first_row[part], plan.rows(part, M), dA, dB, dC, &pb);
+            return rc ? rc : run(pb, Choice{plan.whole.variant, 1}, stream, nullptr, false);
         }
         return acc950_gemm_batched(in_type, out_type, batch, M, N, K, dA, a_bs, a_rs, a_cs, dB, b_bs, b_rs, b_cs, dC, c_bs, c_rs, c_cs,
                                    prologue, prologue_arg, epilogue, epilogue_arg, variant, k_splits, stream);
     }, &status);
     if (status != ACC950_OK) return status; // (the launcher's own error text stands)
     if (e != hipSuccess) return fail_hip(e, "host-pointer path (allocation or copy)");
+    return ACC950_OK;
+}
+
+int acc950_host_parts(const acc950_gemm_call* c, int* parts)
+{
+    if (!c || !parts) return fail(ACC950_INVALID_ARGUMENT, "null call or result");
+    for (int64_t v : {c->in_type, c->out_type, c->batch, c->M, c->N, c->K, c->prologue, c->epilogue, c->variant, c->k_splits})
+        if (v != (int)v) return fail(ACC950_INVALID_ARGUMENT, "sizes, types, ops and kernel choices are 32-bit numbers");
+    Problem check;
+    Batch bt;
+    bt.count = (int)c->batch; bt.a_bs = c->a_batch_stride; bt.b_bs = c->b_batch_stride; bt.c_bs = c->c_batch_stride;
+    const int rc = make_problem((int)c->in_type, (int)c->out_type, (int)c->M, (int)c->N, (int)c->K, c->A, c->a_row_stride, c->a_col_stride, c->B, c->b_row_stride, c->b_col_stride,
+                                c->C, c->c_row_stride, c->c_col_stride, (int)c->prologue, (int)c->epilogue, true, &check, c->prologue_arg, c->epilogue_arg, bt);
+    if (rc) return rc;
+    *parts = 0;
+    if (c->M == 0 || c->N == 0 || c->batch == 0) return ACC950_OK;
+    HostPlan plan;
+    plan_host_parts(*c, host_operands(*c), &plan);
+    *parts = plan.parts.empty() ? 1 : (int)plan.parts.size();
     return ACC950_OK;
 }
 

@@ -18,19 +18,17 @@ struct HostOperands {
 };
 
 // Part of a call whose result depends on all of B and on one stretch of A's bytes only, and is one stretch of C's (rows of a row-major
-// product).  The parts of a call cover A and C.
+// product).  The parts of a call cover A and C, in order, and no part's stretch of C lies over a later part's stretch of A.
 struct HostPart {
     size_t a_off, a_bytes, c_off, c_bytes;
 };
-// the call's parts, in the order they are to run, once its device copies of A, B, C have their places (empty: one part)
-typedef std::function<std::vector<HostPart>(void* dA, void* dB, void* dC)> HostPlanFn;
-// launches part number `part` (of a call in one part: all of it) on device copies of A, B, C on `stream`; returns the library's status code (0: ok)
+// launches part number `part` (-1: all of the call) on device copies of A, B, C on `stream`; returns the library's status code (0: ok)
 typedef std::function<int(int part, void* dA, void* dB, void* dC, hipStream_t stream)> HostLaunchFn;
 
-// Copies in, launches, copies C back, and returns when C is in the caller's memory.  With several parts, one part of C travels back while later
+// Copies in, launches, copies C back, and returns when C is in the caller's memory.  With several parts (none or one: in one piece), one part of C travels back while later
 // parts of A are still on their way in.  The HIP error of a copy or an allocation comes back as the return value, the
 // launcher's status in *launch_status.  Calls from different host threads run side by side, each on a context of its own.
-hipError_t host_path_run(const HostOperands& h, const HostPlanFn& plan, const HostLaunchFn& launch, int* launch_status);
+hipError_t host_path_run(const HostOperands& h, const std::vector<HostPart>& parts, const HostLaunchFn& launch, int* launch_status);
 
 // Frees the contexts of `device` that no call is using (their device buffers, pinned staging slots, events and streams);
 // the next call on a host pointer makes a new one.

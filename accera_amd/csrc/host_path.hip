@@ -331,13 +331,13 @@ hipError_t passed(hipEvent_t event, bool* yes)
 // bus: 3.1 ms one after the other, 2.45 in eight parts.
 hipError_t run_parts(HostContext& c, const HostOperands& h, const std::vector<HostPart>& parts, const HostLaunchFn& launch, int* launch_status)
 {
-    struct Piece { char* dev; char* host; size_t bytes; int part; bool first, last; };
+    struct Piece { char* dev; char* host; size_t bytes; int part; bool last; };
     std::vector<Piece> in, back;
     const auto cut = [](std::vector<Piece>& to, char* dev, char* host, size_t bytes, int part) {
         const size_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes, step = ((bytes + pieces - 1) / pieces + 4095) & ~(size_t)4095; // (equal ones)
         for (size_t off = 0; off < bytes; off += step) {
             const size_t n = std::min(bytes - off, step);
-            to.push_back(Piece{dev + off, host + off, n, part, off == 0, off + n == bytes});
+            to.push_back(Piece{dev + off, host + off, n, part, off + n == bytes});
         }
     };
     cut(in, (char*)c.b.p, (char*)h.B, h.b_bytes, -1);
@@ -368,7 +368,7 @@ hipError_t run_parts(HostContext& c, const HostOperands& h, const std::vector<Ho
             const int s = (int)(sent % kSlots);
             bool free_slot = false;
             if ((e = passed(c.event[s], &free_slot)) != hipSuccess) return e;
-            // (neither ring has a slot ready: four pieces are on their way in, the oldest is next)
+            // (neither ring has a slot ready: every slot of the way in is on the bus, the oldest is next)
             if (!free_slot && (e = hipEventSynchronize(c.event[s])) != hipSuccess) return e;
             copy_pool().copy(c.slot[s], p.host, p.bytes);
             if ((e = hipMemcpyAsync(p.dev, c.slot[s], p.bytes, hipMemcpyHostToDevice, c.stream)) != hipSuccess) return e;
@@ -430,7 +430,7 @@ hipError_t host_path_release_idle(int device)
     return first;
 }
 
-hipError_t host_path_run(const HostOperands& h, const HostPlanFn& plan, const HostLaunchFn& launch, int* launch_status)
+hipError_t host_path_run(const HostOperands& h, const std::vector<HostPart>& parts, const HostLaunchFn& launch, int* launch_status)
 {
     HostContext* c = nullptr;
     hipError_t e = acquire(&c);
@@ -443,21 +443,22 @@ hipError_t host_path_run(const HostOperands& h, const HostPlanFn& plan, const Ho
         if ((e = reserve(c->a, h.a_bytes ? h.a_bytes : 16)) != hipSuccess) break;
         if ((e = reserve(c->b, h.b_bytes ? h.b_bytes : 16)) != hipSuccess) break;
         if ((e = reserve(c->c, h.c_bytes ? h.c_bytes : 16)) != hipSuccess) break;
-        const std::vector<HostPart> parts = plan(c->a.p, c->b.p, c->c.p);
         if (parts.size() > 1) {
-            if ((e = prepare_parts(*c)) != hipSuccess) break;
-            in_parts = true;
-            e = run_parts(*c, h, parts, launch, launch_status);
-            break;
+            if (prepare_parts(*c) == hipSuccess) {
+                in_parts = true;
+                e = run_parts(*c, h, parts, launch, launch_status);
+                break;
+            }
+            (void)hipGetLastError(); // (no second ring to be had: in one piece then)
         }
         if ((e = upload(*c, c->a.p, h.A, h.a_bytes)) != hipSuccess) break;
         if ((e = upload(*c, c->b.p, h.B, h.b_bytes)) != hipSuccess) break;
         if (h.send_c && (e = upload(*c, c->c.p, h.C, h.c_bytes)) != hipSuccess) break;
-        *launch_status = launch(0, c->a.p, c->b.p, c->c.p, c->stream);
+        *launch_status = launch(-1, c->a.p, c->b.p, c->c.p, c->stream);
         if (*launch_status != 0) break;
         if ((e = download(*c, h.C, c->c.p, h.c_bytes)) != hipSuccess) break;
     } while (false);
-    } catch (const std::exception&) { // (the lists of parts and pieces, or a copying thread: no memory for them)
+    } catch (const std::exception&) { // (the lists of pieces, or a copying thread: no memory for them)
         e = hipErrorOutOfMemory;
     }
     // whatever happened, the streams are idle and the slots are free when the context goes back

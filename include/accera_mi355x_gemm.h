@@ -259,6 +259,13 @@ int acc950_variant_name(int variant, char* buf, size_t buf_len);
  */
 int acc950_workspace_probe(void* stream, void** partial_sums, void** counters);
 
+/*
+ * In how many parts of rows a call of acc950_gemm_batched_host with these arguments (host pointers; `stream` is not read)
+ * goes through the device: 1 in one piece, 0 nothing to do.  Parts overlap the copies of A and C; operands that lie over
+ * each other are answered as if all of A and B were read before C is written, whatever the number.  Host only, nothing runs.
+ */
+int acc950_host_parts(const acc950_gemm_call* call, int* parts);
+
 /* Number of device allocations (hipMalloc) the GEMM entry points of this process have made so far: K-split
  * workspaces and the device buffers of the host-pointer path.  A test of an entry point that must not allocate
  * reads it before and after. */

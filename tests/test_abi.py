@@ -432,3 +432,32 @@ def test_large_tiles_in_slices_for_unaligned_problems_with_a_long_k(in_type, M, 
     i, o = {"f16": (_lib.F16, _lib.F16), "bf16": (_lib.BF16, _lib.BF16), "i8": (_lib.I8, _lib.I32)}[in_type]
     variant, splits = tune.own_choice(i, o, M, N, K, False, False, 1.0, 0.0)
     assert f"mfma {tile} " in _lib.variant_name(variant) and "any-alignment" in _lib.variant_name(variant) and splits == slices, (_lib.variant_name(variant), splits)
+
+
+def _host_parts(tin, tout, M, N, K, a=1 << 40, b=2 << 40, c=3 << 40, a_rs=None, c_rs=None, b_strides=None, prologue=1, batch=1):
+    import struct
+    parts, (b_rs, b_cs) = ctypes.c_int(-1), b_strides or (N, 1)
+    call = struct.Struct("19qdqd3q").pack(tin, tout, batch, M, N, K, a, M * K * (batch > 1), a_rs or K, 1, b, K * N * (batch > 1), b_rs, b_cs, c, M * N * (batch > 1), c_rs or N, 1,
+                                          prologue, 0.0, _lib.EPILOGUE_RELU, 0.0, _lib.VARIANT_AUTO, 0, 0)
+    _lib.check(_lib.lib().acc950_host_parts(call, ctypes.byref(parts)))
+    return parts.value
+
+
+def test_host_calls_whose_operands_overlap_go_in_one_piece():
+    """In parts, C's first rows are written while A's later rows are unread: not where they are the same bytes."""
+    F16, F32 = _lib.F16, _lib.F32
+    n, row, x = 4096, 2 * 4096, 1 << 40
+    whole = _host_parts(F16, F16, n, n, n)
+    assert whole == 8
+    assert _host_parts(F16, F16, n, n, n, a=x, c=x + row) == 1                       # A = X[:-1], C = X[1:]
+    assert _host_parts(F16, F16, n, n, n, a=x, c=x + 2) == 1                         # one element on
+    assert _host_parts(F16, F16, n, n, n, a=x, c=x + (n - 1) * row) == 1             # C over A's last row
+    assert _host_parts(F16, F32, n, n, n, a=x, c=x) == 1                             # an fp16 A at the start of an fp32 C's buffer
+    assert _host_parts(F16, F16, n, n, n, a=x, c=x, a_rs=n + 8) == whole             # C's rows lie before A's of the same number ...
+    assert _host_parts(F16, F16, n, n, n, a=x + row, c=x) == whole                   # ... A = X[1:], C = X[:-1]
+    assert _host_parts(F16, F16, n, n, n, a=x, c=x) == whole                         # the same array
+    assert _host_parts(F16, F16, n, n, n, b=3 << 40) == whole                        # C over B, which is read first
+    assert _host_parts(F16, F16, n, n, n, a=x, c=x + n * row) == whole               # neighbours
+    assert _host_parts(F16, F16, n, n, n, prologue=0) == 1 and _host_parts(F16, F16, n, n, n, batch=2) == 1 and _host_parts(F16, F16, 0, n, n) == 0
+    parts = ctypes.c_int()
+    assert _lib.lib().acc950_host_parts(None, ctypes.byref(parts)) == _lib.INVALID_ARGUMENT

@@ -1615,15 +1615,26 @@ def test_short_k_problems_run_on_the_short_k_kernel():
         assert ((C.double() - want).norm() / want.norm()).item() < 2.0 ** -11
 
 
-@pytest.mark.parametrize("in_type,out_type,M,N,K,b_layout,pad", [
-    ("f16", "f32", 2048, 2048, 512, "row", 0),     # four parts of 512 rows
-    ("bf16", "bf16", 1111, 8192, 512, "col", 0),   # a last part with the remainder
-    ("i8", "i32", 1536, 3000, 333, "row", 0),      # nothing aligned
-    ("f32", "f32", 1024, 4096, 512, "row", 8),     # rows of A further apart than they are long
-    ("f16", "f16", 4100, 3000, 128, "col", 0),     # pieces of C that are no multiple of anything
-    ("f16", "f16", 511, 16384, 256, "row", 0),     # too few rows: one piece
+def _host_parts(in_id, out_id, M, N, K, a, a_rs, b, b_strides, c):
+    """In how many parts acc950_gemm_ops_host takes such a call through the device."""
+    import ctypes
+    import struct
+    from accera_amd import _lib
+    parts = ctypes.c_int(-1)
+    _lib.check(_lib.lib().acc950_host_parts(struct.Struct("19qdqd3q").pack(in_id, out_id, 1, M, N, K, a, 0, a_rs, 1, b, 0, *b_strides, c, 0, N, 1, _lib.PROLOGUE_SET0, 0.0,
+                                                                          _lib.EPILOGUE_RELU, 0.0, _lib.VARIANT_AUTO, 0, 0), ctypes.byref(parts)))
+    return parts.value
+
+
+@pytest.mark.parametrize("in_type,out_type,M,N,K,b_layout,pad,parts", [
+    ("f16", "f32", 2048, 2048, 512, "row", 0, 4),     # four parts of 512 rows
+    ("bf16", "bf16", 1111, 8192, 512, "col", 0, 4),   # a last part with the remainder
+    ("i8", "i32", 1536, 3000, 333, "row", 0, 4),      # nothing aligned
+    ("f32", "f32", 1024, 4096, 512, "row", 8, 4),     # rows of A further apart than they are long
+    ("f16", "f16", 4100, 3000, 128, "col", 0, 6),     # pieces of C that are no multiple of anything
+    ("f16", "f16", 511, 16384, 256, "row", 0, 1),     # too few rows: one piece
 ])
-def test_host_call_in_parts_gives_the_bits_of_the_device_call(in_type, out_type, M, N, K, b_layout, pad):
+def test_host_call_in_parts_gives_the_bits_of_the_device_call(in_type, out_type, M, N, K, b_layout, pad, parts):
     """A large product on host arrays goes through the device in parts of whole rows; every element comes out as from one call on
     device memory, twice in a row on the same context."""
     import ctypes
@@ -1644,7 +1655,31 @@ def test_host_call_in_parts_gives_the_bits_of_the_device_call(in_type, out_type,
     strides = (N, 1) if b_layout == "row" else (1, K)
     for n in range(2):
         C = np.full((M, N), 3, ora.NP_STORAGE[out_type])
+        assert _host_parts(ids[in_type], ids[out_type], M, N, K, A.ctypes.data, K + pad, B.ctypes.data, strides, C.ctypes.data) == parts
         _lib.check(_lib.lib().acc950_gemm_ops_host(ids[in_type], ids[out_type], M, N, K, A.ctypes.data_as(ctypes.c_void_p), K + pad, 1,
                                                    B.ctypes.data_as(ctypes.c_void_p), *strides, C.ctypes.data_as(ctypes.c_void_p), N, 1,
                                                    _lib.PROLOGUE_SET0, 0.0, _lib.EPILOGUE_RELU, 0.0))
         assert (C.view(np.uint8) == want.view(np.uint8)).all(), n
+
+
+@pytest.mark.parametrize("a_row,c_row,parts", [(0, 1, 1), (1, 0, 8), (0, 0, 8), (0, 300, 1), (0, 2500, 1), (2500, 0, 8)])
+def test_host_call_whose_c_lies_over_a(a_row, c_row, parts):
+    """A and C as views of one host array, some rows apart: the result is that of a C of its own."""
+    import ctypes
+    import torch
+    from accera_amd import _lib
+    M, N = 4096, 2048
+    rng = np.random.default_rng(5)
+    B = (make_input(rng, (N, N), "f16", "normal").astype(np.float32) * N ** -0.5).astype(np.float16)
+    X = make_input(rng, (M + 2500, N), "f16", "normal")
+    A, C = X[a_row:a_row + M], X[c_row:c_row + M]
+    dC = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    dA, dB = to_device(A, "f16"), to_device(B, "f16")
+    _lib.check(_lib.lib().acc950_gemm_ops(_lib.F16, _lib.F16, M, N, N, dA.data_ptr(), N, 1, dB.data_ptr(), N, 1, dC.data_ptr(), N, 1, _lib.PROLOGUE_SET0, 0.0, _lib.EPILOGUE_RELU, 0.0,
+                                          _lib.VARIANT_AUTO, 1, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    want = to_host(dC, "f16")
+    assert _host_parts(_lib.F16, _lib.F16, M, N, N, A.ctypes.data, N, B.ctypes.data, (N, 1), C.ctypes.data) == parts
+    P = lambda x: x.ctypes.data_as(ctypes.c_void_p)
+    _lib.check(_lib.lib().acc950_gemm_ops_host(_lib.F16, _lib.F16, M, N, N, P(A), N, 1, P(B), N, 1, P(C), N, 1, _lib.PROLOGUE_SET0, 0.0, _lib.EPILOGUE_RELU, 0.0))
+    assert (C.view(np.uint16) == want.view(np.uint16)).all()
