@@ -126,7 +126,9 @@ __global__ void __launch_bounds__(256, 2) gemm_short_k_kernel(ACC950_HEAD_PARAMS
     const auto c_rsrc = __builtin_amdgcn_make_buffer_rsrc((char*)p.C + (int64_t)m0 * p.c_rs * OS, 0, (int)((unsigned)(rows - 1) * row_bytes + (unsigned)p.N * OS), 0x00020000);
     const bool whole_lines = !c_part_lines(p.C, p.c_rs, OS);
     constexpr unsigned kOutside = 0x80000000u; // (C's rows of a tile span less than 2 GiB)
-    const scalar_t set_value = (scalar_t)p.prologue_arg;
+    // The SET constant: integers start from it; floats add it once to the whole sum, as the other kernels do (a constant far above the products would
+    // round every step of the sum at its own size: 100, K = 96, fp32 result, 3.8e-8 from float64 where one addition is 2.2e-8).
+    const scalar_t set_value = (scalar_t)p.prologue_arg, start = IN == IN_I8 ? set_value : scalar_t(0);
     const scalar_t epi_arg = (scalar_t)p.epilogue_arg;
 
     for (int n = 0; n < len; ++n) {
@@ -142,7 +144,7 @@ __global__ void __launch_bounds__(256, 2) gemm_short_k_kernel(ACC950_HEAD_PARAMS
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{set_value, set_value, set_value, set_value};
+            for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{start, start, start, start};
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
             i32x4 bf[TN];
@@ -164,6 +166,8 @@ __global__ void __launch_bounds__(256, 2) gemm_short_k_kernel(ACC950_HEAD_PARAMS
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[i][j][e] = fn(acc[i][j][e]);
         };
+        if constexpr (IN != IN_I8)
+            if (set_value != scalar_t(0)) each([&](scalar_t v) { return v + set_value; });
         if (p.epilogue == EPI_RELU) each([](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); });
         else if (p.epilogue == EPI_SCALE) each([&](scalar_t v) { return wrap_mul(v, epi_arg); });
 

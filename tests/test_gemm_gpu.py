@@ -1598,6 +1598,42 @@ def test_short_k_kernel(in_type, out_type, a_layout, b_layout):
                     assert (np.abs(ora.widen(got[:, :N], out_type).astype(np.float64) - want[z]) <= eps).all()
 
 
+@pytest.mark.parametrize("in_type,out_type", [("f16", "f32"), ("bf16", "f32"), ("f16", "f16"), ("bf16", "bf16"), ("i8", "i32"), ("i8", "i16"), ("i8", "i8")])
+@pytest.mark.parametrize("epilogue", [ora.EPI_NONE, ora.EPI_RELU, ora.EPI_SCALE])
+def test_short_k_kernel_with_a_set_constant(in_type, out_type, epilogue):
+    """A constant is added once, to the whole sum, whatever its size: integers bit for bit; an fp32 result with a constant of 1000 is off by the sum's own roundings
+    (K of 2^-24 of the products' absolute sum) and one rounding of the total, 2^-24 of it (a scale one more)."""
+    import torch
+    import accera_amd as acc
+    from accera_amd import _lib
+    es = 1 if in_type == "i8" else 2
+    for steps, const in ((1, 1000.0), (2, 2.0), (3, 1000.0), (4, 1000.0)):
+        M, N, K = 80, 528, steps * 64 // es
+        rng = np.random.default_rng(steps)
+        A, B = make_input(rng, (M, K), in_type, "normal"), make_input(rng, (K, N), in_type, "normal")
+        dA, dB, dC = to_device(A, in_type), to_device(B, in_type), to_device(np.full((M, N), 3, ora.NP_STORAGE[out_type]), out_type)
+        acc.GemmCall(dA, dB, dC, prologue=_lib.PROLOGUE_SET, prologue_arg=const, epilogue=epilogue, epilogue_arg=3.0, variant=_lib.VARIANT_SHORT_K, k_splits=1)()
+        torch.cuda.synchronize()
+        got = to_host(dC, out_type)
+        a, b = (ora.widen(x, in_type).astype(np.float64) for x in (A, B))
+        want = a @ b + const
+        want = np.maximum(want, 0) if epilogue == ora.EPI_RELU else want * 3 if epilogue == ora.EPI_SCALE else want
+        if in_type == "i8":
+            assert (got == want.astype(np.int64).astype(ora.NP_STORAGE[out_type])).all()
+            continue
+        err, f = np.abs(ora.widen(got, out_type).astype(np.float64) - want), 3 if epilogue == ora.EPI_SCALE else 1
+        half = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8, "f32": 0}[out_type] * np.abs(want)
+        roundings = (2 if epilogue == ora.EPI_SCALE else 1) * 2.0 ** -24 * np.abs(want)
+        assert (err <= half + roundings + f * K * 2.0 ** -24 * (np.abs(a) @ np.abs(b))).all()
+        if out_type == "f32" and const > 100:
+            # one rounding of the total (a scale's of the result beside it) is an error spread evenly over half a unit either way: unit / sqrt(12) in the 2-norm; the
+            # sum's own are a hundredth of that; a tenth more for 42000 samples.  (Three or four steps at the constant's size: 1.7 and 2 times as much.)
+            unit = lambda x: np.spacing(x.astype(np.float32)).astype(np.float64)
+            total = a @ b + const
+            limit = np.sqrt(((f * unit(total)) ** 2 + (unit(want) ** 2 if epilogue == ora.EPI_SCALE else 0)).mean() / 12) * 1.1
+            assert np.sqrt((err ** 2).mean()) <= limit, (steps, np.sqrt((err ** 2).mean()) / limit)
+
+
 def test_short_k_problems_run_on_the_short_k_kernel():
     """The automatic choice on both sides of its lines, against the float64 product."""
     import torch
