@@ -15,7 +15,8 @@ the accumulator file for anything of its own in between (copies of vector regist
 not today -- the kernels ask for all 256 vector registers and the allocator prefers them -- and the check keeps it so.
 
 And the register-staged edge kernels: a CU holds four workgroups of the 64 x 64 tiles, which is 128 vector registers each and
-no scratch; the 128 x 128 ones (two) use no scratch; the 256 x 256 ones spill 68 to 76 bytes per lane, and not more.
+no scratch; the 128 x 128 ones (two) use no scratch; the 256 x 256 ones none for 16-bit inputs and up to 20 bytes per lane for int8.  The other
+32x32-shape kernels: no scratch for 16-bit and fp32 inputs, up to 76 bytes for int8.
 
     python3 check_resources.py <remarks .txt | assembly .s> [...]
 """
@@ -42,8 +43,11 @@ def kernels(text):
 
 
 # register-staged edge kernels: (edge length of the tile) -> most vector registers, most bytes of scratch per lane
-_STAGED = re.compile(r"gemm_mfma_kernelINS_10MfmaConfigILi\d+ELi(\d+)ELi\d+ELi\d+ELi\d+ELb[01]ELb[01]ELb0ELb1E")
-_STAGED_LIMITS = {64: (128, 0), 128: (256, 0), 256: (256, 76)}
+_STAGED = re.compile(r"gemm_mfma_kernelINS_10MfmaConfigILi(\d+)ELi(\d+)ELi\d+ELi\d+ELi\d+ELb[01]ELb[01]ELb0ELb1E")
+_STAGED_LIMITS = {64: (128, 0), 128: (256, 0), 256: (256, 0)}
+_I8 = 2  # (number of the input type in a kernel's name)
+# every other 32x32-shape kernel: most bytes of scratch per lane
+_OTHERS = re.compile(r"gemm_mfma_kernelINS_10MfmaConfigILi(\d+)E")
 
 _AREG = re.compile(r"(?<![\w.$])a(\d+|\[\d+:\d+\])(?!\w)")
 
@@ -82,9 +86,11 @@ def main(paths):
         seen[path] = 0
         for name, f in kernels(open(path, errors="replace").read()):
             scratch = int(f.get("ScratchSize [bytes/lane]", "0"))
-            staged = _STAGED.search(name)
-            if staged:
-                vgprs, most = _STAGED_LIMITS[int(staged.group(1))]
+            staged, other = _STAGED.search(name), _OTHERS.search(name)
+            if staged or other:
+                vgprs, most = _STAGED_LIMITS[int(staged.group(2))] if staged else (256, 0)
+                if other and int(other.group(1)) == _I8:
+                    most = (20 if int(staged.group(2)) == 256 else 0) if staged else 76
                 if int(f.get("VGPRs", "0")) > vgprs or scratch > most:
                     staged_bad.append(f"{name}: {f.get('VGPRs')} vector registers (at most {vgprs}), {scratch} bytes of scratch per lane (at most {most})")
             if "gemm_mfma16w4_kernel" not in name:
@@ -96,7 +102,7 @@ def main(paths):
         print("four-wave GEMM kernels must not use scratch memory, nor the compiler their accumulator registers:\n  " + "\n  ".join(bad), file=sys.stderr)
         return 1
     if staged_bad:
-        print("register-staged edge kernels take more than they may:\n  " + "\n  ".join(staged_bad), file=sys.stderr)
+        print("kernels take more than they may:\n  " + "\n  ".join(staged_bad), file=sys.stderr)
         return 1
     unread = [path for path, n in seen.items() if not n] # (a file in which nothing is found is one that was not understood)
     if unread:

@@ -1065,11 +1065,15 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
     // ---- pass B: ReLU after a SET-0 prologue is the fused hot path, one max per element; every other combination shares one copy
     // without a select: (v + constant) * factor, times 0 where ReLU_NoConditional cuts, max with itself or 0, the SET operand over it -- nine instructions
     // per element.  (With wave-uniform selects over the ops it was about fourteen: 32 x (2048x2048x128) fp16 scaled by alpha 110 us on
-    // 128 x 128 tiles, 82 this way.  Loops of their own per op, two instructions each, are as fast where they fit, but the sums on either side of each
+    // 128 x 128 tiles, 96 this way.  Loops of their own per op, two instructions each, took 82, but the sums on either side of each
     // branch are as many registers again: a kilobyte of scratch per lane on 256 x 256 tiles.)
-    if (p.epilogue == EPI_RELU && !(p.prologue == PRO_SET && p.prologue_arg != 0.f)) {
-        for_each_acc([&](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); });
-    } else if (p.epilogue != EPI_NONE || (p.prologue == PRO_SET && p.prologue_arg != 0.f)) {
+    // The two conditions are worked out without branches and asked one after the other: as a chain of && and || the way of a plain ReLU went through
+    // a dozen jumps into far-off pieces of code and a copy of the sums (fp16 3408x1104x128 to fp32 with a ReLU 6.03 us, 5.80 this way), and the 256 x 256 kernels
+    // had 68 bytes of scratch, which are gone.  The int8 kernels with direct fills do better as one chain: 56 to 76 bytes there, 150 to 280 with two tests.
+    const bool set_constant = (p.prologue == PRO_SET) & (p.prologue_arg != 0.f);
+    const bool plain_relu = (p.epilogue == EPI_RELU) & !set_constant, other_ops = ((p.epilogue != EPI_NONE) | set_constant) & !plain_relu;
+    auto relu_pass = [&]() __attribute__((always_inline)) { for_each_acc([&](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); }); };
+    auto ops_pass = [&]() __attribute__((always_inline)) {
         const scalar_t set_value = p.prologue == PRO_SET ? (scalar_t)p.prologue_arg : scalar_t(0);
         const scalar_t factor = p.epilogue == EPI_SCALE ? (scalar_t)p.epilogue_arg : scalar_t(1); // (x 1 is exact)
         [[maybe_unused]] const scalar_t cut = scalar_t(p.epilogue == EPI_RELU_NOCOND ? 0 : 1);
@@ -1083,6 +1087,13 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
             else v = __builtin_fmaxf(v, lo);
             return __builtin_bit_cast(scalar_t, (__builtin_bit_cast(unsigned, v) & keep) | put);
         });
+    };
+    if constexpr (IN == IN_I8 && !EDGE) {
+        if (plain_relu) relu_pass();
+        else if (other_ops) ops_pass();
+    } else {
+        if (plain_relu) relu_pass();
+        if (other_ops) ops_pass();
     }
     };
 
@@ -1168,7 +1179,7 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
     };
     auto store_all = [&](auto relu_tag) __attribute__((always_inline)) {
         auto fin = [&](scalar_t v) { return decltype(relu_tag)::value ? (v > scalar_t(0) ? v : scalar_t(0)) : v; };
-        const unsigned os = p.out_type == T_I8 ? 1 : (p.out_type == T_F32 || p.out_type == T_I32) ? 4 : 2;
+        const unsigned os = IN == IN_I8 ? (p.out_type == T_I32 ? 4 : p.out_type == T_I16 ? 2 : 1) : p.out_type == T_F32 ? 4 : 2; // (each input type's own results: one or two selects)
         // (whole 16-byte pieces of rows: rows 16 bytes apart, and a tile -- a moved last one may start at any column when B is K-contiguous -- on a 16-byte boundary)
         const bool staged = CAN_STAGE && (p.c_rs * os) % 16 == 0 && ((size_t)p.C & 15) == 0 && ((unsigned)n0 * os) % 16 == 0;
         // Rows of C that do not start on 64-byte boundaries have a copy of the stores of their own, out of the way of the others (with a branch at every

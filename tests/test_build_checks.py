@@ -48,7 +48,7 @@ def _staged(edge, any_alignment=True):
 
 
 @pytest.mark.parametrize("edge,vgprs,scratch,fails", [(64, 128, 0, False), (64, 132, 0, True), (64, 128, 8, True), (128, 222, 0, False), (128, 222, 16, True),
-                                                      (256, 256, 68, False), (256, 254, 132, True)])
+                                                      (256, 256, 20, False), (256, 254, 68, True)])
 def test_registers_and_scratch_of_the_register_staged_kernels(edge, vgprs, scratch, fails, tmp_path, capsys):
     """A CU holds four workgroups of the 64 x 64 tiles (the kernel choice counts on it), and none of these kernels may spill
     more than they do."""
@@ -58,3 +58,19 @@ def test_registers_and_scratch_of_the_register_staged_kernels(edge, vgprs, scrat
     path.write_text(_remarks(form, [(W4, 0)]) + own)
     assert check.main([str(path)]) == int(fails)
     assert not fails or f"{vgprs} vector registers" in capsys.readouterr().err
+
+
+@pytest.mark.parametrize("name,scratch,fails", [
+    # 32x32-shape kernels with direct fills: fp16, int8
+    (_staged(256).replace("ELb0ELb1ELi128ELi2E", "ELb1ELb0ELi64ELi4E").replace("ConfigILi2E", "ConfigILi0E"), 0, False),
+    (_staged(256).replace("ELb0ELb1ELi128ELi2E", "ELb1ELb0ELi64ELi4E").replace("ConfigILi2E", "ConfigILi0E"), 68, True),
+    (_staged(256).replace("ELb0ELb1ELi128ELi2E", "ELb1ELb0ELi64ELi4E"), 76, False),
+    (_staged(256).replace("ELb0ELb1ELi128ELi2E", "ELb1ELb0ELi64ELi4E"), 276, True),
+    (_staged(256).replace("ConfigILi2E", "ConfigILi1E"), 20, True),
+])
+def test_scratch_of_the_other_kernels(name, scratch, fails, tmp_path, capsys):
+    check, path = _check(), tmp_path / "unit.resources.txt"
+    form = "remark: ./gemm_mfma.h:512:0: {}"
+    path.write_text(_remarks(form, [(W4, 0), (name, scratch)]))
+    assert check.main([str(path)]) == int(fails)
+    assert not fails or f"{scratch} bytes of scratch" in capsys.readouterr().err
