@@ -18,6 +18,8 @@ And the register-staged edge kernels: a CU holds four workgroups of the 64 x 64 
 no scratch; the 128 x 128 ones (two) use no scratch; the 256 x 256 ones none for 16-bit inputs and up to 20 bytes per lane for int8.  The other
 32x32-shape kernels: no scratch for 16-bit and fp32 inputs, up to 76 bytes for int8.
 
+And the short-K kernels: two workgroups to a CU, which is 256 vector registers each, and no scratch.
+
     python3 check_resources.py <remarks .txt | assembly .s> [...]
 """
 import re
@@ -46,8 +48,9 @@ def kernels(text):
 _STAGED = re.compile(r"gemm_mfma_kernelINS_10MfmaConfigILi(\d+)ELi(\d+)ELi\d+ELi\d+ELi\d+ELb[01]ELb[01]ELb0ELb1E")
 _STAGED_LIMITS = {64: (128, 0), 128: (256, 0), 256: (256, 0)}
 _I8 = 2  # (number of the input type in a kernel's name)
-# every other 32x32-shape kernel: most bytes of scratch per lane
+# every other 32x32-shape kernel, and the short-K kernels: most bytes of scratch per lane
 _OTHERS = re.compile(r"gemm_mfma_kernelINS_10MfmaConfigILi(\d+)E")
+_SHORT_K = "gemm_short_k_kernel"
 
 _AREG = re.compile(r"(?<![\w.$])a(\d+|\[\d+:\d+\])(?!\w)")
 
@@ -87,12 +90,14 @@ def main(paths):
         for name, f in kernels(open(path, errors="replace").read()):
             scratch = int(f.get("ScratchSize [bytes/lane]", "0"))
             staged, other = _STAGED.search(name), _OTHERS.search(name)
-            if staged or other:
+            if staged or other or _SHORT_K in name:
                 vgprs, most = _STAGED_LIMITS[int(staged.group(2))] if staged else (256, 0)
                 if other and int(other.group(1)) == _I8:
                     most = (20 if int(staged.group(2)) == 256 else 0) if staged else 76
                 if int(f.get("VGPRs", "0")) > vgprs or scratch > most:
                     staged_bad.append(f"{name}: {f.get('VGPRs')} vector registers (at most {vgprs}), {scratch} bytes of scratch per lane (at most {most})")
+            if _SHORT_K in name:
+                seen[path] += 1
             if "gemm_mfma16w4_kernel" not in name:
                 continue
             seen[path] += 1
@@ -106,7 +111,7 @@ def main(paths):
         return 1
     unread = [path for path, n in seen.items() if not n] # (a file in which nothing is found is one that was not understood)
     if unread:
-        print("no four-wave GEMM kernel found in " + ", ".join(unread), file=sys.stderr)
+        print("no four-wave or short-K GEMM kernel found in " + ", ".join(unread), file=sys.stderr)
         return 1
     return 0
 

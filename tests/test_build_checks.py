@@ -60,7 +60,11 @@ def test_registers_and_scratch_of_the_register_staged_kernels(edge, vgprs, scrat
     assert not fails or f"{vgprs} vector registers" in capsys.readouterr().err
 
 
+SHORT_K = "_ZN6acc95019gemm_short_k_kernelINS_12ShortKConfigILi0ELb1ELb1ELi4ELi4EEEEEvPKv"
+
+
 @pytest.mark.parametrize("name,scratch,fails", [
+    (SHORT_K, 0, False), (SHORT_K, 4, True),
     # 32x32-shape kernels with direct fills: fp16, int8
     (_staged(256).replace("ELb0ELb1ELi128ELi2E", "ELb1ELb0ELi64ELi4E").replace("ConfigILi2E", "ConfigILi0E"), 0, False),
     (_staged(256).replace("ELb0ELb1ELi128ELi2E", "ELb1ELb0ELi64ELi4E").replace("ConfigILi2E", "ConfigILi0E"), 68, True),
@@ -74,3 +78,5 @@ def test_scratch_of_the_other_kernels(name, scratch, fails, tmp_path, capsys):
     path.write_text(_remarks(form, [(W4, 0), (name, scratch)]))
     assert check.main([str(path)]) == int(fails)
     assert not fails or f"{scratch} bytes of scratch" in capsys.readouterr().err
+    path.write_text(_remarks(form, [(SHORT_K, 0)]))
+    assert check.main([str(path)]) == 0    # (a unit of short-K kernels is understood)
