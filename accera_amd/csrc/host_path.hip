@@ -15,15 +15,12 @@
 //   * device to host: the same ring the other way round -- the copies of the first slots are queued at once, each slot is
 //     copied out to the caller's array when its event has passed and then queued again for a later piece.
 #include "host_path.h"
+#include "copy_pool.h"
 
 #include <algorithm>
 #include <atomic>
-#include <condition_variable>
 #include <exception>
-#include <cstring>
-#include <immintrin.h>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 namespace acc950 {
@@ -34,125 +31,6 @@ namespace {
 // three slots of 8 MB, 2.65 with four of 4, 2.95 with eight of 2.)
 constexpr size_t kSlotBytes = (size_t)8 << 20;
 constexpr int kSlots = 3;
-constexpr int kCopyThreads = 6;               // workers that move bytes between the caller's arrays and the staging slots
-constexpr size_t kParallelFrom = (size_t)256 << 10; // smaller pieces are copied by the calling thread alone
-
-// ---- copies on the host ------------------------------------------------------------------------
-// Stores that go past the caches: neither side of these copies is read again by this program soon, and an ordinary store would
-// first fetch the line it is about to overwrite, half as much memory traffic again.
-__attribute__((target("avx2"))) void stream_copy(char* dst, const char* src, size_t bytes)
-{
-    const size_t head = (32 - ((size_t)dst & 31)) & 31;
-    if (bytes < 4096 + head) { std::memcpy(dst, src, bytes); return; }
-    std::memcpy(dst, src, head);
-    dst += head; src += head; bytes -= head;
-    for (; bytes >= 128; bytes -= 128, dst += 128, src += 128) {
-        const __m256i a = _mm256_loadu_si256((const __m256i*)src), b = _mm256_loadu_si256((const __m256i*)(src + 32)),
-                      c = _mm256_loadu_si256((const __m256i*)(src + 64)), d = _mm256_loadu_si256((const __m256i*)(src + 96));
-        _mm256_stream_si256((__m256i*)dst, a);
-        _mm256_stream_si256((__m256i*)(dst + 32), b);
-        _mm256_stream_si256((__m256i*)(dst + 64), c);
-        _mm256_stream_si256((__m256i*)(dst + 96), d);
-    }
-    std::memcpy(dst, src, bytes);
-    _mm_sfence();
-}
-void copy_bytes(char* dst, const char* src, size_t bytes)
-{
-    static const bool wide = __builtin_cpu_supports("avx2");
-    if (wide) stream_copy(dst, src, bytes);
-    else std::memcpy(dst, src, bytes);
-}
-
-// A fixed set of threads, started at the first large copy.  One copy at a time is dealt out (callers take turns);
-// the calling thread takes a share itself.  While a large call is under way (Busy) the threads wait for the next copy without
-// sleeping: a call is a dozen or two copies of 1 to 8 MB, 15 to 100 us each, and waking six sleeping threads takes half as long again.
-// The threads live until the process ends, asleep between calls.
-class CopyPool {
-public:
-    class Busy {
-    public:
-        Busy(CopyPool& pool, bool large) : pool_(large ? &pool : nullptr) { if (pool_) pool_->busy(1); }
-        ~Busy() { if (pool_) pool_->busy(-1); }
-        Busy(const Busy&) = delete;
-        Busy& operator=(const Busy&) = delete;
-
-    private:
-        CopyPool* pool_;
-    };
-    void copy(char* dst, const char* src, size_t bytes)
-    {
-        if (bytes < kParallelFrom) { std::memcpy(dst, src, bytes); return; }
-        std::lock_guard<std::mutex> turn(turn_);
-        start_workers();
-        Busy awake(*this, true);
-        Job job;
-        job.dst = dst; job.src = src; job.bytes = bytes;
-        job.per = ((bytes + kCopyThreads) / (kCopyThreads + 1) + 4095) & ~(size_t)4095;
-        job.left = (bytes + job.per - 1) / job.per;
-        job_ = &job;
-        ++generation_;
-        work(job); // the caller's share
-        while (job.left) __builtin_ia32_pause();
-        // (a thread that is still looking at the job counts itself in before it does: none is once the count is zero)
-        job_ = nullptr;
-        while (inside_) __builtin_ia32_pause();
-    }
-
-private:
-    struct Job {
-        char* dst;
-        const char* src;
-        size_t bytes, per;
-        std::atomic<size_t> next{0}, left{0};
-    };
-    void start_workers()
-    {
-        if (started_) return;
-        started_ = true;
-        for (int i = 0; i < kCopyThreads; ++i) std::thread([this] { loop(); }).detach();
-    }
-    void busy(int change)
-    {
-        {
-            std::lock_guard<std::mutex> lock(m_);
-            busy_ += change;
-        }
-        if (change > 0) wake_.notify_all();
-    }
-    // takes pieces of the job until none is left
-    static void work(Job& job)
-    {
-        for (;;) {
-            const size_t off = job.next++ * job.per;
-            if (off >= job.bytes) return;
-            copy_bytes(job.dst + off, job.src + off, job.bytes - off < job.per ? job.bytes - off : job.per);
-            --job.left;
-        }
-    }
-    void loop()
-    {
-        unsigned long long seen = 0;
-        for (;;) {
-            if (generation_ == seen) {
-                if (busy_) { __builtin_ia32_pause(); continue; }
-                std::unique_lock<std::mutex> lock(m_);
-                wake_.wait(lock, [&] { return busy_ != 0; });
-                continue;
-            }
-            seen = generation_;
-            ++inside_;
-            if (Job* job = job_) work(*job);
-            --inside_;
-        }
-    }
-    std::mutex turn_, m_;
-    std::condition_variable wake_;
-    bool started_ = false;
-    std::atomic<Job*> job_{nullptr};
-    std::atomic<unsigned long long> generation_{0};
-    std::atomic<int> inside_{0}, busy_{0};
-};
 
 CopyPool& copy_pool()
 {
@@ -278,7 +156,7 @@ hipError_t upload(HostContext& c, void* dev, const void* host, size_t bytes)
         // (the slot's last copy to the device -- of this call or an earlier one -- has read it)
         hipError_t e = hipEventSynchronize(c.event[s]);
         if (e != hipSuccess) return e;
-        copy_pool().copy(c.slot[s], src + off, n);
+        copy_pool().copy(c.slot[s], src + off, n, true);
         e = hipMemcpyAsync((char*)dev + off, c.slot[s], n, hipMemcpyHostToDevice, c.stream);
         if (e == hipSuccess) e = hipEventRecord(c.event[s], c.stream);
         if (e != hipSuccess) return e;
@@ -307,7 +185,7 @@ hipError_t download(HostContext& c, void* host, const void* dev, size_t bytes)
         const int s = (int)(piece % kSlots);
         hipError_t e = hipEventSynchronize(c.event[s]);
         if (e != hipSuccess) return e;
-        copy_pool().copy(dst + off, c.slot[s], n);
+        copy_pool().copy(dst + off, c.slot[s], n, true);
         if (piece + kSlots < pieces)
             if (e = queue(piece + kSlots); e != hipSuccess) return e;
     }
@@ -359,7 +237,7 @@ hipError_t run_parts(HostContext& c, const HostOperands& h, const std::vector<Ho
             }
             if (ready) {
                 const Piece& p = back[drained];
-                copy_pool().copy(p.host, c.back_slot[drained % kSlots], p.bytes);
+                copy_pool().copy(p.host, c.back_slot[drained % kSlots], p.bytes, true);
                 ++drained;
             }
         }
@@ -370,7 +248,7 @@ hipError_t run_parts(HostContext& c, const HostOperands& h, const std::vector<Ho
             if ((e = passed(c.event[s], &free_slot)) != hipSuccess) return e;
             // (neither ring has a slot ready: every slot of the way in is on the bus, the oldest is next)
             if (!free_slot && (e = hipEventSynchronize(c.event[s])) != hipSuccess) return e;
-            copy_pool().copy(c.slot[s], p.host, p.bytes);
+            copy_pool().copy(c.slot[s], p.host, p.bytes, true);
             if ((e = hipMemcpyAsync(p.dev, c.slot[s], p.bytes, hipMemcpyHostToDevice, c.stream)) != hipSuccess) return e;
             if ((e = hipEventRecord(c.event[s], c.stream)) != hipSuccess) return e;
             ++sent;
