@@ -31,6 +31,11 @@ namespace {
 // three slots of 8 MB, 2.65 with four of 4, 2.95 with eight of 2.)
 constexpr size_t kSlotBytes = (size_t)8 << 20;
 constexpr int kSlots = 3;
+// A result of up to this size -- half of the last-level cache it was measured with, 32 MB -- is stored through the caches, where the caller, who reads it next,
+// finds it.  (The call and then C.sum(), us, stores past the caches / through them: fp16 to fp32 1024^3, 4 MB, 483 to 500 / 460 to 465, 1024x2048x1024, 8 MB,
+// 792 / 745, 2048x2048x1024, 16 MB, 1281 to 1325 / 1195 to 1270; 4096x2048x512, 32 MB, 2155 / 2238 and on another day 2248 / 2073, 4096x4096x512, 64 MB, 4157 / 4124;
+// the call alone 311 / 313, 469 / 475, 670 / 678, 937 / 962, 1641 / 1667.)
+constexpr size_t kCachedResult = (size_t)16 << 20;
 
 CopyPool& copy_pool()
 {
@@ -185,7 +190,7 @@ hipError_t download(HostContext& c, void* host, const void* dev, size_t bytes)
         const int s = (int)(piece % kSlots);
         hipError_t e = hipEventSynchronize(c.event[s]);
         if (e != hipSuccess) return e;
-        copy_pool().copy(dst + off, c.slot[s], n, true);
+        copy_pool().copy(dst + off, c.slot[s], n, bytes > kCachedResult);
         if (piece + kSlots < pieces)
             if (e = queue(piece + kSlots); e != hipSuccess) return e;
     }
@@ -237,7 +242,7 @@ hipError_t run_parts(HostContext& c, const HostOperands& h, const std::vector<Ho
             }
             if (ready) {
                 const Piece& p = back[drained];
-                copy_pool().copy(p.host, c.back_slot[drained % kSlots], p.bytes, true);
+                copy_pool().copy(p.host, c.back_slot[drained % kSlots], p.bytes, h.c_bytes > kCachedResult);
                 ++drained;
             }
         }
