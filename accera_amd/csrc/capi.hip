@@ -1059,10 +1059,39 @@ struct HostPlan {
     int rows(size_t part, int M) const { return (part + 1 < first_row.size() ? first_row[part + 1] : M) - first_row[part]; }
 };
 
+// Microseconds of a call on host arrays in parts of blocks of 256 rows, the remainder with the last one: B and the rows of A come in over the bus one after
+// the other, a part is computed when its rows are there and the part before is done, and its rows of C go back when they are computed and the part before is back.
+// The kernel counts by its rounds of tiles over the chip: a part of few tiles takes as long as one that fills it.
+double host_parts_us(const GemmArgs& g, const Choice& whole, const HostOperands& h, int n)
+{
+    const double bus = 48e3, per_part = 5; // bytes per us and direction, both in use; launches and copies queued
+    const double rate = g.in_type == T_F32 ? 0.54e6 : g.in_type == T_I8 ? 8.5e6 : 4.3e6; // operations per us and CU
+    int tables = 0;
+    const MfmaVariant* tab = mfma_table(g.in_type, &tables);
+    const auto kernel_us = [&](int64_t rows) {
+        if (whole.variant == ACC950_VARIANT_SHORT_K) return 5 + (double)rows * g.N * elem_size(g.out_type) / 4.5e6;
+        const MfmaVariant& v = tab[whole.variant];
+        const int64_t tiles = (rows + v.bm - 1) / v.bm * ((g.N + v.bn - 1) / v.bn);
+        return 5 + (double)((tiles + kComputeUnits - 1) / kComputeUnits) * 2.0 * v.bm * v.bn * g.K / rate;
+    };
+    const int blocks = g.M / 256;
+    double in = (double)h.b_bytes / bus, computed = 0, back = 0;
+    for (int i = 0; i < n; ++i) {
+        const int64_t r0 = n == 1 ? 0 : 256 * ((int64_t)blocks * i / n), r1 = i + 1 == n ? g.M : 256 * ((int64_t)blocks * (i + 1) / n);
+        in += (double)h.a_bytes * (double)(r1 - r0) / g.M / bus;
+        computed = std::max(in, computed) + kernel_us(r1 - r0);
+        back = std::max(computed, back) + (double)h.c_bytes * (double)(r1 - r0) / g.M / bus;
+    }
+    return back + (n > 1 ? per_part * n : 0);
+}
+
 // A large product goes in parts of whole rows of a row-major A and C, so that the first rows of C travel back while later rows of A travel
 // in: with the kernel that the whole product would run on, unsplit, so that every element is summed as it would be in one piece
 // (whole rows of 256-row tiles, the remainder with the last part); at least 4 MB of A and C to a part, eight parts at most, from 16 MB on (1024^3 fp16 with an fp32
-// result, 6 MB, 320 us in one piece, 350 in two).
+// result, 6 MB, 320 us in one piece, 350 in two); as many as host_parts_us() has done soonest, if that
+// is soon enough.  (us in one piece / eight parts, or as many as there are blocks / so, fp32 4096^3 5182 / 6674 / 4239 in two, 1500x3000x2000 1568 / 1571 / 1271 in two, 1024x8192x8192
+// 7829 / 7834 / 7164 in two, fp16 2048^3 738 / 615 / 621 in four, with an fp32 result 4096^3 2969 / 2466 in eight, int8 1024x16384x1024, all of whose way is B's and C's,
+// 1894 / 1935 / 1894; 46 problems of 512 to 8192 rows: 0.91 of one piece on average, none slower, 1 % off the best number of parts.)
 // Not where a part's rows of C lie over bytes of A that a later part has yet to read (A and C as shifted views of one array): in one piece all of A is
 // read before anything is written.  (C over B, which is all read first, and C over its own part's or earlier rows of A may stay.)
 bool plan_host_parts_of(const acc950_gemm_call& c, const HostOperands& h, HostPlan* plan)
@@ -1070,8 +1099,8 @@ bool plan_host_parts_of(const acc950_gemm_call& c, const HostOperands& h, HostPl
     const int M = (int)c.M;
     const size_t part_bytes = (size_t)4 << 20, bytes = h.a_bytes + h.c_bytes;
     if (c.batch != 1 || h.send_c || c.c_col_stride != 1 || c.a_col_stride != 1 || c.a_row_stride < c.K || c.K < 1 || M < 512 || bytes < 4 * part_bytes) return false;
-    const int blocks = M / 256, n = (int)std::min<size_t>(std::min<size_t>(8, bytes / part_bytes), (size_t)blocks);
-    if (n < 2) return false;
+    const int blocks = M / 256, most = (int)std::min<size_t>(std::min<size_t>(8, bytes / part_bytes), (size_t)blocks);
+    if (most < 2) return false;
     // (addresses of the device copies do not matter beyond their alignment, which is an allocation's)
     void* const at = (void*)(uintptr_t)4096;
     Problem pb;
@@ -1079,6 +1108,14 @@ bool plan_host_parts_of(const acc950_gemm_call& c, const HostOperands& h, HostPl
     int tables = 0;
     mfma_table((int)c.in_type, &tables);
     if (plan->whole.variant != ACC950_VARIANT_SHORT_K && (plan->whole.variant < 0 || plan->whole.variant >= tables)) return false;
+    // (parts of as many blocks each, or two or four; a fiftieth at least)
+    int n = 1;
+    double soonest = 0.98 * host_parts_us(pb.g, plan->whole, h, 1);
+    for (int parts = 2; parts <= most; ++parts) {
+        if (blocks % parts && parts != 2 && parts != 4) continue;
+        if (const double us = host_parts_us(pb.g, plan->whole, h, parts); us < soonest) { n = parts; soonest = us; }
+    }
+    if (n < 2) return false;
     for (int i = 0; i < n; ++i) plan->first_row.push_back(256 * (int)((int64_t)blocks * i / n));
     const size_t a_row = (size_t)c.a_row_stride * elem_size((int)c.in_type), c_row = (size_t)c.c_row_stride * elem_size((int)c.out_type);
     for (size_t i = 0; i < plan->first_row.size(); ++i) {

@@ -1664,10 +1664,13 @@ def _host_parts(in_id, out_id, M, N, K, a, a_rs, b, b_strides, c):
 
 @pytest.mark.parametrize("in_type,out_type,M,N,K,b_layout,pad,parts", [
     ("f16", "f32", 2048, 2048, 512, "row", 0, 4),     # four parts of 512 rows
-    ("bf16", "bf16", 1111, 8192, 512, "col", 0, 4),   # a last part with the remainder
-    ("i8", "i32", 1536, 3000, 333, "row", 0, 4),      # nothing aligned
+    ("bf16", "bf16", 1111, 8192, 512, "col", 0, 1),   # little of A to overlap with C: one piece
+    ("bf16", "bf16", 2111, 2104, 2048, "col", 0, 4),  # a last part with the remainder
+    ("i8", "i32", 1536, 3000, 333, "row", 0, 1),
+    ("i8", "i32", 3704, 1000, 4063, "row", 0, 7),     # nothing aligned
     ("f32", "f32", 1024, 4096, 512, "row", 8, 4),     # rows of A further apart than they are long
-    ("f16", "f16", 4100, 3000, 128, "col", 0, 6),     # pieces of C that are no multiple of anything
+    ("f16", "f16", 4100, 3000, 128, "col", 0, 1),
+    ("f16", "f16", 4100, 2000, 1500, "col", 0, 4),    # pieces of C that are no multiple of anything
     ("f16", "f16", 511, 16384, 256, "row", 0, 1),     # too few rows: one piece
 ])
 def test_host_call_in_parts_gives_the_bits_of_the_device_call(in_type, out_type, M, N, K, b_layout, pad, parts):
