@@ -474,3 +474,31 @@ def test_host_calls_go_in_as_many_parts_as_pay(tin, tout, M, N, K, parts):
     """Parts that leave the chip idle, or that have nothing to overlap, are not made."""
     ids = {"f16": _lib.F16, "f32": _lib.F32, "i8": _lib.I8, "i32": _lib.I32}
     assert _host_parts(ids[tin], ids[tout], M, N, K) == parts
+
+
+def _choice(in_type, out_type, M, N, K, a_col=False, b_col=False, epilogue=_lib.EPILOGUE_RELU, epilogue_arg=0.0, batch=1, prologue_arg=0.0):
+    """(variant, K slices) the library takes for dense, aligned operands (nothing is launched)."""
+    ids = {"f16": _lib.F16, "bf16": _lib.BF16, "i8": _lib.I8, "f32": _lib.F32, "i32": _lib.I32, "i16": _lib.I16}
+    L, h, v, ks, P = _lib.lib(), ctypes.c_int(-1), ctypes.c_int(), ctypes.c_int(), ctypes.c_void_p
+    many = int(batch > 1)
+    _lib.check(L.acc950_bind(ids[in_type], ids[out_type], batch, M, N, K, P(1 << 40), many * M * K, *((1, M) if a_col else (K, 1)), P(2 << 40), many * K * N, *((1, K) if b_col else (N, 1)),
+                             P(3 << 40), many * M * N, N, 1, _lib.PROLOGUE_SET0, prologue_arg, epilogue, epilogue_arg, _lib.VARIANT_AUTO, 0, None, ctypes.byref(h)))
+    try:
+        _lib.check(L.acc950_bound_choice(h.value, ctypes.byref(v), ctypes.byref(ks)))
+    finally:
+        L.acc950_unbind(h.value)
+    return v.value, ks.value
+
+
+@pytest.mark.parametrize("in_type,out_type,batch,M,N,K,ops,short_k", [
+    ("f16", "f16", 32, 2048, 2048, 128, "scale", True), ("f16", "f16", 1, 8192, 8192, 64, "relu", True), ("bf16", "f32", 1, 6352, 2952, 96, "relu", True), ("bf16", "bf16", 1, 51424, 4096, 128, "relu", True),
+    ("f16", "f16", 1, 50176, 256, 128, "none", False), ("f16", "f16", 1, 69872, 256, 128, "none", True), ("f16", "f16", 1, 67168, 256, 64, "none", True),  # one column tile
+    ("bf16", "f32", 1, 22592, 4864, 128, "relu", False), ("bf16", "f32", 1, 22592, 4864, 128, "scale", True), ("bf16", "f32", 1, 22592, 4864, 96, "relu", True),  # what the four-wave kernel takes too
+    ("bf16", "f32", 80, 992, 1024, 128, "none", True), ("i8", "i32", 1, 10624, 9728, 256, "relu", False), ("i8", "i16", 1, 10624, 9728, 256, "relu", True),
+    ("bf16", "bf16", 1, 15072, 22256, 128, "none", False), ("bf16", "bf16", 1, 2656, 5144, 128, "none", True), ("bf16", "bf16", 1, 15072, 22272, 128, "none", True),  # rows off 128-byte boundaries
+    ("f16", "f32", 1, 19904, 8240, 32, "none", False), ("f16", "f32", 1, 19904, 8256, 32, "none", True), ("f16", "f32", 160, 64, 1136, 96, "relu", True),  # ... on odd multiples of 64 bytes
+])
+def test_where_the_short_k_kernel_is_taken(in_type, out_type, batch, M, N, K, ops, short_k):
+    """Both sides of the lines where another kernel is level or ahead (figures beside the rule)."""
+    epilogue, arg = {"none": (_lib.EPILOGUE_NONE, 0.0), "relu": (_lib.EPILOGUE_RELU, 0.0), "scale": (_lib.EPILOGUE_SCALE, 0.125)}[ops]
+    assert (_choice(in_type, out_type, M, N, K, epilogue=epilogue, epilogue_arg=arg, batch=batch)[0] == _lib.VARIANT_SHORT_K) == short_k
