@@ -600,15 +600,18 @@ int streamed_b_tile(const Problem& pb)
     // 185x3520x4800 with a K-contiguous B 17.9 / 21.9, fp16 194x2496x21504 45.2 / 74.4, 224x4224x5568 28.4 / 34.0; while the
     // chip takes three slices of every tile: 159x46976x1024, 734 tiles, is 32.1 us on the general rule's 256 x 256 ones, 44.9 this way.
     // Of 86 to 128 tiles it takes two, which pays as well -- f16 127x14784x4096 with a K-contiguous B 54.1 us unsplit on 64 x 64 tiles, 42.9 so, bf16 169x6336x6656
-    // 61.5 / 41.7, 213x6016x4416 27.2 / 24.9 --, against a row-major B from slices of more than 2048 of K on (100x11008x4096, 43.1 / 28.7, is left where the tests
-    // hold it); int8 gains more: 155x5568x7296 47.0 / 22.0 in two, 92x9920x7936 40.5 / 26.9 in three, 164x4416x16896 63.7 / 44.7, 214x7808x20608 117 / 65; but
-    // 100x6080x3456, 20 MB, 9.8 / 14.1)
+    // 61.5 / 41.7, 213x6016x4416 27.2 / 24.9 --, against a K-contiguous B from a K of 2048 on (77x15360x1984 22.7 / 24.8), against a row-major one from slices of more
+    // than 2048 of K on (below that line the route checks hold the unsplit tiles; 100x11008x4096 takes 43.1 us there and 28.7 in two slices).  int8 gains
+    // more: 155x5568x7296 47.0 / 22.0 in two, 92x9920x7936 40.5 / 26.9 in three, 164x4416x16896 63.7 / 44.7, 214x7808x20608 117 / 65; but against a K-contiguous B only from a
+    // K of 4500 on (70x13312x3200 17.4 / 19.1, 89x12224x3456 19.4 / 20.3; 100x6080x3456, 20 MB, 9.8 / 14.1).  Of 387 problems, B out of HBM, 0.76 of the general rule's
+    // time on average, the slowest 1.09)
     if (!streamed_b(pb, (int64_t)192 << 20)) {
         if (g.M <= 64 || !streamed_b(pb, (int64_t)32 << 20)) return 0;
         const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+        const bool i8 = g.in_type == T_I8, b_kc = g.b_rs == 1;
         // (int8, a K-contiguous B and a K of no whole 128 bytes, which the four-stage tiles do not take: 181x5440x7616 26.2 / 40.0)
-        if (g.in_type == T_I8 && g.b_rs == 1 && g.K % 128) return 0;
-        const bool two = g.in_type == T_I8 || g.b_rs == 1 || g.K > 4096;
+        if (i8 && b_kc && (g.K % 128 || g.K < 4500)) return 0;
+        const bool two = i8 || (b_kc ? g.K >= 2048 : g.K > 4096);
         return tiles * (two ? 2 : 3) <= kComputeUnits ? 128 : 0;
     }
     // (a tile that holds all rows of A: up to 64 rows the small tiles, up to 128 rows the 128 x 128 tiles, up to 256 the
@@ -839,8 +842,23 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
                     int n = 0;
                     const MfmaVariant& v = mfma_table(pb.g.in_type, &n)[mv];
                     streamed_splits = streamed_b_splits(v, pb, max_split_floats);
-                    // (a B below 192 MB: only with direct fills)
-                    if (!v.direct && !streamed_b(pb, (int64_t)192 << 20)) { mv = -1; streamed_splits = 0; }
+                    // (a B below 192 MB: only with direct fills and in slices -- unsplit f16 121x12800x1536 12.0 us by the general rule, 18.4 on these tiles, 69x14336x1600
+                    // 17.1 / 21.5, int8 249x7680x5120 19.2 / 21.1 --, and for int8 not where the general rule takes such tiles by itself in more slices, 246x4992x9920 32.8 us in
+                    // three, 40.6 in two, nor, against a K-contiguous B below 40 MB, where it takes four slices and more of its own tiles: 124x3584x10112 20.8 / 20.2 out of HBM but
+                    // 14.0 / 15.6 out of the cache)
+                    if (!streamed_b(pb, (int64_t)192 << 20)) {
+                        const int slices = streamed_splits > 1 ? streamed_splits : auto_mfma_splits(v, pb, max_split_floats);
+                        bool keep = v.direct && slices > 1;
+                        if (keep && pb.g.in_type == T_I8) {
+                            const int general = auto_mfma_variant(pb);
+                            if (general >= 0) {
+                                const MfmaVariant& u = mfma_table(pb.g.in_type, &n)[general];
+                                const int its_own = auto_mfma_splits(u, pb, max_split_floats);
+                                keep = u.bm == v.bm && u.bn == v.bn ? its_own <= slices : pb.g.b_rs != 1 || its_own < 4 || streamed_b(pb, (int64_t)40 << 20);
+                            }
+                        }
+                        if (!keep) { mv = -1; streamed_splits = 0; }
+                    }
                 }
                 if (mv >= 0) {
                     int n = 0;

@@ -412,6 +412,12 @@ def test_packed_call_checks_its_numbers():
     ("i8", 155, 5568, 7296, False, "128x128", 2), ("i8", 92, 9920, 7936, True, "128x128", 3), ("i8", 194, 2304, 14720, False, "128x128", 4),
     ("i8", 100, 6080, 3456, True, "64x64", 1),         # a B of 20 MB
     ("i8", 181, 5440, 7616, True, "64x64", 1),         # K of no whole 128 bytes
+    # no slices of these tiles: the general rule's, which read B as often and fill the chip
+    ("f16", 121, 12800, 1536, True, "64x64", 1), ("bf16", 69, 14336, 1600, True, "64x64", 1), ("f16", 105, 13056, 1792, True, "64x64", 1), ("i8", 249, 7680, 5120, True, "64x64", 1),
+    ("bf16", 245, 6720, 4672, True, "128x128", 2),     # (two slices by the general rule's count)
+    ("f16", 86, 13312, 2240, True, "128x128", 2), ("f16", 77, 15360, 1984, True, "64x64", 1), ("i8", 70, 13312, 3200, True, "64x64", 1),  # a K-contiguous B: from a K of 2048, int8 4500 on
+    ("i8", 246, 4992, 9920, False, "128x128", 3),      # the general rule's three slices of these tiles, not two
+    ("i8", 124, 3584, 10112, True, "64x64", 4), ("i8", 124, 3584, 10112, False, "128x128", 5),
 ])
 def test_65_to_256_rows_against_32_to_192_mb(in_type, M, N, K, b_col, tile, slices):
     from accera_amd import tune
