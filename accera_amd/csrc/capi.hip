@@ -685,9 +685,12 @@ bool short_k_pays(const Problem& pb)
 
 // Problems of any alignment with a long K and 30 to 128 tiles of 256 x 256: these tiles fetch half as much per MFMA as the 128 x 128 ones the
 // general rule takes, which unaligned operands pay for dearly, and in as many K slices as the chip holds of them (six at most) they
-// fill it; the sums of the slices need a K of about 3800, int8, with twice as many to a byte, 5000 and fewer tiles (us, 128 x 128 unsplit / so: fp16 1234x5678x4321
+// fill it; the sums of the slices need a K of about 3800, int8, with twice as many to a byte, 5000 and fewer tiles; against a K-contiguous B more where
+// the 128 x 128 tiles are a round over the chip that is nearly full (5300), int8 where they are one round at most (6000).  us, 128 x 128 unsplit / so: fp16 1234x5678x4321
 // 122.9 / 104.9 in two, 3913x893x6825 108 / 86 in four, bf16 5060x941x3879 105 / 75 in three, 703x3293x5909 86 / 62 in six, int8 644x7700x5155 86 / 66; but fp16 2140x1916x3269
-// 54.4 / 59.8, int8 2287x1790x4547 47 / 54, 2576x2645x4099, 121 tiles, 67.7 / 70.5).  Moves *mv to that kernel and returns the slices, or 1.
+// 54.4 / 59.8, int8 2287x1790x4547 47 / 54, 2576x2645x4099, 121 tiles, 67.7 / 70.5, K-contiguous fp16 3296x1088x5026 68.0 / 72.5, 1177x2704x4124 52.9 / 56.8, int8 416x7360x5092
+// 37.7 / 47.9, 5056x640x5080 1.10 times as long.  (399 problems, operands out of HBM: 0.76 on average, the slowest 1.02.)  Moves *mv to that kernel and returns
+// the slices, or 1.
 int staged_large_slices(const Problem& pb, int* mv, size_t max_floats)
 {
     const GemmArgs& g = pb.g;
@@ -695,8 +698,10 @@ int staged_large_slices(const Problem& pb, int* mv, size_t max_floats)
     const MfmaVariant* tab = mfma_table(g.in_type, &n);
     if (!tab[*mv].any || g.in_type == T_F32 || g.batch > 1) return 1;
     const bool i8 = g.in_type == T_I8;
-    const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
-    if (g.K < (i8 ? 5000 : 3800) || tiles < 30 || tiles > (i8 ? 100 : 128) || (double)g.M * g.N < 0.75 * 65536.0 * (double)tiles) return 1;
+    const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256), small = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+    const bool b_kc = g.b_rs == 1;
+    const int least = i8 ? (b_kc && small <= kComputeUnits ? 6000 : 5000) : b_kc && small > 200 && small <= kComputeUnits ? 5300 : 3800;
+    if (g.K < least || tiles < 30 || tiles > (i8 ? 100 : 128) || (double)g.M * g.N < 0.75 * 65536.0 * (double)tiles) return 1;
     const int want = (int)std::min<int64_t>(6, kComputeUnits / tiles);
     if ((size_t)want * (size_t)g.M * (size_t)g.N > ((size_t)1 << 24)) return 1; // 64 MiB of partial sums at most without being asked
     for (int i = 0; i < n; ++i) {

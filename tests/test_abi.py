@@ -432,6 +432,7 @@ def test_65_to_256_rows_against_32_to_192_mb(in_type, M, N, K, b_col, tile, slic
     ("f16", 2600, 2900, 4321, "128x128", 1),      # 132 tiles: no two slices of each
     ("i8", 2576, 2645, 6001, "128x128", 1),
     ("f16", 520, 8001, 4321, "128x128", 1),       # a last row of tiles that is nearly empty
+    ("i8", 5184, 736, 5790, "256x256", 4),
 ])
 def test_large_tiles_in_slices_for_unaligned_problems_with_a_long_k(in_type, M, N, K, tile, slices):
     from accera_amd import tune
@@ -508,3 +509,14 @@ def test_where_the_short_k_kernel_is_taken(in_type, out_type, batch, M, N, K, op
     """Both sides of the lines where another kernel is level or ahead (figures beside the rule)."""
     epilogue, arg = {"none": (_lib.EPILOGUE_NONE, 0.0), "relu": (_lib.EPILOGUE_RELU, 0.0), "scale": (_lib.EPILOGUE_SCALE, 0.125)}[ops]
     assert (_choice(in_type, out_type, M, N, K, epilogue=epilogue, epilogue_arg=arg, batch=batch)[0] == _lib.VARIANT_SHORT_K) == short_k
+
+
+@pytest.mark.parametrize("in_type,M,N,K,tile,slices", [
+    ("f16", 3296, 1088, 5026, "128x128", 1), ("f16", 3296, 1088, 5306, "256x256", 3),   # 234 tiles of 128 x 128: nearly a whole round
+    ("f16", 1520, 1344, 3802, "256x256", 6),                                            # 132 of them
+    ("i8", 5184, 736, 5790, "128x128", 1), ("i8", 5184, 736, 6002, "256x256", 4), ("i8", 644, 7700, 5155, "256x256", 2),
+])
+def test_large_tiles_in_slices_against_a_k_contiguous_b(in_type, M, N, K, tile, slices):
+    """K has to be longer where the 128 x 128 tiles fill the chip in one round."""
+    v, ks = _choice(in_type, "i32" if in_type == "i8" else in_type, M, N, K, b_col=True)
+    assert f"mfma {tile} " in _lib.variant_name(v) and "any-alignment" in _lib.variant_name(v) and ks == slices, (_lib.variant_name(v), ks)
