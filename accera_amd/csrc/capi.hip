@@ -239,7 +239,7 @@ int auto_skinny_variant(const Problem& pb)
 // Partial sums (fp32) and one arrival counter per column block.  One workspace per (device, stream): launches on one
 // stream run one after the other and may share it, launches on different streams may overlap and must not.  A
 // workspace that is missing or too small while its stream is being captured is not made (an allocation would end the
-// capture): the call runs unsplit then, as calls of the same shape did that had needed none.  A
+// capture): the call runs unsplit then, on the kernel the library takes for a call that has none.  A
 // workspace only grows, and an outgrown block stays allocated, because launches queued earlier may still be using
 // it, until acc950_release_workspaces frees everything on an idle device.  The pointers are copied out while the
 // lock is held.
@@ -717,6 +717,7 @@ int staged_large_slices(const Problem& pb, int* mv, size_t max_floats)
 struct Choice {
     int variant;
     int splits;
+    bool own = false; // kernel and slices are the library's choice, for a call that has a workspace
 };
 
 // Few rows of A, a large B (decode shapes with a long K or many columns): the 256-column blocks of the streaming kernel
@@ -774,6 +775,7 @@ bool wide_skinny_blocks_pay(const Problem& pb, int sv_wide, size_t max_floats, s
 int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_split_floats = kMaxSplitFloats, size_t max_counters = ~(size_t)0)
 {
     c->splits = 1;
+    c->own = variant == ACC950_VARIANT_AUTO && k_splits == 0;
     if (variant == ACC950_VARIANT_AUTO) {
         if (k_splits <= 1 && short_k_pays(pb)) { c->variant = ACC950_VARIANT_SHORT_K; return ACC950_OK; }
         const int sv = auto_skinny_variant(pb);
@@ -1049,8 +1051,15 @@ int run(const Problem& pb, const Choice& c, hipStream_t stream, LaunchGeom* geom
                     if (e != hipSuccess) return fail_hip(e, "address of the built-in workspace");
                 } else {
                     e = workspace_for(stream, floats, 0, &ws, &unused);
-                    if (e == hipErrorStreamCaptureUnsupported) split = false; // (under capture, and no workspace yet: unsplit)
-                    else if (e != hipSuccess) return fail_hip(e, "workspace allocation");
+                    if (e == hipErrorStreamCaptureUnsupported) {
+                        // Under capture, and no workspace yet: unsplit.  Tiles that were chosen for their slices need not be the ones then (fp16 1234x5678x4321: 256 x 256 in two
+                        // slices 105 us, unsplit 145 on 115 of 256 CUs, 128 x 128 unsplit 115), so the library chooses again, for a call without a workspace.
+                        split = false;
+                        if (Choice again; c.own && choose(pb, ACC950_VARIANT_AUTO, 0, &again, 0, 0) == ACC950_OK) {
+                            again.own = false;
+                            return run(pb, again, stream, geom, dry_run);
+                        }
+                    } else if (e != hipSuccess) return fail_hip(e, "workspace allocation");
                 }
             }
         }

@@ -172,3 +172,80 @@ def test_a_captured_call_without_a_workspace_runs_unsplit(M, N, K):
             graph.replay()
             torch.cuda.synchronize()
             assert_matches(to_host(dC, "f16"), want, "f16", K)
+
+
+def _captured_kernels(call, stream):
+    """Grids of the kernel nodes of a HIP graph into which call() has been captured on `stream`, and what replays it."""
+    import ctypes
+
+    class Dim3(ctypes.Structure):
+        _fields_ = [("x", ctypes.c_uint32), ("y", ctypes.c_uint32), ("z", ctypes.c_uint32)]
+
+    class KernelNodeParams(ctypes.Structure):  # hipKernelNodeParams
+        _fields_ = [("blockDim", Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("gridDim", Dim3), ("kernelParams", ctypes.c_void_p), ("sharedMemBytes", ctypes.c_uint)]
+
+    with open("/proc/self/maps") as maps:  # (the runtime that is loaded, whichever it is)
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    ok = lambda rc: rc == 0 or pytest.fail(f"HIP error {rc}")
+    s, graph, n = ctypes.c_void_p(stream), ctypes.c_void_p(), ctypes.c_size_t()
+    ok(hip.hipStreamBeginCapture(s, 1))
+    try:
+        call()
+    finally:
+        ok(hip.hipStreamEndCapture(s, ctypes.byref(graph)))
+    ok(hip.hipGraphGetNodes(graph, None, ctypes.byref(n)))
+    nodes = (ctypes.c_void_p * n.value)()
+    ok(hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)))
+    grids = []
+    for node in nodes:
+        kind, params = ctypes.c_int(), KernelNodeParams()
+        ok(hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)))
+        assert kind.value == 0  # (hipGraphNodeTypeKernel: nothing else is recorded)
+        ok(hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)))
+        grids.append([params.gridDim.x, params.gridDim.y, params.gridDim.z])
+    executable = ctypes.c_void_p()
+    ok(hip.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, ctypes.c_size_t(0)))
+
+    def replay():
+        ok(hip.hipGraphLaunch(executable, s))
+        ok(hip.hipStreamSynchronize(s))
+
+    def done():
+        ok(hip.hipGraphExecDestroy(executable))
+        ok(hip.hipGraphDestroy(graph))
+    return grids, replay, done
+
+
+@pytest.mark.parametrize("M,N,K,b_col", [(1234, 5678, 4321, False), (703, 3293, 5909, True), (127, 14784, 4096, True)])
+def test_a_captured_call_without_a_workspace_takes_the_kernel_of_an_unsplit_call(M, N, K, b_col):
+    """Tiles that the library takes for their K slices are not what it runs when there is no workspace for the slices."""
+    import torch
+    from accera_amd import _lib
+    L = _lib.lib()
+    _lib.check(L.acc950_init(0))
+    rng = np.random.default_rng(M)
+    A, B = make_input(rng, (M, K), "f16", "normal"), (make_input(rng, (K, N), "f16", "normal").astype(np.float32) * K ** -0.5).astype(np.float16)
+    dA, dB, dC = to_device(A, "f16"), to_device(np.asfortranarray(B) if b_col else B, "f16"), to_device(np.zeros((M, N), np.float16), "f16")
+    strides = (1, K) if b_col else (N, 1)
+
+    def call(k_splits, stream):
+        _lib.check(L.acc950_gemm_ops(_lib.F16, _lib.F16, M, N, K, dA.data_ptr(), K, 1, dB.data_ptr(), *strides, dC.data_ptr(), N, 1, _lib.PROLOGUE_SET0, 0.0, _lib.EPILOGUE_RELU, 0.0,
+                                     _lib.VARIANT_AUTO, k_splits, stream))
+    torch.cuda.synchronize()
+    current = torch.cuda.current_stream().cuda_stream
+    call(1, current)   # (unsplit, eagerly: loads the kernel's code)
+    torch.cuda.synchronize()
+    want = to_host(dC, "f16").copy()
+    unsplit = _lib.launch_geometry(_lib.F16, _lib.F16, M, N, K, (K, 1), strides, (N, 1), k_splits=1)[0]
+    split = _lib.launch_geometry(_lib.F16, _lib.F16, M, N, K, (K, 1), strides, (N, 1))[0]
+    assert split[2] > 1 and unsplit[2] == 1 and split[0] < unsplit[0]   # (larger tiles, in slices)
+    side = torch.cuda.Stream()
+    before = _lib.allocation_probe()
+    grids, replay, done = _captured_kernels(lambda: call(0, side.cuda_stream), side.cuda_stream)
+    assert grids == [unsplit] and _lib.allocation_probe() == before
+    for _ in range(3):
+        dC.fill_(3)
+        torch.cuda.synchronize()
+        replay()
+        assert np.array_equal(to_host(dC, "f16").view(np.uint16), want.view(np.uint16))
+    done()
