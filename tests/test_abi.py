@@ -418,6 +418,7 @@ def test_packed_call_checks_its_numbers():
     ("f16", 86, 13312, 2240, True, "128x128", 2), ("f16", 77, 15360, 1984, True, "64x64", 1), ("i8", 70, 13312, 3200, True, "64x64", 1),  # a K-contiguous B: from a K of 2048, int8 4500 on
     ("i8", 246, 4992, 9920, False, "128x128", 3),      # the general rule's three slices of these tiles, not two
     ("i8", 124, 3584, 10112, True, "64x64", 4), ("i8", 124, 3584, 10112, False, "128x128", 5),
+    ("i8", 144, 14581, 5122, True, "128x128", 1), ("i8", 191, 13089, 6526, False, "128x128", 1),   # register-staged tiles: the sums of two slices are too much beside B
 ])
 def test_65_to_256_rows_against_32_to_192_mb(in_type, M, N, K, b_col, tile, slices):
     from accera_amd import tune
