@@ -83,7 +83,7 @@ def recorded(in_id, out_id, M, N, K, a_rs, a_cs, b_rs, b_cs, c_rs, c_cs, ops):
 def _variant_by_name(name):
     global _names
     if _names is None:
-        ids = list(range(_lib.num_variants())) + [_lib.VARIANT_SKINNY_BASE + i for i in range(_lib.num_skinny_variants())]
+        ids = list(range(_lib.num_variants())) + [_lib.VARIANT_SKINNY_BASE + i for i in range(_lib.num_skinny_variants())] + [_lib.VARIANT_SHORT_K]
         _names = {_lib.variant_name(v): v for v in ids}
     return _names.get(name)
 

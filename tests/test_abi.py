@@ -387,6 +387,25 @@ def test_recorded_choices_without_asking_the_library(tmp_path, monkeypatch):
         tuned.reset()
 
 
+def test_a_recorded_short_k_kernel_is_found(tmp_path, monkeypatch):
+    """What a sweep saves for the short-K kernel, which it tries like any other, is what the look-ups of both kinds of call find."""
+    from accera_amd import tune, tuned
+    M, N, K = 12544, 1024, 128
+    assert (_lib.VARIANT_SHORT_K, 0) in tune.candidates(_lib.F16, _lib.F16, M, N, K, (K, 1), (N, 1), (N, 1))
+    path = tmp_path / "table.json"
+    row = dict(m=M, n=N, k=K, transA=0, transB=0, alpha=1.0, beta=0.0, type="f16", out_type="f16", variant=_lib.VARIANT_SHORT_K, k_splits=0,
+               kernel=_lib.variant_name(_lib.VARIANT_SHORT_K), time_ms=0.01, TFlops=1.0, correct=True)
+    monkeypatch.setenv("ACCERA_AMD_TUNED", str(path))
+    assert tuned.save([row], str(path)) == 1
+    tuned.reset()
+    try:
+        assert tuned.lookup(_lib.F16, _lib.F16, M, N, K, (K, 1), (N, 1), (N, 1), "lean") == (_lib.VARIANT_SHORT_K, 0)
+        assert tuned.recorded(_lib.F16, _lib.F16, M, N, K, K, 1, N, 1, N, 1, "lean") == (_lib.VARIANT_SHORT_K, 0)
+    finally:
+        monkeypatch.undo()
+        tuned.reset()
+
+
 def test_packed_call_checks_its_numbers():
     import struct
     pack = struct.Struct("19qdqd3q").pack
