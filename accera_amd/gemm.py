@@ -46,9 +46,13 @@ def _problem(A, B, C):
     return (in_type, out_type, batch, M, N, K, *_mat(A, "A"), *_mat(B, "B"), *_mat(C, "C"))
 
 
+# (a raw handle without a stream object around it, a microsecond less per call; torch does not document it, so it may be missing)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _current_stream(C):
     """Raw hipStream_t of the stream that is current on C's device."""
-    return torch._C._cuda_getCurrentRawStream(C.get_device())
+    return _raw_stream(C.get_device()) if _raw_stream else torch.cuda.current_stream(C.device).cuda_stream
 
 
 _pack = struct.Struct("19qdqd3q").pack  # acc950_gemm_call
@@ -130,9 +134,11 @@ def gemm_relu(A, B, C, prologue=_lib.PROLOGUE_SET0, epilogue=_lib.EPILOGUE_RELU,
             variant, k_splits = hit
     if stream is None:
         stream = _current_stream(C)
+    elif isinstance(stream, ctypes.c_void_p):
+        stream = stream.value or 0
     run = _lib.lib().acc950_gemm_packed
     rc = run(_pack(*problem, prologue, prologue_arg, epilogue, epilogue_arg, variant, k_splits, stream))
-    if rc and hit:
+    if rc == _lib.UNSUPPORTED and hit:
         rc = run(_pack(*problem, prologue, prologue_arg, epilogue, epilogue_arg, _lib.VARIANT_AUTO, 0, stream))
     if rc:
         _lib.check(rc)

@@ -540,3 +540,48 @@ def test_large_tiles_in_slices_against_a_k_contiguous_b(in_type, M, N, K, tile, 
     """K has to be longer where the 128 x 128 tiles fill the chip in one round."""
     v, ks = _choice(in_type, "i32" if in_type == "i8" else in_type, M, N, K, b_col=True)
     assert f"mfma {tile} " in _lib.variant_name(v) and "any-alignment" in _lib.variant_name(v) and ks == slices, (_lib.variant_name(v), ks)
+
+
+def test_eager_call_passes_streams_and_falls_back_on_a_refusal_only(monkeypatch):
+    """accera_amd.gemm_relu against a stand-in for the library: the raw stream as an int, a c_void_p or the current one; a recorded kernel that the library
+    refuses makes way for its own choice, a launch that fails does not."""
+    import struct
+    import types
+
+    import torch
+    from accera_amd import gemm, tuned
+
+    class Matrix:  # what the front end asks of a tensor
+        shape, dtype, is_cuda, device = torch.Size((64, 64)), torch.float16, True, "cuda:0"
+        def stride(self): return (64, 1)
+        def dim(self): return 2
+        def data_ptr(self): return 1 << 20
+        def get_device(self): return 0
+
+    calls, codes = [], []
+
+    def packed(call):
+        calls.append(struct.Struct("19qdqd3q").unpack(call)[-3:])   # variant, K slices, stream
+        return codes.pop(0)
+
+    monkeypatch.setattr(gemm._lib, "lib", lambda: types.SimpleNamespace(acc950_gemm_packed=packed, acc950_last_error=lambda: b"stand-in"))
+    monkeypatch.setattr(tuned, "recorded", lambda *a: (7, 2))
+    run = lambda **kw: gemm.gemm_relu(Matrix(), Matrix(), Matrix(), **kw)
+    for stream, raw in ((5, 5), (ctypes.c_void_p(6), 6), (ctypes.c_void_p(None), 0), (0, 0)):
+        codes[:] = [_lib.OK]
+        run(stream=stream)
+        assert calls.pop() == (7, 2, raw) and not calls
+    for way in ((lambda device: 9), None):
+        monkeypatch.setattr(gemm, "_raw_stream", way)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(cuda_stream=9))
+        codes[:] = [_lib.OK]
+        run()
+        assert calls.pop() == (7, 2, 9)
+    codes[:] = [_lib.UNSUPPORTED, _lib.OK]
+    run(stream=5)
+    assert calls == [(7, 2, 5), (_lib.VARIANT_AUTO, 0, 5)]
+    calls.clear()
+    codes[:] = [_lib.HIP_ERROR]
+    with pytest.raises(_lib.Acc950Error):
+        run(stream=5)
+    assert calls == [(7, 2, 5)]
