@@ -22,9 +22,10 @@
 
 namespace acc950 {
 
-// STEPS: k-steps of 64 bytes (1 to 4).  OS: bytes of an element of C.
-template <int IN_, bool A_KC_, bool B_KC_, int STEPS_, int OS_>
+// STEPS: k-steps of 64 bytes (1 to 4).  OS: bytes of an element of C.  CONSTANT: floats, a SET constant other than 0.
+template <int IN_, bool A_KC_, bool B_KC_, int STEPS_, int OS_, bool CONSTANT_>
 struct ShortKConfig {
+    static constexpr bool CONSTANT = CONSTANT_;
     static constexpr int IN = IN_, STEPS = STEPS_, OS = OS_, BM = 64, BN = 256, NT = 256;
     static constexpr bool A_KC = A_KC_, B_KC = B_KC_;
     static constexpr int KB = STEPS_ % 2 == 0 ? 128 : 64; // bytes of K of one staged sub-tile
@@ -127,7 +128,9 @@ __global__ void __launch_bounds__(256, 2) gemm_short_k_kernel(ACC950_HEAD_PARAMS
     const bool whole_lines = !c_part_lines(p.C, p.c_rs, OS);
     constexpr unsigned kOutside = 0x80000000u; // (C's rows of a tile span less than 2 GiB)
     // The SET constant: integers start from it; floats add it once to the whole sum, as the other kernels do (a constant far above the products would
-    // round every step of the sum at its own size: 100, K = 96, fp32 result, 3.8e-8 from float64 where one addition is 2.2e-8).
+    // round every step of the sum at its own size: 100, K = 96, fp32 result, 3.8e-8 from float64 where one addition is 2.2e-8).  In kernels of their own:
+    // a test for it beside those for the ops cost a ReLU without one up to 7 % (us, with / without: fp16 32 x (2048x2048x128) 62.6 / 58.6, 18 x (752x2624x96) 19.4 / 18.0, bf16
+    // 20 x (272x4096x128) 14.0 / 13.5; 0.5 % over 42 problems).
     const scalar_t set_value = (scalar_t)p.prologue_arg, start = IN == IN_I8 ? set_value : scalar_t(0);
     const scalar_t epi_arg = (scalar_t)p.epilogue_arg;
 
@@ -166,8 +169,7 @@ __global__ void __launch_bounds__(256, 2) gemm_short_k_kernel(ACC950_HEAD_PARAMS
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[i][j][e] = fn(acc[i][j][e]);
         };
-        if constexpr (IN != IN_I8)
-            if (set_value != scalar_t(0)) each([&](scalar_t v) { return v + set_value; });
+        if constexpr (Cfg::CONSTANT) each([&](scalar_t v) { return v + set_value; });
         if (p.epilogue == EPI_RELU) each([](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); });
         else if (p.epilogue == EPI_SCALE) each([&](scalar_t v) { return wrap_mul(v, epi_arg); });
 
@@ -241,10 +243,12 @@ inline int short_k_run(int64_t tiles_m, int64_t tiles_n, int64_t batch)
     return best;
 }
 
-template <int IN, bool A_KC, bool B_KC, int STEPS, int OS>
+template <int IN, bool A_KC, bool B_KC, int STEPS, int OS, bool CONSTANT = false>
 hipError_t launch_short_k_steps(const GemmArgs& args, int run, unsigned grid, hipStream_t stream)
 {
-    using Cfg = ShortKConfig<IN, A_KC, B_KC, STEPS, OS>;
+    if constexpr (IN != IN_I8 && !CONSTANT)
+        if (args.prologue_arg != 0.f) return launch_short_k_steps<IN, A_KC, B_KC, STEPS, OS, true>(args, run, grid, stream);
+    using Cfg = ShortKConfig<IN, A_KC, B_KC, STEPS, OS, CONSTANT>;
     auto kern = gemm_short_k_kernel<Cfg>;
     static LdsLimitOnce lds_limit; // per instantiation
     if (hipError_t e = lds_limit.ensure((const void*)kern, Cfg::LDS_BYTES); e != hipSuccess) return e;
