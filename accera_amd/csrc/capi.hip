@@ -650,37 +650,44 @@ int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats
     return plan_split(v, pb, (int)want, &sp, max_floats) ? sp.splits : 1;
 }
 
-// K of one to four whole k-steps and many tiles of C: does the short-K kernel (gemm_short_k.h) pay?  Against the other kernels' choice on 880
-// problems of K = 64 to 256 bytes, 1 to 700 MB of C, every type, layout and ops of this range: with more than three of its 64 x 256 tiles per
-// CU, and these mostly full, it takes 0.72 of the time on average (us, fp16 32 x (2048x2048x128) scaled 85 / 57, 8192x8192x64 39 / 29, bf16 6352x2952x96 with an
-// fp32 result 54 / 28, int8 47 x (128x4816x128) 105 / 29); where rows of C end inside 64 bytes, parts of which the stores of most other kernels send to memory, from one
-// per CU on 0.7; fewer, and a workgroup has nothing to walk along (us, other / this: 5136x384x64 3.0 / 4.4, bf16 4 x (2704x608x96), 516 tiles, with an fp32 result
-// 7.7 / 10.1), and so where tiles stick out by half (195 x (4608x128x32) 58 / 84).
+// K of one to four whole k-steps and many tiles of C: does the short-K kernel (gemm_short_k.h) pay?  Against the other kernels' choice on 3076
+// problems of K = 64 to 256 bytes, 6 to 500 MB of C, every type, layout and ops of this range (two thirds of them with all four k-steps and a 32-bit result): with more
+// than three of its 64 x 256 tiles per CU, and these mostly full, or where rows of C end inside 64 bytes, parts of which the stores of most other kernels send to memory,
+// with more than one, it takes 0.83 of the time on average, as this rule has it (us, fp16 32 x (2048x2048x128) scaled 85 / 57, 8192x8192x64 39 / 29, bf16 6352x2952x96 with an
+// fp32 result 54 / 28, int8 47 x (128x4816x128) 105 / 29, 9376x9800x256 206 / 98); fewer, and a workgroup has nothing to walk along (us, other / this: 5136x384x64 3.0 / 4.4, bf16
+// 4 x (2704x608x96), 516 tiles, with an fp32 result 7.7 / 10.1), and so where tiles stick out by half (195 x (4608x128x32) 58 / 84).  What it leaves are ranges that are slower
+// by it on average, not single problems: a tenth of those it takes are slower by 2 % and more, 1.4 times at most.
 bool short_k_pays(const Problem& pb)
 {
     const GemmArgs& g = pb.g;
     if (!short_k_can_take(pb)) return false;
     const int os = elem_size(g.out_type), k_bytes = g.K * elem_size(g.in_type);
-    const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 255) / 256), batch = g.batch > 1 ? g.batch : 1;
-    const bool part_lines = (g.c_rs * os) % 64 != 0;
-    if ((double)g.M * g.N < 0.6 * 64 * 256 * (double)tiles || tiles * batch <= (part_lines ? 1 : 3) * kComputeUnits) return false;
+    const int64_t rows = (g.M + 63) / 64, cols = (g.N + 255) / 256, tiles = rows * cols, batch = g.batch > 1 ? g.batch : 1;
+    const int64_t row_bytes = g.c_rs * os, c_bytes = (int64_t)g.M * g.N * os;
+    const bool i8 = g.in_type == T_I8, part_lines = row_bytes % 64 != 0;
     // C = A*B or relu(A*B): no op for the other kernels to lose time with
     const bool lean = g.prologue == PRO_SET && g.prologue_arg == 0.f && (g.epilogue == EPI_RELU || g.epilogue == EPI_NONE);
-    // One column tile is nothing to walk along: with all four k-steps only from four row tiles per CU on (f16 50176x256x128, 784 of them, 10.3 / 11.3;
-    // fp32 results of 61232x256x128 and more level).
-    if (g.N <= 256 && k_bytes == 256 && tiles * batch < 4 * kComputeUnits) return false;
-    // All four k-steps of one large problem: what the four-wave kernel takes too.  It is level and ahead by up to a tenth where the result has 32 bits --
-    // 56 problems 0.97 on average, from 0.82 to bf16 7376x20816x128 127 / 148, 22592x4864x128 85.5 / 90.8, int8 10624x9728x256 85.0 / 88.7,
-    // 8192x8192x256 60.8 / 63.5 -- and so with a 16-bit one whose rows do not start on 128-byte boundaries, from 16 tiles per CU on (bf16 15072x22256x128 234 / 263,
-    // 8176x17680x128 103 / 109; fewer, 2656x5144x128 scaled 14.7 / 12.0).  A scale costs it more than it costs here (fp16 29264x560x128 22.4 / 18.7).
-    if (k_bytes == 256 && batch <= 1 && g.M >= 256 && g.N >= 256) {
-        if (os == 4 && (lean || (g.in_type == T_I8 && g.a_cs == 1))) return false;
-        if (os == 2 && lean && (g.c_rs * os) % 128 && tiles > 16 * kComputeUnits) return false;
+    // One problem, lean, of a 16-bit type: where the other kernels do best.  (Parts of lines, one to two tiles per CU: 0.96 on average up to 1024 rows, 1.07 beyond, 74 problems;
+    // two to three 0.97.)
+    const bool plain = batch == 1 && lean && !i8;
+    if ((double)g.M * g.N < 0.6 * 64 * 256 * (double)tiles || tiles * batch <= (!part_lines ? 3 : plain && g.M > 1024 ? 2 : 1) * kComputeUnits) return false;
+    // One column tile is nothing to walk along: with all four k-steps and whole lines only from four row tiles per CU on (f16 50176x256x128, 784 of them, 10.3 / 11.3;
+    // fp32 results of 61232x256x128 and more level; scaled 0.85).
+    if (g.N <= 256 && k_bytes == 256 && lean && row_bytes % 128 == 0 && tiles * batch < 4 * kComputeUnits) return false;
+    // Two column tiles and a few more than two row tiles per CU: the workgroups, which walk both, are one round over the chip and little of a second one (f16
+    // 36240x384x128 9.6 / 13.9; fourteen problems of up to 672 row tiles 1.10 on average, 24 of more 0.84).
+    if (plain && cols == 2 && rows > 2 * kComputeUnits && rows <= 672) return false;
+    // (int8 to int32, all four k-steps, a row-major B: the four-wave kernel is level -- 8192x6144x256 43.2 us, 42.6 here; 8192x8192x256 60.8 / 63.5 -- and keeps them)
+    if (i8 && os == 4 && g.K == 256 && g.a_cs == 1 && g.b_cs == 1 && batch == 1 && g.M >= 256 && g.N >= 256) return false;
+    // A C far beyond the caches: rows on odd multiples of 64 bytes, whose line of 128 bytes between two column tiles is written in halves, cost this kernel more than the
+    // others -- 32-bit results from 256 MB on, whatever the ops, 1.08 on average of 122 problems, 16-bit inputs with no op from 128 MB on 1.06 (f16 19904x8240x32 110 / 134), smaller
+    // ones 0.97; 16-bit results with no op and fewer than four k-steps from 256 MB on 1.15 of 14 --, and so does any 32-bit result of 16-bit inputs with no op from 256 MB on, 1.03 on
+    // average (bf16 7376x20816x128 127 / 148, 22592x4864x128 85.5 / 90.8; 150 to 256 MB 0.95).
+    if (batch == 1 && row_bytes % 128 == 64) {
+        if (os == 4 && c_bytes > (int64_t)(plain ? 128 : 256) << 20) return false;
+        if (os == 2 && plain && k_bytes < 256 && c_bytes > (int64_t)256 << 20) return false;
     }
-    // 32-bit results in rows on odd multiples of 64 bytes: the line of 128 bytes between two column tiles is written in halves, which costs this kernel more
-    // than the others once C is nearly all of the traffic (34 problems 0.98 on average, but f16 19904x8240x32 110 / 134, 47408x2768x32 102 / 118,
-    // 41 x (384x4400x64) 57 / 66; with C no more than eight times the operands 0.84).
-    if (os == 4 && lean && (g.c_rs * os) % 128 == 64 && (double)g.M * g.N * os > 8.0 * (double)(g.M + g.N) * k_bytes) return false;
+    if (plain && os == 4 && row_bytes % 128 == 0 && c_bytes > (int64_t)256 << 20) return false;
     return true;
 }
 

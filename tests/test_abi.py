@@ -520,15 +520,20 @@ def _choice(in_type, out_type, M, N, K, a_col=False, b_col=False, epilogue=_lib.
 @pytest.mark.parametrize("in_type,out_type,batch,M,N,K,ops,short_k", [
     ("f16", "f16", 32, 2048, 2048, 128, "scale", True), ("f16", "f16", 1, 8192, 8192, 64, "relu", True), ("bf16", "f32", 1, 6352, 2952, 96, "relu", True), ("bf16", "bf16", 1, 51424, 4096, 128, "relu", True),
     ("f16", "f16", 1, 50176, 256, 128, "none", False), ("f16", "f16", 1, 69872, 256, 128, "none", True), ("f16", "f16", 1, 67168, 256, 64, "none", True),  # one column tile
-    ("bf16", "f32", 1, 22592, 4864, 128, "relu", False), ("bf16", "f32", 1, 22592, 4864, 128, "scale", True), ("bf16", "f32", 1, 22592, 4864, 96, "relu", True),  # what the four-wave kernel takes too
+    ("f16", "f16", 1, 36240, 384, 128, "relu", False), ("f16", "f16", 1, 36240, 384, 128, "scale", True), ("f16", "f16", 1, 46080, 384, 128, "relu", True),  # two, a little more than a round
+    ("bf16", "f32", 1, 22592, 4864, 128, "relu", False), ("bf16", "f32", 1, 22592, 4864, 128, "scale", True), ("bf16", "f32", 1, 12288, 4864, 128, "relu", True),  # 440 and 239 MB of C
     ("bf16", "f32", 80, 992, 1024, 128, "none", True), ("i8", "i32", 1, 10624, 9728, 256, "relu", False), ("i8", "i16", 1, 10624, 9728, 256, "relu", True),
-    ("bf16", "bf16", 1, 15072, 22256, 128, "none", False), ("bf16", "bf16", 1, 2656, 5144, 128, "none", True), ("bf16", "bf16", 1, 15072, 22272, 128, "none", True),  # rows off 128-byte boundaries
-    ("f16", "f32", 1, 19904, 8240, 32, "none", False), ("f16", "f32", 1, 19904, 8256, 32, "none", True), ("f16", "f32", 160, 64, 1136, 96, "relu", True),  # ... on odd multiples of 64 bytes
+    ("i8", "i32", 1, 10624, 4864, 256, "relu/col", True), ("i8", "i32", 1, 9376, 9800, 256, "relu/col", True), ("i8", "i32", 1, 3792, 1352, 256, "none/col", True),  # not the four-wave kernel's
+    ("bf16", "bf16", 1, 15072, 22256, 128, "none", True), ("bf16", "bf16", 1, 2656, 5144, 128, "none", True), ("f16", "f16", 1, 7264, 9592, 128, "relu", True),  # rows off 64-byte boundaries
+    ("bf16", "bf16", 1, 5152, 1832, 96, "none", True), ("bf16", "bf16", 1, 3232, 1832, 96, "none", False), ("bf16", "bf16", 1, 560, 13512, 64, "none", True), ("i8", "i32", 1, 3232, 1832, 128, "none/col", True),  # ... two, one tile per CU
+    ("f16", "f32", 1, 19904, 8240, 32, "none", False), ("f16", "f32", 1, 3904, 8240, 32, "none", True), ("f16", "f32", 160, 64, 1136, 96, "relu", True),  # on odd multiples of 64 bytes
+    ("i8", "i32", 1, 10000, 9744, 128, "none", False), ("i8", "i32", 1, 5000, 9744, 128, "none", True), ("f16", "f16", 1, 20000, 8224, 64, "none", False), ("f16", "f16", 1, 20000, 8224, 128, "none", True),
 ])
 def test_where_the_short_k_kernel_is_taken(in_type, out_type, batch, M, N, K, ops, short_k):
     """Both sides of the lines where another kernel is level or ahead (figures beside the rule)."""
+    ops, _, b = ops.partition("/")
     epilogue, arg = {"none": (_lib.EPILOGUE_NONE, 0.0), "relu": (_lib.EPILOGUE_RELU, 0.0), "scale": (_lib.EPILOGUE_SCALE, 0.125)}[ops]
-    assert (_choice(in_type, out_type, M, N, K, epilogue=epilogue, epilogue_arg=arg, batch=batch)[0] == _lib.VARIANT_SHORT_K) == short_k
+    assert (_choice(in_type, out_type, M, N, K, epilogue=epilogue, epilogue_arg=arg, batch=batch, b_col=b == "col")[0] == _lib.VARIANT_SHORT_K) == short_k
 
 
 @pytest.mark.parametrize("in_type,M,N,K,tile,slices", [
