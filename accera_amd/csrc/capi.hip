@@ -634,12 +634,18 @@ int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats
     const int64_t tiles = (((int64_t)g.M + v.bm - 1) / v.bm) * (((int64_t)g.N + v.bn - 1) / v.bn);
     if (v.direct && tiles >= 160) return 1;
     const int64_t target = v.direct && v.bm * v.bn > 64 * 64 ? kComputeUnits : 2 * kComputeUnits;
-    int64_t want = std::min<int64_t>(target / tiles, 32);
     const int64_t b_bytes = (int64_t)g.N * g.K * elem_size(g.in_type);
-    // (int8 on 128 x 128 tiles with direct fills: a quarter, 155x5568x7296 22.0 us in two slices with their 7 MB, 41 MB of B, 47.0 unsplit; not on register-staged ones, 144x14581x5122
-    // with a K-contiguous B 52.7 unsplit, 58.6 in two)
-    const int64_t sums_at_most = b_bytes / (g.in_type == T_I8 && v.direct && v.bm * v.bn == 128 * 128 ? 4 : 6);
-    while (want > 1 && (g.K / want < 960 || want * (int64_t)g.M * g.N * 4 > sums_at_most)) --want;
+    const auto within = [&](int64_t share) {
+        int64_t n = std::min<int64_t>(target / tiles, 32);
+        while (n > 1 && (g.K / n < 960 || n * (int64_t)g.M * g.N * 4 > b_bytes / share)) --n;
+        return n;
+    };
+    int64_t want = within(6);
+    // (int8 on 128 x 128 tiles: a quarter, with direct fills always -- 155x5568x7296 22.0 us in two slices with their 7 MB, 41 MB of B, 47.0 unsplit --, on register-staged ones
+    // for a third slice, 34 problems 0.80 of the time in two, 92x16535x4956 55.1 / 44.9, 227x9408x15424 reading C 107 / 82, not for a second one, 102 problems 1.10 of the unsplit time,
+    // 144x14581x5122 with a K-contiguous B 52.7 / 58.6)
+    if (g.in_type == T_I8 && v.bm * v.bn == 128 * 128)
+        if (const int64_t quarter = within(4); v.direct || quarter >= 3) want = quarter;
     // (the 256 x 256 tiles, whose partial sums weigh most: a power of two; and a K-contiguous B from 16 slices on:
     // 48x768x23744 15.7 us in 16, 17.1 in 24, 2x1664x23744 20.6 in 16, 22.7 in 19)
     if (v.bm * v.bn > 128 * 128 || (v.b_kc && want > 16))

@@ -438,6 +438,7 @@ def test_packed_call_checks_its_numbers():
     ("i8", 246, 4992, 9920, False, "128x128", 3),      # the general rule's three slices of these tiles, not two
     ("i8", 124, 3584, 10112, True, "64x64", 4), ("i8", 124, 3584, 10112, False, "128x128", 5),
     ("i8", 144, 14581, 5122, True, "128x128", 1), ("i8", 191, 13089, 6526, False, "128x128", 1),   # register-staged tiles: the sums of two slices are too much beside B
+    ("i8", 92, 16535, 4956, False, "128x128", 3), ("i8", 78, 21032, 5208, True, "128x128", 3),     # ... three pay for themselves
 ])
 def test_65_to_256_rows_against_32_to_192_mb(in_type, M, N, K, b_col, tile, slices):
     from accera_amd import tune
