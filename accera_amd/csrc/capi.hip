@@ -927,8 +927,13 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
             if (mv < 0) { c->variant = ACC950_VARIANT_F32_MFMA; return ACC950_OK; }
         }
         if (mv >= 0 && k_splits == 0) {
-            const int slices = staged_large_slices(pb, &mv, max_split_floats);
-            if (slices > 1) { c->variant = mv; c->splits = slices; return ACC950_OK; }
+            int n = 0, staged = mv;
+            const MfmaVariant& v = mfma_table(pb.g.in_type, &n)[mv];
+            const int slices = staged_large_slices(pb, &staged, max_split_floats);
+            // (a B of 192 MB and more, which the rule above has more slices of these tiles for that the chip holds at once: 240x7808x26496 reading C 141 us in eight, 168 in six;
+            // 33 tiles of them in eight, a little more than a round, 240 / 161)
+            const bool more = streamed_splits > slices && v.bm == 256 && (int64_t)((pb.g.M + 255) / 256) * ((pb.g.N + 255) / 256) * streamed_splits <= kComputeUnits;
+            if (slices > 1 && !more) { c->variant = staged; c->splits = slices; return ACC950_OK; }
         }
         c->variant = mv >= 0 ? mv : ACC950_VARIANT_GENERIC;
         if (mv >= 0) {
