@@ -699,12 +699,13 @@ bool short_k_pays(const Problem& pb)
 
 // Problems of any alignment with a long K and 30 to 128 tiles of 256 x 256: these tiles fetch half as much per MFMA as the 128 x 128 ones the
 // general rule takes, which unaligned operands pay for dearly, and in as many K slices as the chip holds of them (six at most) they
-// fill it; the sums of the slices need a K of about 3800, int8, with twice as many to a byte, 5000 and fewer tiles; against a K-contiguous B more where
-// the 128 x 128 tiles are a round over the chip that is nearly full (5300), int8 where they are one round at most (6000).  us, 128 x 128 unsplit / so: fp16 1234x5678x4321
-// 122.9 / 104.9 in two, 3913x893x6825 108 / 86 in four, bf16 5060x941x3879 105 / 75 in three, 703x3293x5909 86 / 62 in six, int8 644x7700x5155 86 / 66; but fp16 2140x1916x3269
-// 54.4 / 59.8, int8 2287x1790x4547 47 / 54, 2576x2645x4099, 121 tiles, 67.7 / 70.5, K-contiguous fp16 3296x1088x5026 68.0 / 72.5, 1177x2704x4124 52.9 / 56.8, int8 416x7360x5092
-// 37.7 / 47.9, 5056x640x5080 1.10 times as long.  (399 problems, operands out of HBM: 0.76 on average, the slowest 1.02.)  Moves *mv to that kernel and returns
-// the slices, or 1.
+// fill it; the sums of the slices need a K of about 3800, int8, with twice as many to a byte, 5000 and fewer tiles.  Against a K-contiguous B whose
+// rows are whole dwords apart, which the 128 x 128 tiles fetch with less loss, a longer one where those are at most one round over the chip: int8 7000 (52 problems of 5000 to 7000
+// 1.11 of the smaller tiles' time; in rows off dwords 5000, 5500 against 64 x 64 tiles and 6000 from 190 tiles of 128 x 128 on, 0.97 of 232), 16-bit types 5300 where they are a full round and the large ones
+// more than 61 (1.04 of 14; fewer, or in rows off dwords, 0.98 of 18 and 0.88 of 41).  us, 128 x 128 unsplit / so: fp16 1234x5678x4321
+// 122.9 / 104.9 in two, 3913x893x6825 108 / 86 in four, bf16 5060x941x3879 105 / 75 in three, 703x3293x5909 86 / 62 in six, int8 644x7700x5155 86 / 66, K-contiguous bf16
+// 1283x2399x5129 86.4 / 68.2, int8 447x5145x5765 55.8 / 44.4; but fp16 2140x1916x3269 54.4 / 59.8, int8 2287x1790x4547 47 / 54, 2576x2645x4099, 121 tiles, 67.7 / 70.5, K-contiguous
+// fp16 3296x1088x5026 68.0 / 72.5, int8 416x7360x5092 37.7 / 47.9.  Moves *mv to that kernel and returns the slices, or 1.
 int staged_large_slices(const Problem& pb, int* mv, size_t max_floats)
 {
     const GemmArgs& g = pb.g;
@@ -714,7 +715,8 @@ int staged_large_slices(const Problem& pb, int* mv, size_t max_floats)
     const bool i8 = g.in_type == T_I8;
     const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256), small = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
     const bool b_kc = g.b_rs == 1;
-    const int least = i8 ? (b_kc && small <= kComputeUnits ? 6000 : 5000) : b_kc && small > 200 && small <= kComputeUnits ? 5300 : 3800;
+    const bool one_round = b_kc && small <= kComputeUnits, dwords = g.b_cs * elem_size(g.in_type) % 4 == 0;
+    const int least = i8 ? (!one_round ? 5000 : dwords ? 7000 : small > 189 ? 6000 : tab[*mv].bm == 64 ? 5500 : 5000) : one_round && dwords && small > 200 && tiles > 61 ? 5300 : 3800;
     if (g.K < least || tiles < 30 || tiles > (i8 ? 100 : 128) || (double)g.M * g.N < 0.75 * 65536.0 * (double)tiles) return 1;
     const int want = (int)std::min<int64_t>(6, kComputeUnits / tiles);
     if ((size_t)want * (size_t)g.M * (size_t)g.N > ((size_t)1 << 24)) return 1; // 64 MiB of partial sums at most without being asked

@@ -540,10 +540,12 @@ def test_where_the_short_k_kernel_is_taken(in_type, out_type, batch, M, N, K, op
 @pytest.mark.parametrize("in_type,M,N,K,tile,slices", [
     ("f16", 3296, 1088, 5026, "128x128", 1), ("f16", 3296, 1088, 5306, "256x256", 3),   # 234 tiles of 128 x 128: nearly a whole round
     ("f16", 1520, 1344, 3802, "256x256", 6),                                            # 132 of them
+    ("bf16", 3713, 800, 4933, "256x256", 4), ("f16", 1046, 3061, 5162, "256x256", 4),   # rows of B off dwords; 60 large tiles
+    ("i8", 447, 5145, 5765, "256x256", 6), ("i8", 447, 5145, 5764, "128x128", 1),       # rows of B off dwords, and on them
     ("i8", 5184, 736, 5790, "128x128", 1), ("i8", 5184, 736, 6002, "256x256", 4), ("i8", 644, 7700, 5155, "256x256", 2),
 ])
 def test_large_tiles_in_slices_against_a_k_contiguous_b(in_type, M, N, K, tile, slices):
-    """K has to be longer where the 128 x 128 tiles fill the chip in one round."""
+    """K has to be longer where the 128 x 128 tiles fill the chip in one round and rows of B are whole dwords apart."""
     v, ks = _choice(in_type, "i32" if in_type == "i8" else in_type, M, N, K, b_col=True)
     assert f"mfma {tile} " in _lib.variant_name(v) and "any-alignment" in _lib.variant_name(v) and ks == slices, (_lib.variant_name(v), ks)
 
