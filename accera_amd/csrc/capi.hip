@@ -602,16 +602,23 @@ int streamed_b_tile(const Problem& pb)
     // Of 86 to 128 tiles it takes two, which pays as well -- f16 127x14784x4096 with a K-contiguous B 54.1 us unsplit on 64 x 64 tiles, 42.9 so, bf16 169x6336x6656
     // 61.5 / 41.7, 213x6016x4416 27.2 / 24.9 --, against a K-contiguous B from a K of 2048 on (77x15360x1984 22.7 / 24.8), against a row-major one from slices of more
     // than 2048 of K on (below that line the route checks hold the unsplit tiles; 100x11008x4096 takes 43.1 us there and 28.7 in two slices).  int8 gains
-    // more: 155x5568x7296 47.0 / 22.0 in two, 92x9920x7936 40.5 / 26.9 in three, 164x4416x16896 63.7 / 44.7, 214x7808x20608 117 / 65; but against a K-contiguous B only from a
-    // K of 4500 on (70x13312x3200 17.4 / 19.1, 89x12224x3456 19.4 / 20.3; 100x6080x3456, 20 MB, 9.8 / 14.1).  Of 387 problems, B out of HBM, 0.76 of the general rule's
-    // time on average, the slowest 1.09)
+    // more: 155x5568x7296 47.0 / 22.0 in two, 92x9920x7936 40.5 / 26.9 in three, 164x4416x16896 63.7 / 44.7, 214x7808x20608 117 / 65; but against a K-contiguous B, C only written, from
+    // a K of 3800 on, 4200 with more than 400 of the 64 x 64 tiles, 5500 with no more than the chip holds at once (0.90 of their time from there to 5200, 0.97, 0.84; below 1.07,
+    // 1.09, 1.11: 70x13312x3200 17.4 / 19.1, 127x7936x4864 17.5 / 21.7; 66x10752x3840 21.6 / 19.1; 100x6080x3456, 20 MB, 9.8 / 14.1).  Reading C, which leaves the general rule
+    // register-staged tiles, from any K on: 67x10112x3584 25.6 / 17.5, 105x11520x4096 30.4 / 22.4, 25 problems 0.89.)
     if (!streamed_b(pb, (int64_t)192 << 20)) {
         if (g.M <= 64 || !streamed_b(pb, (int64_t)32 << 20)) return 0;
         const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
         const bool i8 = g.in_type == T_I8, b_kc = g.b_rs == 1;
+        // (C read: the general rule has register-staged tiles only, which lose by a fifth against a K-contiguous B, however short K is)
+        const bool reads_c = g.prologue != PRO_SET;
         // (int8, a K-contiguous B and a K of no whole 128 bytes, which the four-stage tiles do not take: 181x5440x7616 26.2 / 40.0)
-        if (i8 && b_kc && (g.K % 128 || g.K < 4500)) return 0;
-        const bool two = i8 || (b_kc ? g.K >= 2048 : g.K > 4096);
+        if (i8 && b_kc && g.K % 128) return 0;
+        if (i8 && b_kc && !reads_c) {
+            const int64_t small = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64);
+            if (g.K < (small <= kComputeUnits ? 5500 : small <= 400 ? 3800 : 4200)) return 0;
+        }
+        const bool two = i8 || (b_kc ? g.K >= 2048 || reads_c : g.K > 4096);
         return tiles * (two ? 2 : 3) <= kComputeUnits ? 128 : 0;
     }
     // (a tile that holds all rows of A: up to 64 rows the small tiles, up to 128 rows the 128 x 128 tiles, up to 256 the
@@ -868,11 +875,13 @@ int choose(const Problem& pb, int variant, int k_splits, Choice* c, size_t max_s
                     // (a B below 192 MB: only with direct fills and in slices -- unsplit f16 121x12800x1536 12.0 us by the general rule, 18.4 on these tiles, 69x14336x1600
                     // 17.1 / 21.5, int8 249x7680x5120 19.2 / 21.1 --, and for int8 not where the general rule takes such tiles by itself in more slices, 246x4992x9920 32.8 us in
                     // three, 40.6 in two, nor, against a K-contiguous B below 40 MB, where it takes four slices and more of its own tiles: 124x3584x10112 20.8 / 20.2 out of HBM but
-                    // 14.0 / 15.6 out of the cache)
+                    // 14.0 / 15.6 out of the cache; all that with C only written: the general rule's tiles are register-staged ones else, 80x3712x9472 22.5 in four slices, 16.4
+                    // this way in seven, bf16 102x12800x2240 32.6 / 26.8 unsplit)
                     if (!streamed_b(pb, (int64_t)192 << 20)) {
                         const int slices = streamed_splits > 1 ? streamed_splits : auto_mfma_splits(v, pb, max_split_floats);
-                        bool keep = v.direct && slices > 1;
-                        if (keep && pb.g.in_type == T_I8) {
+                        const bool reads_c = pb.g.prologue != PRO_SET;
+                        bool keep = v.direct && (slices > 1 || reads_c);
+                        if (keep && pb.g.in_type == T_I8 && !reads_c) {
                             const int general = auto_mfma_variant(pb);
                             if (general >= 0) {
                                 const MfmaVariant& u = mfma_table(pb.g.in_type, &n)[general];

@@ -434,7 +434,8 @@ def test_packed_call_checks_its_numbers():
     # no slices of these tiles: the general rule's, which read B as often and fill the chip
     ("f16", 121, 12800, 1536, True, "64x64", 1), ("bf16", 69, 14336, 1600, True, "64x64", 1), ("f16", 105, 13056, 1792, True, "64x64", 1), ("i8", 249, 7680, 5120, True, "64x64", 1),
     ("bf16", 245, 6720, 4672, True, "128x128", 2),     # (two slices by the general rule's count)
-    ("f16", 86, 13312, 2240, True, "128x128", 2), ("f16", 77, 15360, 1984, True, "64x64", 1), ("i8", 70, 13312, 3200, True, "64x64", 1),  # a K-contiguous B: from a K of 2048, int8 4500 on
+    ("f16", 86, 13312, 2240, True, "128x128", 2), ("f16", 77, 15360, 1984, True, "64x64", 1), ("i8", 70, 13312, 3200, True, "64x64", 1),  # a K-contiguous B: from a K of 2048, int8 3800
+    ("i8", 66, 10752, 3840, True, "128x128", 3), ("i8", 105, 16320, 4096, True, "64x64", 1), ("i8", 105, 16320, 4352, True, "128x128", 2), ("i8", 127, 7936, 4864, True, "64x64", 1),  # ... by the number of smaller tiles
     ("i8", 246, 4992, 9920, False, "128x128", 3),      # the general rule's three slices of these tiles, not two
     ("i8", 124, 3584, 10112, True, "64x64", 4), ("i8", 124, 3584, 10112, False, "128x128", 5),
     ("i8", 144, 14581, 5122, True, "128x128", 1), ("i8", 191, 13089, 6526, False, "128x128", 1),   # register-staged tiles: the sums of two slices are too much beside B
@@ -445,6 +446,16 @@ def test_65_to_256_rows_against_32_to_192_mb(in_type, M, N, K, b_col, tile, slic
     i, o = {"f16": (_lib.F16, _lib.F16), "bf16": (_lib.BF16, _lib.BF16), "i8": (_lib.I8, _lib.I32)}[in_type]
     variant, splits = tune.own_choice(i, o, M, N, K, False, b_col, 1.0, 0.0)
     assert f"mfma {tile} " in _lib.variant_name(variant) and splits == slices, (_lib.variant_name(variant), splits)
+
+
+@pytest.mark.parametrize("in_type,M,N,K,slices", [("i8", 67, 10112, 3584, 3), ("i8", 105, 11520, 4096, 2), ("i8", 80, 3712, 9472, 7), ("bf16", 102, 12800, 2240, 1)])
+def test_65_to_256_rows_against_a_k_contiguous_b_reading_c(in_type, M, N, K, slices):
+    """The general rule's tiles are register-staged here: the 128 x 128 ones with direct fills, in slices or not."""
+    from accera_amd import tune
+    i, o = {"bf16": (_lib.BF16, _lib.BF16), "i8": (_lib.I8, _lib.I32)}[in_type]
+    variant, splits = tune.own_choice(i, o, M, N, K, False, True, 1.0, 0.5)
+    name = _lib.variant_name(variant)
+    assert "mfma 128x128 " in name and "fill=direct" in name and splits == slices, (name, splits)
 
 
 @pytest.mark.parametrize("in_type,M,N,K,tile,slices", [
