@@ -105,7 +105,7 @@ private:
     void wake()
     {
         if (!asleep_) return; // (a thread counts itself asleep before it looks for a reason not to for the last time: one of the two sees the other)
-        std::lock_guard<std::mutex> lock(m_);
+        { std::lock_guard<std::mutex> lock(m_); } // (who has looked is asleep by now; told while the lock is held, they wake up to wait for it, 5 us of every copy)
         wake_.notify_all();
     }
     // waits for what another thread is about to do: a moment awake, then giving its core to whom it may belong
