@@ -142,9 +142,11 @@ hipError_t reserve(DevBuf& b, size_t bytes)
 }
 
 // Bytes of a piece of a transfer: four pieces, so that one is copied on the host while another is on the bus, but
-// not less than two megabytes (1024^3 fp16 with an fp32 result 367 us with one), and never more than a slot.
+// not less than two megabytes (1024^3 fp16 with an fp32 result 367 us with one), and never more than a slot; below four megabytes one
+// piece, as a second one wakes the copying threads and calls the copy again (23x2366x321 fp32, a B of 3 MB, 201 us in two, 163 so; 234x1536x1024 fp16 240 / 199).
 size_t piece_bytes(size_t bytes)
 {
+    if (bytes < (size_t)4 << 20) return bytes;
     const size_t quarter = (bytes / 4 + 65535) & ~(size_t)65535;
     return std::min(std::max(quarter, (size_t)2 << 20), kSlotBytes);
 }
