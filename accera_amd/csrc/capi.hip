@@ -663,13 +663,13 @@ int streamed_b_splits(const MfmaVariant& v, const Problem& pb, size_t max_floats
     return plan_split(v, pb, (int)want, &sp, max_floats) ? sp.splits : 1;
 }
 
-// K of one to four whole k-steps and many tiles of C: does the short-K kernel (gemm_short_k.h) pay?  Against the other kernels' choice on 3076
-// problems of K = 64 to 256 bytes, 6 to 500 MB of C, every type, layout and ops of this range (two thirds of them with all four k-steps and a 32-bit result): with more
-// than three of its 64 x 256 tiles per CU, and these mostly full, or where rows of C end inside 64 bytes, parts of which the stores of most other kernels send to memory,
-// with more than one, it takes 0.83 of the time on average, as this rule has it (us, fp16 32 x (2048x2048x128) scaled 85 / 57, 8192x8192x64 39 / 29, bf16 6352x2952x96 with an
+// K of one to four whole k-steps and many tiles of C: does the short-K kernel (gemm_short_k.h) pay?  Against the other kernels' choice on 3562
+// problems of K = 64 to 256 bytes, 6 MB to 1 GB of C, every type, layout and ops of this range (half of them with all four k-steps and a 32-bit result): with more than three
+// of its 64 x 256 tiles per CU, and these mostly full, or where rows of C end inside 64 bytes, parts of which the stores of most other kernels send to memory, with more
+// than one, it takes 0.81 of the time on average, where this rule has it (us, fp16 32 x (2048x2048x128) scaled 85 / 57, 8192x8192x64 39 / 29, bf16 6352x2952x96 with an
 // fp32 result 54 / 28, int8 47 x (128x4816x128) 105 / 29, 9376x9800x256 206 / 98); fewer, and a workgroup has nothing to walk along (us, other / this: 5136x384x64 3.0 / 4.4, bf16
 // 4 x (2704x608x96), 516 tiles, with an fp32 result 7.7 / 10.1), and so where tiles stick out by half (195 x (4608x128x32) 58 / 84).  What it leaves are ranges that are slower
-// by it on average, not single problems: a tenth of those it takes are slower by 2 % and more, 1.4 times at most.
+// by it on average, not single problems: one in eight of those it takes is slower by 2 % and more, 1.45 times at most.
 bool short_k_pays(const Problem& pb)
 {
     const GemmArgs& g = pb.g;
