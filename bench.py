@@ -17,7 +17,7 @@ of milliseconds of load to settle, whatever W is.  One JSON line is printed with
   roofline      algorithmic FLOP (or bytes) per launch / average launch duration from
                 HIP events on the launch stream, against the MI355X dense peak
   cpu_baseline  the CPU oracle (a restatement of the reference's HOST schedule, not an
-                Accera-generated package) timed on this box's host cores
+                Accera-generated package) timed on this host's cores
 
 (`--all` is accepted and means the default: all five configurations.)
 """
@@ -62,7 +62,7 @@ def algorithmic_flops(c):
 
 
 def make_inputs(c, n_sets, seed):
-    """Device-resident inputs in the distributions BASELINE names; n_sets rotating copies."""
+    """Device-resident inputs in the distributions the headline workloads name; n_sets rotating copies."""
     import torch
     tt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16, "i8": torch.int8, "i32": torch.int32}
     g = torch.Generator(device="cuda")
@@ -293,7 +293,7 @@ def main():
     ap.add_argument("--k-splits", type=int, default=0)
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--only", action="store_true", help="measure --config alone (default: the four other configurations ride along)")
-    ap.add_argument("--all", action="store_true", help="all five BASELINE configurations (the default)")
+    ap.add_argument("--all", action="store_true", help="all five headline configurations (the default)")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         print("bench.py: this build runs on ONE GPU only (no collectives, no sharding); run with --gpus 1", file=sys.stderr)
