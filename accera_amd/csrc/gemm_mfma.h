@@ -1069,7 +1069,9 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
     // branch are as many registers again: a kilobyte of scratch per lane on 256 x 256 tiles.)
     // The two conditions are worked out without branches and asked one after the other: as a chain of && and || the way of a plain ReLU went through
     // a dozen jumps into far-off pieces of code and a copy of the sums (fp16 3408x1104x128 to fp32 with a ReLU 6.03 us, 5.80 this way), and the 256 x 256 kernels
-    // had 68 bytes of scratch, which are gone.  The int8 kernels with direct fills do better as one chain: 56 to 76 bytes there, 150 to 280 with two tests.
+    // had 68 bytes of scratch, which are gone.  The int8 kernels do better as one chain with direct fills (56 to 76 bytes, 150 to 280 with two tests) and on
+    // register-staged tiles of up to 128 x 128 (63 x (64x1464x48) with a K-contiguous B and a constant 13.1 us with two tests, 12.75 so, 2000x3000x777 20.4 / 19.9); not on 256 x 256 ones
+    // of those (none or 20 bytes with two tests, 68 to 76 so: 1234x5678x7401 105.5 / 106.7).
     const bool set_constant = (p.prologue == PRO_SET) & (p.prologue_arg != 0.f);
     const bool plain_relu = (p.epilogue == EPI_RELU) & !set_constant, other_ops = ((p.epilogue != EPI_NONE) | set_constant) & !plain_relu;
     auto relu_pass = [&]() __attribute__((always_inline)) { for_each_acc([&](scalar_t v) { return v > scalar_t(0) ? v : scalar_t(0); }); };
@@ -1088,7 +1090,7 @@ __global__ void __launch_bounds__(Cfg::NT, Cfg::WGS_PER_CU) gemm_mfma_kernel(ACC
             return __builtin_bit_cast(scalar_t, (__builtin_bit_cast(unsigned, v) & keep) | put);
         });
     };
-    if constexpr (IN == IN_I8 && !EDGE) {
+    if constexpr (IN == IN_I8 && (!EDGE || BM * BN <= 128 * 128)) {
         if (plain_relu) relu_pass();
         else if (other_ops) ops_pass();
     } else {
